@@ -27,7 +27,6 @@
 
 #include "m2d_internal.h"
 #include "msi_stencil.h"
-#include "seqsum.h"
 
 namespace m2d {
 
@@ -795,15 +794,6 @@ __global__ __launch_bounds__(kTx) void k_mass_terms(Fields F)
     const long t = (long)(j - 2) * (F.nx - 2) + (i - 2);
     F.out[1][t] = fabs((ro[np] - roa[np]) * rp[np] / (Jp[np] * F.dt) + fme - fmw + fmn - fms);
 }
-// the terms added in the reference's order by one wave (seq_sum)
-__global__ __launch_bounds__(kSeqThreads) void k_mass_sum(Fields F)
-{
-    const long n = (long)(F.nx - 2) * (F.ny - 2);
-    const double *t = F.out[1];
-    __shared__ double lds[kSeqSlots * kSeqChunk];
-    const double r = seq_sum(t, n, lds);
-    if (threadIdx.x == 0) F.out[0][0] = r;
-}
 
 // ---------------------------------------------------------------------------
 // Fictitious-row writers of the internal-flow case,
@@ -1043,7 +1033,7 @@ struct Routine {
     int nout;
     int outk[6];  // N-vectors per output; 0 = one scalar
     int grid;     // kInterior, kFaces (1..nx-1 x 1..ny-1), kAll or kBoundary
-    void (*post)(Fields);  // one-workgroup follow-up over a scratch output
+    bool sum;     // the kernel fills a scratch output; output 0 is its in-order sum
     int iny1;     // 1 + index of an input of ny values (0: none)
 };
 
@@ -1087,14 +1077,16 @@ int run(const Routine &R, Fields F)
         grid = dim3((unsigned)((2L * nx + 2L * (ny - 2) + kTx - 1) / kTx), 1);
     else
         grid = dim3((unsigned)((N + kTx - 1) / kTx), 1);
-    // device buffer: staged host arrays and the scratch output of `post`
-    long tot = R.post ? N : 0;
+    // device buffer: staged host arrays and the terms of a sum
+    const long nin = (long)(nx - 2) * (ny - 2);
+    long tot = R.sum ? nin + seq_scratch(nin, 1) : 0;
     if (!dev) {
         for (int k = 0; k < R.nin; ++k) tot += in_len(R, k, N, ny);
         for (int k = 0; k < R.nout; ++k) tot += out_len(R, k, N);
     }
-    double *d = nullptr;
-    if (tot && hipMalloc((void **)&d, sizeof(double) * tot) != hipSuccess) return M2D_ERR_HIP;
+    Scratch S;
+    double *const d = tot ? S.get((size_t)tot) : nullptr;
+    if (tot && !d) return M2D_ERR_HIP;
     Fields G = F;
     hipStream_t s = dev ? g_stream : nullptr;
     if (dev) {
@@ -1121,10 +1113,10 @@ int run(const Routine &R, Fields F)
             off += n;
         }
     }
-    if (R.post) G.out[R.nout] = d + off;  // scratch
+    if (R.sum) G.out[R.nout] = d + off;  // the terms
     if (!rc) {
         hipLaunchKernelGGL(R.kernel, grid, block, 0, s, G);
-        if (R.post) hipLaunchKernelGGL(R.post, dim3(1), dim3(kSeqThreads), 0, s, G);
+        if (R.sum) seq_sums_enqueue(d + off, nin, 1, G.out[0], false, d + off + nin, s);
         if (hipGetLastError() != hipSuccess) rc = M2D_ERR_HIP;
     }
     if (!dev)
@@ -1132,39 +1124,37 @@ int run(const Routine &R, Fields F)
             if (hipMemcpy(F.out[k], G.out[k], sizeof(double) * out_len(R, k, N),
                           hipMemcpyDeviceToHost) != hipSuccess)
                 rc = M2D_ERR_HIP;
-    if (d) {
-        if (dev && hipStreamSynchronize(s) != hipSuccess) rc = M2D_ERR_HIP;  // scratch in use
-        (void)hipFree(d);
-    }
+    if (d && dev && hipStreamSynchronize(s) != hipSuccess) rc = M2D_ERR_HIP;  // scratch in use
+    if (!rc) S.done();
     return rc;
 }
 
-const Routine kNodes = {k_density_at_nodes, 2, {-1, -1}, 1, {1}, kAll, nullptr};
-const Routine kDensity = {k_density_at_faces, 3, {-1, -1}, 2, {1, 1}, kFaces, nullptr};
-const Routine kU = {k_u_coefficients, 19, {-1, -1}, 1, {9}, kInterior, nullptr};
-const Routine kV = {k_v_coefficients, 20, {-1, -1}, 1, {9}, kInterior, nullptr};
-const Routine kUs = {k_u_source, 25, {-1, -1}, 3, {1, 1, 1}, kInterior, nullptr};
-const Routine kVs = {k_v_source, 25, {-1, -1}, 3, {1, 1, 1}, kInterior, nullptr};
-const Routine kT = {k_T_coefficients_and_source, 43, {-1, -1}, 2, {9, 1}, kInterior, nullptr};
-const Routine kPc = {k_p_coefficients, 11, {-1, -1}, 1, {5}, kInterior, nullptr};
-const Routine kPs = {k_p_source, 14, {-1, -1}, 1, {1}, kInterior, nullptr};
+const Routine kNodes = {k_density_at_nodes, 2, {-1, -1}, 1, {1}, kAll, false};
+const Routine kDensity = {k_density_at_faces, 3, {-1, -1}, 2, {1, 1}, kFaces, false};
+const Routine kU = {k_u_coefficients, 19, {-1, -1}, 1, {9}, kInterior, false};
+const Routine kV = {k_v_coefficients, 20, {-1, -1}, 1, {9}, kInterior, false};
+const Routine kUs = {k_u_source, 25, {-1, -1}, 3, {1, 1, 1}, kInterior, false};
+const Routine kVs = {k_v_source, 25, {-1, -1}, 3, {1, 1, 1}, kInterior, false};
+const Routine kT = {k_T_coefficients_and_source, 43, {-1, -1}, 2, {9, 1}, kInterior, false};
+const Routine kPc = {k_p_coefficients, 11, {-1, -1}, 1, {5}, kInterior, false};
+const Routine kPs = {k_p_source, 14, {-1, -1}, 1, {1}, kInterior, false};
 const Routine kVel = {k_velocities_at_internal_faces, 26, {16, 17}, 6, {1, 1, 1, 1, 1, 1},
-                      kInterior, nullptr};
+                      kInterior, false};
 const Routine kSimplec = {k_internal_simplec_coefficients, 8, {6, 7}, 6, {1, 1, 1, 1, 1, 1},
-                          kInterior, nullptr};
-const Routine kPcor = {k_pressure_correction_with_pl, 1, {-1, -1}, 1, {1}, kAll, nullptr};
-const Routine kRcor = {k_density_correction_with_pl, 2, {-1, -1}, 1, {1}, kAll, nullptr};
-const Routine kUVcor = {k_u_v_at_real_nodes_with_pl, 8, {6, 7}, 2, {1, 1}, kInterior, nullptr};
+                          kInterior, false};
+const Routine kPcor = {k_pressure_correction_with_pl, 1, {-1, -1}, 1, {1}, kAll, false};
+const Routine kRcor = {k_density_correction_with_pl, 2, {-1, -1}, 1, {1}, kAll, false};
+const Routine kUVcor = {k_u_v_at_real_nodes_with_pl, 8, {6, 7}, 2, {1, 1}, kInterior, false};
 const Routine kFcor = {k_velocity_correction_at_faces_with_pl, 11, {-1, -1}, 6,
-                       {1, 1, 1, 1, 1, 1}, kFaces, nullptr};
-const Routine kFlags = {k_boundary_faces_flags, 0, {-1, -1}, 2, {1, 1}, kAll, nullptr};
-const Routine kMass = {k_mass_terms, 10, {-1, -1}, 1, {0}, kInterior, k_mass_sum};
-const Routine kBcU = {k_intflow_bc_uv<0>, 6, {-1, -1}, 2, {9, 1}, kBoundary, nullptr};
-const Routine kBcV = {k_intflow_bc_uv<1>, 6, {-1, -1}, 2, {9, 1}, kBoundary, nullptr};
-const Routine kBcPl = {k_intflow_bc_pl, 4, {-1, -1}, 2, {5, 1}, kBoundary, nullptr, 4};
-const Routine kBcT = {k_intflow_bc_T, 4, {-1, -1}, 2, {9, 1}, kBoundary, nullptr, 4};
+                       {1, 1, 1, 1, 1, 1}, kFaces, false};
+const Routine kFlags = {k_boundary_faces_flags, 0, {-1, -1}, 2, {1, 1}, kAll, false};
+const Routine kMass = {k_mass_terms, 10, {-1, -1}, 1, {0}, kInterior, true};
+const Routine kBcU = {k_intflow_bc_uv<0>, 6, {-1, -1}, 2, {9, 1}, kBoundary, false};
+const Routine kBcV = {k_intflow_bc_uv<1>, 6, {-1, -1}, 2, {9, 1}, kBoundary, false};
+const Routine kBcPl = {k_intflow_bc_pl, 4, {-1, -1}, 2, {5, 1}, kBoundary, false, 4};
+const Routine kBcT = {k_intflow_bc_T, 4, {-1, -1}, 2, {9, 1}, kBoundary, false, 4};
 // the boundary grid (2 nx + 2 (ny-2) threads) covers its 2 (nx-2) + 2 (ny-2) faces
-const Routine kVelBf = {k_intflow_vel_bf, 8, {-1, -1}, 6, {1, 1, 1, 1, 1, 1}, kBoundary, nullptr};
+const Routine kVelBf = {k_intflow_vel_bf, 8, {-1, -1}, 6, {1, 1, 1, 1, 1, 1}, kBoundary, false};
 
 Fields fields(const int *nx, const int *ny)
 {

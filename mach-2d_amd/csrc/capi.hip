@@ -1648,10 +1648,11 @@ static int solve9(m2d_system *s9, const m2d_time_step_params *P, const double *a
 }
 
 // The time step's side stream and its scratch: the residual norms' work
-// (norm_l1_work_size), then the in-order sums': the average of p (n + 2
-// doubles), the terms of the four mean coefficients and of the mass check
-// (5 n) and their five sums, n = (nx-2)(ny-2), then kTsNormSlots sums of the
-// step's residual norms, then the inflow update's 3 (ny-2) values; h_ts
+// (norm_l1_work_size), then the in-order sums': the average of p
+// (average_scratch) and its mean, the terms of the four mean coefficients and of the mass
+// check (5 n) and their five sums, n = (nx-2)(ny-2), then kTsNormSlots sums
+// of the step's residual norms, the inflow update's 3 (ny-2) values and the
+// five sums' seq_scratch; h_ts
 // receives p's average, the five sums and the norms' sums, and holds the
 // inflow update's host values.  Created with the first step on the handle.
 constexpr int kTsNormSlots = 8;
@@ -1661,8 +1662,8 @@ static int ts_side_ready(m2d_system *s)
     const long n = (long)(s->nx - 2) * (s->ny - 2), nr = 3L * (s->ny - 2);
     HIP_OK(hipMalloc((void **)&s->ts_scr,
                      sizeof(double) * (size_t)(norm_l1_work_size(s->nx, s->ny) +
-                                               average_scratch(s->nx, s->ny) + 5 * n + 5 +
-                                               kTsNormSlots + nr)));
+                                               average_scratch(s->nx, s->ny) + 1 + 5 * n + 5 +
+                                               kTsNormSlots + nr + seq_scratch(n, 5))));
     HIP_OK(hipHostMalloc((void **)&s->h_ts, sizeof(double) * (size_t)(6 + kTsNormSlots + nr),
                          hipHostMallocDefault));
     HIP_OK(hipEventCreateWithFlags(&s->ev_fork, hipEventDisableTiming));
@@ -1728,7 +1729,7 @@ extern "C" int m2d_intflow_time_step(m2d_system *s9, m2d_system *s5,
     // read once with the step's last wait, then added in the same order.
     // kind 9: norm_l1_9d relative (two sums, slots k and k+1); kind 5:
     // norm_l1_5d (one sum).  A new mass cycle starts the list again.
-    double *const nres = side + average_scratch(nx, ny) + 5 * nin + 5;
+    double *const nres = side + average_scratch(nx, ny) + 1 + 5 * nin + 5;
     int nkind[kTsNormSlots], nslot[kTsNormSlots], nops = 0, nused = 0;
     auto norm9_relative = [&](const double *a, const double *b, const double *x) {
         if (rc) return;
@@ -1773,14 +1774,14 @@ extern "C" int m2d_intflow_time_step(m2d_system *s9, m2d_system *s5,
     auto avg_enqueue = [&]() {
         if (!avg_forked || rc) return;
         avg_forked = false;
-        double *scr = side;
+        double *scr = side, *mean = side + average_scratch(nx, ny);
         if (hipStreamWaitEvent(s5->aux, s5->ev_fork, 0) != hipSuccess) {
             rc = M2D_ERR_HIP;
             return;
         }
-        average_enqueue(nx, ny, f->p, scr, s5->aux);
+        average_enqueue(nx, ny, f->p, scr, mean, s5->aux);
         if (hipGetLastError() != hipSuccess ||
-            hipMemcpyAsync(s5->h_ts, scr, sizeof(double), hipMemcpyDeviceToHost, s5->aux) !=
+            hipMemcpyAsync(s5->h_ts, mean, sizeof(double), hipMemcpyDeviceToHost, s5->aux) !=
                 hipSuccess ||
             hipEventRecord(s5->ev_join, s5->aux) != hipSuccess) {
             rc = M2D_ERR_HIP;
@@ -1801,7 +1802,7 @@ extern "C" int m2d_intflow_time_step(m2d_system *s9, m2d_system *s5,
     // step's longest tail, start as early as they can.  Scratch: terms of
     // the four means at t[0, 4n), of the mass check at t[4n, 5n), the sums
     // at t[5n, 5n + 5).
-    double *tsum = side + average_scratch(nx, ny);
+    double *tsum = side + average_scratch(nx, ny) + 1;
     bool side_forked = false, side_pending = false;
     auto sums_enqueue = [&]() {
         if (side_forked || rc) return;
@@ -1820,7 +1821,8 @@ extern "C" int m2d_intflow_time_step(m2d_system *s9, m2d_system *s5,
             rc = M2D_ERR_HIP;
             return;
         }
-        seq_sums_enqueue(tsum + first * nin, nin, K, tsum + 5 * nin + first, s5->aux);
+        seq_sums_enqueue(tsum + first * nin, nin, K, tsum + 5 * nin + first, false,
+                         nres + kTsNormSlots + 3L * (ny - 2), s5->aux);
         if (hipGetLastError() != hipSuccess ||
             hipMemcpyAsync(s5->h_ts + 1 + first, tsum + 5 * nin + first, sizeof(double) * K,
                            hipMemcpyDeviceToHost, s5->aux) != hipSuccess ||

@@ -28,7 +28,6 @@
 #include <vector>
 
 #include "m2d_internal.h"
-#include "seqsum.h"
 
 using namespace m2d;
 
@@ -330,36 +329,19 @@ __global__ __launch_bounds__(kT) void k_sum(const double *__restrict__ part, lon
 }
 
 // get_average: F over real volumes in the reference's order (j outer, i
-// inner) gathered into t (contiguous, in that order), then added in order
-// by one wave and divided by (nx-2)(ny-2)
+// inner) gathered into t (contiguous, in that order); its in-order sum over
+// (nx-2)(ny-2) is the mean
 __global__ __launch_bounds__(kT) void k_average_gather(const double *__restrict__ F, int nx,
                                                       int ny, double *__restrict__ t)
 {
     const int i = blockIdx.x * kT + threadIdx.x + 1, j = blockIdx.y + 1;
     if (i <= nx - 2) t[(long)(j - 1) * (nx - 2) + (i - 1)] = F[(long)nx * j + i];
 }
-__global__ __launch_bounds__(kSeqThreads) void k_average(const double *__restrict__ t, int nx,
-                                                        int ny, double *__restrict__ out)
-{
-    const long n = (long)(nx - 2) * (ny - 2);
-    __shared__ double lds[kSeqSlots * kSeqChunk];
-    const double s = seq_sum(t, n, lds);
-    if (threadIdx.x == 0) out[0] = s / ((double)(nx - 2) * (double)(ny - 2));
-}
-
 // arrays of one call: pointer, length, written by the call
 struct Arr {
     const double *p;
     long n;
     bool out;
-};
-
-struct Buf {
-    double *d = nullptr;
-    ~Buf()
-    {
-        if (d) (void)hipFree(d);
-    }
 };
 
 // Checks the arrays, stages host arrays, runs launch(device pointers,
@@ -379,9 +361,9 @@ int run(int nx, int ny, std::vector<Arr> arrs, long scratch, bool sync, Launch l
     long tot = scratch;
     if (!dev)
         for (const Arr &a : arrs) tot += a.n;
-    Buf B;
-    if (tot > 0 && hipMalloc((void **)&B.d, sizeof(double) * tot) != hipSuccess)
-        return M2D_ERR_HIP;
+    Scratch B;
+    double *const buf = tot > 0 ? B.get((size_t)tot) : nullptr;
+    if (tot > 0 && !buf) return M2D_ERR_HIP;
     std::vector<double *> d(arrs.size());
     long off = 0;
     for (size_t k = 0; k < arrs.size(); ++k) {
@@ -389,13 +371,13 @@ int run(int nx, int ny, std::vector<Arr> arrs, long scratch, bool sync, Launch l
             d[k] = const_cast<double *>(arrs[k].p);
             continue;
         }
-        d[k] = B.d + off;
+        d[k] = buf + off;
         off += arrs[k].n;
         if (hipMemcpyAsync(d[k], arrs[k].p, sizeof(double) * arrs[k].n, hipMemcpyHostToDevice,
                            s) != hipSuccess)
             return M2D_ERR_HIP;
     }
-    double *scr = B.d ? B.d + off : nullptr;
+    double *scr = buf ? buf + off : nullptr;
     const int L = nx > ny ? nx : ny;
     launch(d, s, scr, dim3((unsigned)((L + kT - 1) / kT)));
     if (hipGetLastError() != hipSuccess) return M2D_ERR_HIP;
@@ -405,23 +387,28 @@ int run(int nx, int ny, std::vector<Arr> arrs, long scratch, bool sync, Launch l
                                               sizeof(double) * arrs[k].n,
                                               hipMemcpyDeviceToHost, s) != hipSuccess)
                 return M2D_ERR_HIP;
-    // host arrays, a value to read, or a scratch buffer that the free below
-    // would release under a running kernel
-    if ((!dev || sync || B.d) && hipStreamSynchronize(s) != hipSuccess) return M2D_ERR_HIP;
+    // host arrays, a value to read, or a scratch buffer the next call uses
+    if ((!dev || sync || buf) && hipStreamSynchronize(s) != hipSuccess) return M2D_ERR_HIP;
+    B.done();
     return M2D_OK;
 }
 
 }  // namespace
 
-// scratch: the mean, the n gathered terms, one more (seq_sum reads whole
-// 16-byte pairs)
-long m2d::average_scratch(int nx, int ny) { return (long)(nx - 2) * (ny - 2) + 2; }
-
-void m2d::average_enqueue(int nx, int ny, const double *F, double *scr, hipStream_t s)
+// scratch: the n gathered terms, what their sum needs
+long m2d::average_scratch(int nx, int ny)
 {
+    const long n = (long)(nx - 2) * (ny - 2);
+    return n + seq_scratch(n, 1);
+}
+
+void m2d::average_enqueue(int nx, int ny, const double *F, double *scr, double *out,
+                          hipStream_t s)
+{
+    const long n = (long)(nx - 2) * (ny - 2);
     const dim3 g((unsigned)((nx - 2 + kT - 1) / kT), (unsigned)(ny - 2));
-    hipLaunchKernelGGL(k_average_gather, g, dim3(kT), 0, s, F, nx, ny, scr + 1);
-    hipLaunchKernelGGL(k_average, dim3(1), dim3(kSeqThreads), 0, s, scr + 1, nx, ny, scr);
+    hipLaunchKernelGGL(k_average_gather, g, dim3(kT), 0, s, F, nx, ny, scr);
+    seq_sums_enqueue(scr, n, 1, out, true, scr + n, s);
 }
 
 void m2d_set_last_status_code(int status);
@@ -625,14 +612,15 @@ extern "C" double m2d_get_average(const int *nx, const int *ny, const double *F)
         return 0.0;
     }
     const int NX = *nx, NY = *ny;
-    const long n = (long)(NX - 2) * (NY - 2);
-    double out = 0.0;
+    double *const res = Scratch::results();
+    if (!res) {
+        m2d_set_last_status_code(M2D_ERR_HIP);
+        return 0.0;
+    }
     const int rc = run(NX, NY, {{F, (long)NX * NY, false}}, average_scratch(NX, NY), true,
                        [&](std::vector<double *> &d, hipStream_t s, double *scr, dim3) {
-                           average_enqueue(NX, NY, d[0], scr, s);
-                           (void)hipMemcpyAsync(&out, scr, sizeof(double),
-                                                hipMemcpyDeviceToHost, s);
+                           average_enqueue(NX, NY, d[0], scr, res, s);
                        });
     m2d_set_last_status_code(rc);
-    return out;
+    return rc ? 0.0 : *res;
 }

@@ -136,17 +136,18 @@ hipStream_t assembly_stream_current();
 void assembly_gate(const int *gate, const double *sc);
 
 // ---- in-order statistics of the time step (tstep.hip, intflow.hip) -----------
-// The K mean convergence coefficients of device arrays a[k] (nd[k] = 9 or 5
-// diagonals) enqueued on s: scratch t of K*(nx-2)*(ny-2) + K doubles, the
-// means at its end.
-void mean_cc_enqueue(int nx, int ny, int K, const double *const *a, const int *nd, double *t,
-                     hipStream_t s);
-// the terms of those means only (t + k*n for array k), and K in-order sums of
-// consecutive arrays of n terms (t + k*n) into out[k], each on its own
-// workgroup of one launch
+// The terms of the mean convergence coefficients of K <= 4 device arrays a[k]
+// (nd[k] = 9 or 5 diagonals), (nx-2)(ny-2) at t + k*(nx-2)(ny-2), in the
+// reference's order
 void cc_terms_enqueue(int nx, int ny, int K, const double *const *a, const int *nd, double *t,
                       hipStream_t s);
-void seq_sums_enqueue(const double *t, long n, int K, double *out, hipStream_t s);
+// K sums of consecutive arrays of n terms (t + k*n), each the left-to-right
+// loop's value bit for bit, over n if mean, into out[k]; scratch:
+// seq_scratch(n, K) doubles, 16-byte aligned or not
+constexpr int kSeqSegDoubles = 7;
+long seq_scratch(long n, int K);
+void seq_sums_enqueue(const double *t, long n, int K, double *out, bool mean, double *scratch,
+                      hipStream_t s);
 // check_mass_conservation's terms (in = rp, re, rn, Jp, ro, roa, ron, roe,
 // Uce, Vcn; device arrays) into t[0 .. (nx-2)(ny-2)), in the reference's
 // order, on s; their in-order sum is rmass
@@ -154,12 +155,36 @@ void mass_terms_enqueue(int nx, int ny, double dt, const double *const *in, doub
                         hipStream_t s);
 // tstepper_dt_scarborough's step rule on the four means cc (u, v, T, p')
 double scarborough_dt(double dt, const double *cc, double h0, double mincc, double maxcc);
-// get_average of the device field F enqueued on s: the mean lands in scr[0]
+// get_average of the device field F enqueued on s: the mean lands in *out
 // (scratch of average_scratch(nx, ny) doubles)
 long average_scratch(int nx, int ny);
-void average_enqueue(int nx, int ny, const double *F, double *scr, hipStream_t s);
+void average_enqueue(int nx, int ny, const double *F, double *scr, double *out, hipStream_t s);
 // true for device memory (false for host memory and unknown pointers)
 bool is_device_array(const void *p);
+
+// Device scratch of one call that waits for its stream before it returns.
+// A host thread keeps its last buffer (up to 64 MiB, on the device it was
+// made for) for its next call and gives it back when the thread ends; larger
+// ones, and one asked for while the kept one is in use, live as long as the
+// call.  done: the stream was waited for, so the buffer can be used again;
+// without it the buffer is freed (which waits for the device).
+class Scratch {
+public:
+    ~Scratch();
+    // n doubles, or nullptr
+    double *get(size_t n);
+    // the thread's kResults doubles of pinned host memory for the values the
+    // call returns, which its last kernel writes itself (a copy to the
+    // caller's memory would be one more operation on the stream); nullptr if
+    // there are none.  Read them after the stream was waited for.
+    static constexpr int kResults = 8;
+    static double *results();
+    void done() { done_ = true; }
+
+private:
+    double *p_ = nullptr;
+    bool kept_ = false, done_ = false;
+};
 template <typename TI, typename TO>
 void launch_convert(const TI *in, TO *out, long n, hipStream_t s);
 

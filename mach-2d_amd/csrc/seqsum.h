@@ -1,5 +1,5 @@
-// seqsum.h -- in-order sum of n terms, for results that must equal a
-// sequential loop bit for bit (the reference's left-to-right sums).
+// seqsum.h -- in-order sum of n terms of any sign, one by one: the part of
+// seqsum.hip's sums that its maps do not cover.
 //
 // The chain of dependent FP64 additions is the whole cost (about 10 cycles
 // per term on gfx950, reads included), so one wave does it and keeps it fed.  The terms reach
@@ -194,12 +194,13 @@ __device__ __forceinline__ double seq_add_chunk(const double *slot, double m)
     return m;
 }
 
-// p[0] + p[1] + ... + p[n-1], added left to right; lds: kSeqSlots *
+// m + p[0] + p[1] + ... + p[n-1], added left to right; lds: kSeqSlots *
 // kSeqChunk doubles of LDS.  The loads start at p rounded down to 16
 // bytes (the memory before a misaligned p belongs to the same array: every
 // caller's arrays are 256-byte aligned) and never read past the last
 // 16-byte pair that holds p[n-1].
-__device__ __forceinline__ double seq_sum(const double *__restrict__ p, long n, double *lds)
+__device__ __forceinline__ double seq_sum(const double *__restrict__ p, long n, double *lds,
+                                          double m)
 {
     const int lane = threadIdx.x & 63;
     const int sh = (int)(((unsigned long)p >> 3) & 1);  // p[0] at position sh of the stream
@@ -218,7 +219,6 @@ __device__ __forceinline__ double seq_sum(const double *__restrict__ p, long n, 
         }
     };
     for (long c = 0; c < kSeqSlots - 1; ++c) issue(c);
-    double m = 0.0;
     for (long c = 0; c < nch; ++c) {
         issue(c + kSeqSlots - 1);
         seq_wait_vmem<(kSeqSlots - 1) * kSeqLoads>();

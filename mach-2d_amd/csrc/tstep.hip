@@ -6,18 +6,16 @@
 //
 // The per-point coefficients (sum of |a_nb| over |a_P|, the sums left to
 // right as the reference's SUM intrinsic adds them) are computed in parallel
-// into a scratch array in the reference's loop order (i outer, j inner); one
-// lane then adds them in that order, so the mean is the reference's bit for
-// bit.  That chain of dependent additions bounds the call (about 10 cycles
-// per point); tstepper_dt runs its four means concurrently.  The minimum of dt0 does not depend on the order and is a parallel
-// reduction.  Entries take host or device arrays (all of one kind); they
+// into a scratch array in the reference's loop order (i outer, j inner), whose
+// sum is the left-to-right loop's bit for bit (seqsum.hip), so the mean is the
+// reference's; tstepper_dt runs its four means in the same launches.  The
+// minimum of dt0 does not depend on the order and is a parallel reduction.  Entries take host or device arrays (all of one kind); they
 // return the value, so they synchronise.
 #include <math.h>
 
 #include <vector>
 
 #include "m2d_internal.h"
-#include "seqsum.h"
 
 using namespace m2d;
 
@@ -25,37 +23,48 @@ namespace {
 
 constexpr int kT = 256;
 
-// term of interior point (i, j) (1-based) -> t[(i-2)*(ny-2) + (j-2)]
-template <int ND>
-__global__ __launch_bounds__(kT) void k_cc_terms(const double *__restrict__ a, int nx, int ny,
+// terms of interior points (i, j) (1-based) -> t[(i-2)*(ny-2) + (j-2)].  The
+// diagonals are read along i and the terms written along j: a 64 x 16 tile
+// goes through LDS, so both are whole cache lines (row width 65: no bank
+// conflicts either way).  Grid row z: array z.
+constexpr int kTi = 64, kTj = 16;
+struct CcArrays {
+    const double *a[4];
+    int nd[4];
+};
+__global__ __launch_bounds__(kT) void k_cc_terms(CcArrays A, int nx, int ny,
                                                 double *__restrict__ t)
 {
-    const int i = blockIdx.x * kT + threadIdx.x + 2, j = blockIdx.y + 2;
-    if (i > nx - 1) return;
-    const long N = (long)nx * ny, np = (long)nx * (j - 1) + i - 1;
-    double s1, s2, ap;
-    if constexpr (ND == 9) {
-        s1 = fabs(a[np]) + fabs(a[N + np]) + fabs(a[2 * N + np]) + fabs(a[3 * N + np]);
-        s2 = fabs(a[5 * N + np]) + fabs(a[6 * N + np]) + fabs(a[7 * N + np]) +
-             fabs(a[8 * N + np]);
-        ap = fabs(a[4 * N + np]);
-    } else {
-        s1 = fabs(a[np]) + fabs(a[N + np]);
-        s2 = fabs(a[3 * N + np]) + fabs(a[4 * N + np]);
-        ap = fabs(a[2 * N + np]);
+    __shared__ double tile[kTj][kTi + 1];
+    const double *__restrict__ a = A.a[blockIdx.z];
+    const int nd = A.nd[blockIdx.z];
+    t += (long)blockIdx.z * ((long)(nx - 2) * (ny - 2));
+    const long N = (long)nx * ny;
+    const int i0 = blockIdx.x * kTi + 2, j0 = blockIdx.y * kTj + 2;
+    const int i = i0 + (threadIdx.x & (kTi - 1));
+#pragma unroll
+    for (int r = threadIdx.x / kTi; r < kTj; r += kT / kTi) {
+        const int j = j0 + r;
+        if (i > nx - 1 || j > ny - 1) continue;
+        const long np = (long)nx * (j - 1) + i - 1;
+        double s1, s2, ap;
+        if (nd == 9) {
+            s1 = fabs(a[np]) + fabs(a[N + np]) + fabs(a[2 * N + np]) + fabs(a[3 * N + np]);
+            s2 = fabs(a[5 * N + np]) + fabs(a[6 * N + np]) + fabs(a[7 * N + np]) +
+                 fabs(a[8 * N + np]);
+            ap = fabs(a[4 * N + np]);
+        } else {
+            s1 = fabs(a[np]) + fabs(a[N + np]);
+            s2 = fabs(a[3 * N + np]) + fabs(a[4 * N + np]);
+            ap = fabs(a[2 * N + np]);
+        }
+        tile[r][threadIdx.x & (kTi - 1)] = (s1 + s2) / ap;
     }
-    t[(long)(i - 2) * (ny - 2) + (j - 2)] = (s1 + s2) / ap;
-}
-
-// m = t(q) + m over the terms in order, then m / n (mean) or m; one
-// workgroup per array of n terms (t + blockIdx.x * n)
-__global__ __launch_bounds__(kSeqThreads) void k_seq_mean(const double *__restrict__ t, long n,
-                                                         double *__restrict__ out, int mean)
-{
-    __shared__ double lds[kSeqSlots * kSeqChunk];
-    const double *__restrict__ tt = t + (long)blockIdx.x * n;
-    const double m = seq_sum(tt, n, lds);
-    if (threadIdx.x == 0) out[blockIdx.x] = mean ? m / (double)n : m;
+    __syncthreads();
+    const int j = j0 + (threadIdx.x & (kTj - 1));
+    if (j > ny - 1) return;
+    for (int c = threadIdx.x / kTj; c < kTi && i0 + c <= nx - 1; c += kT / kTj)
+        t[(long)(i0 + c - 2) * (ny - 2) + (j - 2)] = tile[threadIdx.x & (kTj - 1)][c];
 }
 
 // per-block minimum of 1/sqrt(Jp (u^2 + v^2)) over interior points
@@ -102,11 +111,7 @@ __global__ __launch_bounds__(kT) void k_min(const double *__restrict__ part, lon
 // device copies of host inputs (or the inputs themselves), plus scratch
 struct Staged {
     std::vector<const double *> in;
-    double *buf = nullptr;
-    ~Staged()
-    {
-        if (buf) (void)hipFree(buf);
-    }
+    Scratch buf;
 };
 
 int stage(Staged &S, const std::vector<const double *> &ptrs, const std::vector<long> &lens,
@@ -118,25 +123,25 @@ int stage(Staged &S, const std::vector<const double *> &ptrs, const std::vector<
     long tot = scratch;
     if (!dev)
         for (long n : lens) tot += n;
-    if (hipMalloc((void **)&S.buf, sizeof(double) * (size_t)(tot > 0 ? tot : 1)) != hipSuccess)
-        return M2D_ERR_HIP;
+    double *const buf = S.buf.get((size_t)(tot > 0 ? tot : 1));
+    if (!buf) return M2D_ERR_HIP;
     long off = 0;
     for (size_t k = 0; k < ptrs.size(); ++k) {
         if (dev) {
             S.in.push_back(ptrs[k]);
             continue;
         }
-        if (hipMemcpyAsync(S.buf + off, ptrs[k], sizeof(double) * lens[k], hipMemcpyHostToDevice,
+        if (hipMemcpyAsync(buf + off, ptrs[k], sizeof(double) * lens[k], hipMemcpyHostToDevice,
                            s) != hipSuccess)
             return M2D_ERR_HIP;
-        S.in.push_back(S.buf + off);
+        S.in.push_back(buf + off);
         off += lens[k];
     }
-    *scratch_out = S.buf + off;
+    *scratch_out = buf + off;
     return M2D_OK;
 }
 
-// means of K coefficient arrays (nd[k] diagonals each): the terms of all
+// means of K <= 4 coefficient arrays (nd[k] diagonals each): the terms of all
 // K into one scratch, then K concurrent in-order sums
 int mean_cc(int nx, int ny, int K, const double *const *a, const int *nd, double *out)
 {
@@ -148,14 +153,16 @@ int mean_cc(int nx, int ny, int K, const double *const *a, const int *nd, double
     for (int k = 0; k < K; ++k) lens.push_back(nd[k] * N);
     Staged S;
     double *t = nullptr;
-    int rc = stage(S, ptrs, lens, K * n + K, &t, s);
+    int rc = stage(S, ptrs, lens, K * n + seq_scratch(n, K), &t, s);
     if (rc) return rc;
-    mean_cc_enqueue(nx, ny, K, S.in.data(), nd, t, s);
-    if (hipGetLastError() != hipSuccess ||
-        hipMemcpyAsync(out, t + K * n, sizeof(double) * K, hipMemcpyDeviceToHost, s) !=
-            hipSuccess ||
-        hipStreamSynchronize(s) != hipSuccess)
+    double *const res = Scratch::results();
+    if (!res) return M2D_ERR_HIP;
+    cc_terms_enqueue(nx, ny, K, S.in.data(), nd, t, s);
+    seq_sums_enqueue(t, n, K, res, true, t + K * n, s);
+    if (hipGetLastError() != hipSuccess || hipStreamSynchronize(s) != hipSuccess)
         return M2D_ERR_HIP;
+    S.buf.done();
+    for (int k = 0; k < K; ++k) out[k] = res[k];
     return M2D_OK;
 }
 
@@ -164,27 +171,14 @@ int mean_cc(int nx, int ny, int K, const double *const *a, const int *nd, double
 void m2d::cc_terms_enqueue(int nx, int ny, int K, const double *const *a, const int *nd,
                            double *t, hipStream_t s)
 {
-    const long n = (long)(nx - 2) * (ny - 2);
-    const dim3 grid((unsigned)((nx - 2 + kT - 1) / kT), (unsigned)(ny - 2));
-    for (int k = 0; k < K; ++k) {
-        if (nd[k] == 9)
-            hipLaunchKernelGGL(k_cc_terms<9>, grid, dim3(kT), 0, s, a[k], nx, ny, t + k * n);
-        else
-            hipLaunchKernelGGL(k_cc_terms<5>, grid, dim3(kT), 0, s, a[k], nx, ny, t + k * n);
+    CcArrays A;
+    for (int k = 0; k < 4; ++k) {
+        A.a[k] = a[k < K ? k : 0];
+        A.nd[k] = nd[k < K ? k : 0];
     }
-}
-
-void m2d::seq_sums_enqueue(const double *t, long n, int K, double *out, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_seq_mean, dim3(K), dim3(kSeqThreads), 0, s, t, n, out, 0);
-}
-
-void m2d::mean_cc_enqueue(int nx, int ny, int K, const double *const *a, const int *nd,
-                          double *t, hipStream_t s)
-{
-    const long n = (long)(nx - 2) * (ny - 2);
-    cc_terms_enqueue(nx, ny, K, a, nd, t, s);
-    hipLaunchKernelGGL(k_seq_mean, dim3(K), dim3(kSeqThreads), 0, s, t, n, t + K * n, 1);
+    const dim3 grid((unsigned)((nx - 2 + kTi - 1) / kTi), (unsigned)((ny - 2 + kTj - 1) / kTj),
+                    (unsigned)K);
+    hipLaunchKernelGGL(k_cc_terms, grid, dim3(kT), 0, s, A, nx, ny, t);
 }
 
 // tstepper_dt_scarborough's rule (mod_tstepper_scarborough.f90:80-123) on
@@ -202,6 +196,72 @@ double m2d::scarborough_dt(double dt, const double *cc, double h0, double mincc,
     else
         h = 0.0;
     return dt * (1.0 + h);
+}
+
+// The scratch a host thread keeps between calls (m2d::Scratch).
+namespace {
+struct Kept {
+    double *p = nullptr;
+    size_t n = 0;
+    int dev = -1;
+    bool used = false;
+    ~Kept()
+    {
+        if (p) (void)hipFree(p);
+    }
+};
+thread_local Kept g_kept;
+constexpr size_t kKeepDoubles = (size_t)64 << 17;  // 64 MiB
+}  // namespace
+
+double *m2d::Scratch::get(size_t n)
+{
+    Kept &k = g_kept;
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return nullptr;
+    if (k.used || n > kKeepDoubles)
+        return hipMalloc((void **)&p_, sizeof(double) * n) == hipSuccess ? p_ : nullptr;
+    if (!k.p || k.n < n || k.dev != dev) {
+        if (k.p) (void)hipFree(k.p);
+        k.p = nullptr;
+        k.n = 0;
+        if (hipMalloc((void **)&k.p, sizeof(double) * n) != hipSuccess) {
+            k.p = nullptr;
+            return nullptr;
+        }
+        k.n = n;
+        k.dev = dev;
+    }
+    k.used = kept_ = true;
+    return p_ = k.p;
+}
+
+double *m2d::Scratch::results()
+{
+    struct Pinned {
+        double *p = nullptr;
+        ~Pinned()
+        {
+            if (p) (void)hipHostFree(p);
+        }
+    };
+    thread_local Pinned r;
+    if (!r.p && hipHostMalloc((void **)&r.p, sizeof(double) * kResults, hipHostMallocPortable) !=
+                    hipSuccess)
+        r.p = nullptr;
+    return r.p;
+}
+
+m2d::Scratch::~Scratch()
+{
+    if (!p_) return;
+    if (kept_) g_kept.used = false;
+    if (kept_ && done_) return;
+    (void)hipFree(p_);
+    if (kept_) {
+        g_kept.p = nullptr;
+        g_kept.n = 0;
+    }
 }
 
 void m2d_set_last_status_code(int status);
@@ -251,6 +311,8 @@ extern "C" double m2d_tstepper_dt0_scarborough(const int *nx_, const int *ny_, c
                     hipSuccess ||
                 hipStreamSynchronize(s) != hipSuccess)
                 rc = M2D_ERR_HIP;
+            else
+                S.buf.done();
         }
     }
     m2d_set_last_status_code(rc);

@@ -30,3 +30,46 @@ def test_mean_cc_and_dt_match_oracle(gpu, orc, nx, ny):
         want = orc.dt_scarborough(1.5e-3, au, av, at, ap, nx, ny, 0.25, mincc, maxcc)
         assert tstep.dt(1.5e-3, au, av, at, ap, nx, ny, 0.25, mincc, maxcc) == want
         assert tstep.dt(1.5e-3, *dev, nx, ny, 0.25, mincc, maxcc) == want
+
+
+def _sum_patterns(n, rng):
+    """Arrays of n terms at which a sum in parallel can part from the
+    left-to-right loop: exact ties, zeros, numbers that leave the running
+    sum's binade at every size, subnormals, negative and non-finite terms."""
+    wide = 10.0 ** rng.uniform(-300, 300, n)
+    grow = np.minimum(1.5 ** np.minimum(np.arange(n), 1500), 1e250)
+    some = rng.uniform(0, 1, n)
+    neg, late = rng.normal(size=n), rng.uniform(0, 1, n)
+    late[n // 2:] *= -1.0
+    nan, inf = some.copy(), some.copy()
+    nan[n - 1], inf[n // 3] = np.nan, np.inf
+    lead = some.copy()
+    lead[: (3 * n) // 4] = 0.0
+    lead[::7] = -0.0
+    return {
+        "uniform": some, "constant": np.full(n, 0.1), "integers": np.floor(some * 9.0),
+        "halves": np.floor(some * 9.0) / 2.0 + 2.0 ** 52, "ties": rng.integers(0, 64, n) * 2.0 ** -10 + 2.0 ** -53,
+        "few bits": some.astype(np.float32).astype(np.float64) * 2.0 ** rng.integers(-20, 20, n),
+        "wide": wide, "grow": grow, "zeros": np.zeros(n), "leading zeros": lead,
+        "subnormal": some * 1e-310, "overflow": np.full(n, 1e307), "signed": neg,
+        "signed late": late, "nan": nan, "inf": inf,
+    }
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 255, 256, 257, 511, 513, 4095, 4096, 4097, 4608, 32768,
+                               33291, 66049])
+def test_in_order_sums_are_the_left_to_right_loop(gpu, orc, n):
+    """get_average of n real volumes (nx = n + 2, ny = 3): the oracle's loop
+    bit for bit, for sizes at the edges of the groups of 256 terms, the
+    segments of 512 and the one-launch range (4096)."""
+    import torch
+
+    from mach2d import assembly as A
+    nx, ny = n + 2, 3
+    for name, t in _sum_patterns(n, np.random.default_rng(n)).items():
+        F = np.zeros((ny, nx))
+        F[1, 1:-1] = t
+        with np.errstate(over="ignore", invalid="ignore"):
+            want = orc.get_average(nx, ny, F.reshape(-1))
+        got = A.get_average(nx, ny, torch.tensor(F.reshape(-1), device="cuda"))
+        assert np.array_equal(got, want, equal_nan=True), (name, got, want)
