@@ -27,6 +27,7 @@ namespace m2d {
 namespace unet {
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
+typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
 
 constexpr int kMode0 = 0;     // direct
@@ -48,6 +49,9 @@ struct ConvArgs {
     int n, h, w_;         // output (and direct-input) resolution
     int relu;
     int accumulate;       // add into out32 instead of overwriting
+    int vec;              // outputs can be stored four channels at a time
+    int tiles_x, tiles_y; // k_conv3x3_tile's tiles of one image
+    unsigned rc8;         // div_recip(input channels / 8)
 };
 
 __device__ __forceinline__ bf16x8 zero8()
@@ -99,7 +103,9 @@ __device__ __forceinline__ bf16x8 im2col8(const ConvArgs &A, int p, int k0)
                          : load_in(A.in2, ci0 - A.in1.c, n, y, x, A.h, A.w_);
 }
 
-// Forward convolution (also the input gradient, with rotated weights).
+// Forward convolution (also the input gradient, with rotated weights) of any
+// number of input channels: for those whose staged tile does not fit
+// k_conv3x3_tile's LDS.
 // Workgroup: 4 waves x 16 pixels; wave: 16 pixels x 16*NT output channels.
 template <int NT>
 __global__ __launch_bounds__(256) void k_conv3x3(ConvArgs A)
@@ -141,70 +147,295 @@ __global__ __launch_bounds__(256) void k_conv3x3(ConvArgs A)
     }
 }
 
+// Forward convolution through LDS.  A workgroup computes TH = MT WP rows of
+// 16 pixels x 16 NT WC output channels: it stages the (TH + 2) x 18 pixels of
+// input it needs once (pooling or upsampling them on the way, so a pooled
+// value is formed once and not for each of its nine taps) and its waves, WP
+// along the rows and WC along the channels, read the taps from there.  The
+// weights are the first operand, so a lane ends up with four neighbouring
+// channels of one pixel and stores them at once.  Products are added in the
+// order of k_conv3x3 (32 k at a time), so both give the same bits.
+//   bound: the 16-channel layers of the full resolution by memory (an
+// input and an output tensor), the deep ones by the LDS reads and the few
+// workgroups they have.  A pixel's channels lie an odd number of 16-byte
+// units apart, so 16 lanes' reads meet no bank twice.
+constexpr int kTileW = 16, kHaloW = kTileW + 2;
+
+// channels between two pixels of the staged tile
+__host__ __device__ constexpr int stage_stride(int cin) { return cin + (cin / 8 % 2 ? 0 : 8); }
+// bytes of LDS: the tile, then eight zeros for the k beyond 9 cin
+__host__ __device__ constexpr int stage_bytes(int th, int cin)
+{
+    return ((th + 2) * kHaloW * stage_stride(cin) + 8) * 2;
+}
+
+// q / d for 0 <= q < 2^15, 1 <= d < 2^15, r = ceil(2^31 / d)
+__device__ __forceinline__ int div_small(int q, unsigned r)
+{
+    return (int)(((unsigned long long)(unsigned)q * r) >> 31);
+}
+__host__ __device__ constexpr unsigned div_recip(int d)
+{
+    return (unsigned)(((1ull << 31) + d - 1) / d);
+}
+
+// stage rows y0 - 1 .. y0 + th, columns x0 - 1 .. x0 + 16 of image n into
+// tile; zeros outside the image
+__device__ __forceinline__ void stage_tile(const ConvArgs &A, __bf16 *tile, int th, int n, int y0,
+                                           int x0, int cs)
+{
+    const int c8 = (A.in1.c + A.in2.c) >> 3, c18 = A.in1.c >> 3;
+    const unsigned rw = div_recip(kHaloW);
+    const int total = (th + 2) * kHaloW * c8;
+    for (int q = threadIdx.x; q < total; q += 256) {
+        const int px = div_small(q, A.rc8), cg = q - px * c8;
+        const int ty = div_small(px, rw), tx = px - ty * kHaloW;
+        const int y = y0 + ty - 1, x = x0 + tx - 1;
+        bf16x8 v = zero8();
+        if (y >= 0 && y < A.h && x >= 0 && x < A.w_)
+            v = cg < c18 ? load_in(A.in1, 8 * cg, n, y, x, A.h, A.w_)
+                         : load_in(A.in2, 8 * (cg - c18), n, y, x, A.h, A.w_);
+        *reinterpret_cast<bf16x8 *>(tile + px * cs + 8 * cg) = v;
+    }
+}
+
+template <int NT, int MT, int WP, int WC>
+__global__ __launch_bounds__(256) void k_conv3x3_tile(ConvArgs A)
+{
+    static_assert(WP * WC == 4, "four waves");
+    constexpr int TH = MT * WP;
+    extern __shared__ __attribute__((aligned(16))) __bf16 tile[];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int wp = wave % WP, wc = wave / WP;
+    const int row = blockIdx.x / A.tiles_x, x0 = (blockIdx.x - row * A.tiles_x) * kTileW;
+    const int n = row / A.tiles_y, y0 = (row - n * A.tiles_y) * TH;
+    const int cin = A.in1.c + A.in2.c, c8 = cin >> 3, cs = stage_stride(cin);
+    const int zero_at = (TH + 2) * kHaloW * cs;
+    const int co0 = (blockIdx.y * WC + wc) * 16 * NT;
+    if (threadIdx.x == 0) *reinterpret_cast<bf16x8 *>(tile + zero_at) = zero8();
+    stage_tile(A, tile, TH, n, y0, x0, cs);
+    __syncthreads();
+
+    const int px = lane & 15, kg = lane >> 4;
+    f32x4 acc[NT][MT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) acc[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const __bf16 *wrow = A.w + (long)(co0 + px) * A.kpad + 8 * kg;
+    const __bf16 *base = tile + (wp * MT * kHaloW + px) * cs;
+#pragma unroll 2
+    for (int kb = 0; kb < A.kpad; kb += 32) {
+        // the eight k of this lane: one tap, eight channels
+        const int k8 = (kb >> 3) + kg;
+        const int tap = div_small(k8, A.rc8);
+        const int ky = (tap * 11) >> 5;  // tap / 3 for tap < 16
+        const int off = ((ky * kHaloW + (tap - 3 * ky)) * cs) + 8 * (k8 - tap * c8);
+        bf16x8 w[NT], x[MT];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) w[t] = ld8(wrow + (long)t * 16 * A.kpad + kb);
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+            x[m] = ld8(tap < 9 ? base + m * kHaloW * cs + off : tile + zero_at);
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+                acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t], x[m], acc[t][m], 0, 0, 0);
+    }
+
+    const int xo = x0 + px;
+    if (xo >= A.w_) return;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        const int co = co0 + 16 * t + 4 * kg;  // this lane's four channels
+        if (co >= A.cout) continue;
+        float bias[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) bias[i] = A.bias && co + i < A.cout ? A.bias[co + i] : 0.0f;
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            const int yo = y0 + wp * MT + m;
+            if (yo >= A.h) continue;
+            const long o = (((long)n * A.h + yo) * A.w_ + xo) * A.cout_stride + co;
+            float v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                v[i] = acc[t][m][i] + bias[i];
+                if (A.relu) v[i] = fmaxf(v[i], 0.0f);
+            }
+            if (A.vec) {  // four channels, aligned
+                if (A.out) {
+                    bf16x4 r;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) r[i] = (__bf16)v[i];
+                    *reinterpret_cast<bf16x4 *>(A.out + o) = r;
+                }
+                if (A.out32) {
+                    f32x4 *d = reinterpret_cast<f32x4 *>(A.out32 + o);
+                    f32x4 r = {v[0], v[1], v[2], v[3]};
+                    if (A.accumulate) r = *d + r;
+                    *d = r;
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    if (co + i >= A.cout) continue;
+                    if (A.out) A.out[o + i] = (__bf16)v[i];
+                    if (A.out32) A.out32[o + i] = A.accumulate ? A.out32[o + i] + v[i] : v[i];
+                }
+            }
+        }
+    }
+}
+
 // Weight gradient dW[co][k] += sum_p G[p][co] * im2col(p, k): M = output
-// channels, N = k, K = pixels.  One wave per (16 co, 16 k, pixel range);
-// partial sums leave with FP32 atomics.
+// channels, N = k, K = pixels, so both operands want eight neighbouring
+// pixels of one channel where the tensors hold eight channels of one pixel.
+// A workgroup owns 16 input channels (all nine taps of them) and 16 MF output
+// channels and goes through its share of the tiles of 16 x 8 pixels: it
+// stages the input transposed into LDS, once per tap column so that every
+// read is eight aligned pixels, and the gradient transposed, and each wave
+// adds two of the tile's rows (32 pixels) into 9 MF accumulators.  At the end
+// the four waves' sums meet in LDS and leave with one FP32 atomic each.
+//   bound: the staging's two-byte LDS writes; before, every lane fetched
+// every element of both operands from memory by itself.
+constexpr int kGradH = 8;
+constexpr int kGradRow = 16 + 8;                      // pixels between two staged rows
+constexpr int kGradX = (kGradH + 2) * kGradRow + 8;   // ... two channels (input)
+constexpr int kGradG = kGradH * kTileW + 8;           // ... two channels (gradient)
+
 struct WgradArgs {
     ConvArgs c;          // inputs and geometry of the forward convolution
     const __bf16 *g;     // gradient at the convolution's output (pre-activation), cout channels
     float *dw;           // [cout_pad][kpad]
     float *db;           // cout values, or null
-    int pix_per_block;
+    int tiles_x, tiles_y, tiles;
+    int gvec;            // g can be read eight channels at a time
 };
 
-__global__ __launch_bounds__(64) void k_conv3x3_wgrad(WgradArgs W)
+template <int MF>
+__global__ __launch_bounds__(256) void k_conv3x3_wgrad(WgradArgs W)
 {
+    constexpr int kLds = 3 * 16 * kGradX + 16 * MF * kGradG;
+    static_assert(kLds * 2 >= 9 * MF * 64 * 16, "a wave's sums pass through the same LDS");
+    __shared__ __attribute__((aligned(16))) __bf16 lds[kLds];
+    __bf16 *const xt = lds, *const gt = lds + 3 * 16 * kGradX;
     const ConvArgs &A = W.c;
-    const int lane = threadIdx.x;
-    const int k0 = blockIdx.x * 16, co0 = blockIdx.y * 16;
-    const int npix = A.n * A.h * A.w_;
-    const int p_begin = blockIdx.z * W.pix_per_block;
-    const int p_end = min(npix, p_begin + W.pix_per_block);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int ci0 = blockIdx.x * 16, co0 = blockIdx.y * 16 * MF;
     const int cin = A.in1.c + A.in2.c;
-    const int co = co0 + (lane & 15), kk = k0 + (lane & 15);
-    const int pl = 8 * (lane >> 4);
-    const bool co_ok = co < A.cout;
-    // the k column of this lane as (tap, channel group); 8 pixels at a time
-    const bool k_ok = kk < 9 * cin;
-    const int tap = k_ok ? kk / cin : 0, ci = k_ok ? kk - tap * cin : 0;
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    float bsum = 0.0f;
-    for (int p0 = p_begin; p0 < p_end; p0 += 32) {
-        bf16x8 a, b;
+    const int l16 = lane & 15, kg = lane >> 4;
+    f32x4 acc[9][MF];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int p = p0 + pl + i;
-            const bool ok = p < p_end;
-            a[i] = (ok && co_ok) ? W.g[(long)p * A.cout + co] : (__bf16)0.0f;
-            __bf16 x = (__bf16)0.0f;
-            if (ok && k_ok) {
-                const int hw = A.h * A.w_;
-                const int n = p / hw, rem = p - n * hw, y0 = rem / A.w_, x0 = rem - y0 * A.w_;
-                const int y = y0 + tap / 3 - 1, xx = x0 + tap % 3 - 1;
-                if (y >= 0 && y < A.h && xx >= 0 && xx < A.w_) {
-                    const int cg = ci & ~7;
-                    const bf16x8 v = ci < A.in1.c ? load_in(A.in1, cg, n, y, xx, A.h, A.w_)
-                                                  : load_in(A.in2, cg - A.in1.c, n, y, xx,
-                                                            A.h, A.w_);
-                    x = v[ci & 7];
+    for (int t = 0; t < 9; ++t)
+#pragma unroll
+        for (int m = 0; m < MF; ++m) acc[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float bsum[MF];
+#pragma unroll
+    for (int m = 0; m < MF; ++m) bsum[m] = 0.0f;
+    const bool bias = W.db && blockIdx.x == 0;
+
+    for (int tile = blockIdx.z; tile < W.tiles; tile += gridDim.z) {
+        const int n = tile / (W.tiles_x * W.tiles_y), r = tile - n * W.tiles_x * W.tiles_y;
+        const int ty = r / W.tiles_x, y0 = ty * kGradH, x0 = (r - ty * W.tiles_x) * kTileW;
+        __syncthreads();
+        for (int q = threadIdx.x; q < 2 * (kGradH + 2) * kHaloW; q += 256) {
+            const int cg = q / ((kGradH + 2) * kHaloW), px = q - cg * (kGradH + 2) * kHaloW;
+            const int sy = px / kHaloW, sx = px - sy * kHaloW;
+            const int y = y0 + sy - 1, x = x0 + sx - 1, ci = ci0 + 8 * cg;
+            bf16x8 v = zero8();
+            if (ci < cin && y >= 0 && y < A.h && x >= 0 && x < A.w_)
+                v = ci < A.in1.c ? load_in(A.in1, ci, n, y, x, A.h, A.w_)
+                                 : load_in(A.in2, ci - A.in1.c, n, y, x, A.h, A.w_);
+#pragma unroll
+            for (int kx = 0; kx < 3; ++kx) {
+                const int p = sx - kx;
+                if (p < 0 || p >= kTileW) continue;
+                __bf16 *d = xt + (kx * 16 + 8 * cg) * kGradX + sy * kGradRow + p;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) d[i * kGradX] = v[i];
+            }
+        }
+        for (int q = threadIdx.x; q < 2 * MF * kGradH * kTileW; q += 256) {
+            const int cg = q / (kGradH * kTileW), px = q - cg * kGradH * kTileW;
+            const int y = y0 + px / kTileW, x = x0 + px % kTileW, co = co0 + 8 * cg;
+            bf16x8 v = zero8();
+            if (y < A.h && x < A.w_ && co < A.cout) {
+                const __bf16 *g = W.g + (((long)n * A.h + y) * A.w_ + x) * A.cout + co;
+                if (W.gvec) {
+                    v = ld8(g);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 8; ++i)
+                        if (co + i < A.cout) v[i] = g[i];
                 }
             }
-            b[i] = x;
-            if (W.db && blockIdx.x == 0) bsum += (float)a[i];
-        }
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
-    }
-    // D[m][n]: lane holds n = lane%16 (k), m = 4*(lane/16) + i (co)
+            __bf16 *d = gt + 8 * cg * kGradG + px;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int com = co0 + 4 * (lane >> 4) + i, kn = k0 + (lane & 15);
-        if (com < A.cout && kn < A.kpad) atomicAdd(&W.dw[(long)com * A.kpad + kn], acc[i]);
+            for (int i = 0; i < 8; ++i) d[i * kGradG] = v[i];
+        }
+        __syncthreads();
+        // this wave's rows 2 wave and 2 wave + 1; the lane's eight pixels
+        const int row = 2 * wave + (kg >> 1), col = 8 * (kg & 1);
+        bf16x8 g[MF];
+#pragma unroll
+        for (int m = 0; m < MF; ++m) {
+            g[m] = ld8(gt + (16 * m + l16) * kGradG + row * kTileW + col);
+            if (bias) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) bsum[m] += (float)g[m][i];
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < 9; ++t) {
+            const bf16x8 x = ld8(xt + ((t % 3) * 16 + l16) * kGradX + (row + t / 3) * kGradRow + col);
+#pragma unroll
+            for (int m = 0; m < MF; ++m)
+                acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(g[m], x, acc[t][m], 0, 0, 0);
+        }
     }
-    if (W.db && blockIdx.x == 0) {
+    // the other waves' sums into wave 0's
+    f32x4 *const red = reinterpret_cast<f32x4 *>(lds);
+    for (int src = 1; src < 4; ++src) {
+        __syncthreads();
+        if (wave == src) {
+#pragma unroll
+            for (int t = 0; t < 9; ++t)
+#pragma unroll
+                for (int m = 0; m < MF; ++m) red[(t * MF + m) * 64 + lane] = acc[t][m];
+        }
+        __syncthreads();
+        if (wave == 0) {
+#pragma unroll
+            for (int t = 0; t < 9; ++t)
+#pragma unroll
+                for (int m = 0; m < MF; ++m) acc[t][m] += red[(t * MF + m) * 64 + lane];
+        }
+    }
+    // D[m][n]: lane holds n = lane % 16 (ci), m = 4 (lane / 16) + i (co)
+    if (wave == 0 && ci0 + l16 < cin) {
+#pragma unroll
+        for (int t = 0; t < 9; ++t)
+#pragma unroll
+            for (int m = 0; m < MF; ++m)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int co = co0 + 16 * m + 4 * kg + i;
+                    if (co < A.cout)
+                        atomicAdd(&W.dw[(long)co * A.kpad + t * cin + ci0 + l16], acc[t][m][i]);
+                }
+    }
+    if (bias) {
         // lanes l, l+16, l+32, l+48 hold partial sums of channel co0 + l%16
-        bsum += __shfl_xor(bsum, 16);
-        bsum += __shfl_xor(bsum, 32);
-        if (lane < 16 && co_ok) atomicAdd(&W.db[co], bsum);
+#pragma unroll
+        for (int m = 0; m < MF; ++m) {
+            float s = bsum[m];
+            s += __shfl_xor(s, 16);
+            s += __shfl_xor(s, 32);
+            const int co = co0 + 16 * m + l16;
+            if (lane < 16 && co < A.cout) atomicAdd(&W.db[co], s);
+        }
     }
 }
 
@@ -417,10 +648,31 @@ extern "C" int m2d_unet_conv3x3(const void *in1, int c1, int mode1, const void *
     A.accumulate = accumulate;
     const long npix = (long)n * h * w_;
     if (npix > 0x7fffffffL / 2) return M2D_ERR_ARG;
+    A.vec = cout % 4 == 0 && cout_stride % 4 == 0 && ((uintptr_t)out & 7) == 0 &&
+            ((uintptr_t)out32 & 15) == 0;
     const int cpad = (cout + 15) / 16 * 16;  // weight rows available: cout rounded to 16
-    const int nt = cpad >= 64 && cpad % 64 == 0 ? 4 : cpad % 32 == 0 ? 2 : 1;
+    const hipStream_t s = (hipStream_t)stream;
+    // 64 channels per workgroup where the weights have them (the input is
+    // staged once for all of them), else 32, else 16; fewer rows per tile with
+    // 64, whose tensors are the small ones
+    const int nt = cpad % 64 == 0 ? 4 : cpad % 32 == 0 ? 2 : 1;
+    const int th = nt == 4 ? 4 : 8;
+    const int lds = stage_bytes(th, cin);
+    if (lds <= 64 * 1024) {
+        A.tiles_x = (w_ + kTileW - 1) / kTileW;
+        A.tiles_y = (h + th - 1) / th;
+        A.rc8 = div_recip(cin / 8);
+        const long tiles = (long)A.tiles_x * A.tiles_y * n;  // below npix
+        const dim3 grid((unsigned)tiles, (unsigned)(cpad / (16 * nt)));
+        if (nt == 4)
+            hipLaunchKernelGGL((k_conv3x3_tile<2, 2, 2, 2>), grid, dim3(256), lds, s, A);
+        else if (nt == 2)
+            hipLaunchKernelGGL((k_conv3x3_tile<2, 2, 4, 1>), grid, dim3(256), lds, s, A);
+        else
+            hipLaunchKernelGGL((k_conv3x3_tile<1, 2, 4, 1>), grid, dim3(256), lds, s, A);
+        return rc_of(hipGetLastError());
+    }
     dim3 grid((unsigned)((npix + 63) / 64), (unsigned)(cpad / (16 * nt)));
-    hipStream_t s = (hipStream_t)stream;
     if (nt == 4)
         hipLaunchKernelGGL(k_conv3x3<4>, grid, dim3(256), 0, s, A);
     else if (nt == 2)
@@ -450,11 +702,27 @@ extern "C" int m2d_unet_conv3x3_wgrad(const void *in1, int c1, int mode1, const 
     W.g = (const __bf16 *)g;
     W.dw = dw;
     W.db = db;
-    const long npix = (long)n * h * w_;
-    W.pix_per_block = 2048;
-    dim3 grid((unsigned)((9 * cin + 15) / 16), (unsigned)((cout + 15) / 16),
-              (unsigned)((npix + W.pix_per_block - 1) / W.pix_per_block));
-    hipLaunchKernelGGL(k_conv3x3_wgrad, grid, dim3(64), 0, (hipStream_t)stream, W);
+    W.gvec = cout % 8 == 0 && aligned16(g);
+    W.tiles_x = (w_ + kTileW - 1) / kTileW;
+    W.tiles_y = (h + kGradH - 1) / kGradH;
+    const long tiles = (long)W.tiles_x * W.tiles_y * n;
+    if (tiles > 0x7fffffffL) return M2D_ERR_ARG;
+    W.tiles = (int)tiles;
+    // 64 output channels per workgroup where there are as many, and enough
+    // shares of the tiles for about four workgroups per CU: fewer leave CUs
+    // idle, more only add atomics
+    const int mf = cout > 32 ? 4 : cout > 16 ? 2 : 1;
+    const int gx = (cin + 15) / 16, gy = (cout + 16 * mf - 1) / (16 * mf);
+    long gz = (1024 + gx * gy - 1) / (gx * gy);
+    gz = gz < tiles ? gz : tiles;
+    const dim3 grid((unsigned)gx, (unsigned)gy, (unsigned)gz);
+    const hipStream_t s = (hipStream_t)stream;
+    if (mf == 4)
+        hipLaunchKernelGGL(k_conv3x3_wgrad<4>, grid, dim3(256), 0, s, W);
+    else if (mf == 2)
+        hipLaunchKernelGGL(k_conv3x3_wgrad<2>, grid, dim3(256), 0, s, W);
+    else
+        hipLaunchKernelGGL(k_conv3x3_wgrad<1>, grid, dim3(256), 0, s, W);
     return rc_of(hipGetLastError());
 }
 
