@@ -20,6 +20,8 @@
 #include <math.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "m2d_internal.h"
 #include "msi_stencil.h"
 
@@ -51,7 +53,7 @@ struct ConvArgs {
     int accumulate;       // add into out32 instead of overwriting
     int vec;              // outputs can be stored four channels at a time
     int tiles_x, tiles_y; // k_conv3x3_tile's tiles of one image
-    unsigned rc8;         // div_recip(input channels / 8)
+    unsigned rc8, rc1, rc2;  // div_recip(channels / 8): both inputs', each one's
 };
 
 __device__ __forceinline__ bf16x8 zero8()
@@ -169,37 +171,101 @@ __host__ __device__ constexpr int stage_bytes(int th, int cin)
     return ((th + 2) * kHaloW * stage_stride(cin) + 8) * 2;
 }
 
-// q / d for 0 <= q < 2^15, 1 <= d < 2^15, r = ceil(2^31 / d)
+// q / d for 0 <= q < 2^16, 2 <= d < 2^16, r = ceil(2^32 / d) (d = 1: r = 0)
 __device__ __forceinline__ int div_small(int q, unsigned r)
 {
-    return (int)(((unsigned long long)(unsigned)q * r) >> 31);
+    return r ? (int)__umulhi((unsigned)q, r) : q;
 }
 __host__ __device__ constexpr unsigned div_recip(int d)
 {
-    return (unsigned)(((1ull << 31) + d - 1) / d);
+    return d > 1 ? (unsigned)(((1ull << 32) + d - 1) / d) : 0u;
 }
 
-// stage rows y0 - 1 .. y0 + th, columns x0 - 1 .. x0 + 16 of image n into
-// tile; zeros outside the image
-__device__ __forceinline__ void stage_tile(const ConvArgs &A, __bf16 *tile, int th, int n, int y0,
-                                           int x0, int cs)
+// One image of an input, at the output resolution h x w.
+struct Image {
+    const __bf16 *x;
+    int c, h, w;
+};
+__device__ __forceinline__ Image image_of(const In &in, int n, int h, int w)
 {
-    const int c8 = (A.in1.c + A.in2.c) >> 3, c18 = A.in1.c >> 3;
-    const unsigned rw = div_recip(kHaloW);
-    const int total = (th + 2) * kHaloW * c8;
-    for (int q = threadIdx.x; q < total; q += 256) {
-        const int px = div_small(q, A.rc8), cg = q - px * c8;
-        const int ty = div_small(px, rw), tx = px - ty * kHaloW;
-        const int y = y0 + ty - 1, x = x0 + tx - 1;
-        bf16x8 v = zero8();
-        if (y >= 0 && y < A.h && x >= 0 && x < A.w_)
-            v = cg < c18 ? load_in(A.in1, 8 * cg, n, y, x, A.h, A.w_)
-                         : load_in(A.in2, 8 * (cg - c18), n, y, x, A.h, A.w_);
-        *reinterpret_cast<bf16x8 *>(tile + px * cs + 8 * cg) = v;
+    const long px = in.mode == kModePool ? 4l * h * w
+                    : in.mode == kModeUp ? (long)(h >> 1) * (w >> 1)
+                                         : (long)h * w;
+    return Image{in.x + px * in.c * n, in.c, h, w};
+}
+// load_in's eight channels ci.. at pixel (y, x), zeros outside the image or
+// without ok.  No branch: the image's first channels are read instead and
+// dropped, so a lane's loads are all under way together.
+template <int MODE>
+__device__ __forceinline__ bf16x8 load_at(const Image &I, int ci, int y, int x, bool ok)
+{
+    typedef __attribute__((__vector_size__(16))) unsigned u32x4;
+    ok = ok && (unsigned)y < (unsigned)I.h && (unsigned)x < (unsigned)I.w;
+    bf16x8 v;
+    if constexpr (MODE == kModePool) {
+        const int wf = 2 * I.w;
+        const __bf16 *p = I.x + (ok ? (2l * y * wf + 2 * x) * I.c + ci : 0l);
+        const bf16x8 a = ld8(p), b = ld8(p + I.c), c = ld8(p + (long)wf * I.c),
+                     d = ld8(p + (long)wf * I.c + I.c);
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            v[i] = (__bf16)((((float)a[i] + (float)b[i]) + ((float)c[i] + (float)d[i])) * 0.25f);
+    } else if constexpr (MODE == kModeUp) {
+        v = ld8(I.x + (ok ? ((long)(y >> 1) * (I.w >> 1) + (x >> 1)) * I.c + ci : 0l));
+    } else {
+        v = ld8(I.x + (ok ? ((long)y * I.w + x) * I.c + ci : 0l));
+    }
+    const unsigned keep = ok ? 0xffffffffu : 0u;
+    return (bf16x8)((u32x4)v & keep);
+}
+
+// stage the groups of eight channels of one input, rows y0 - 1 .. y0 + TH,
+// columns x0 - 1 .. x0 + 16, into tile (first pixel's first channel there),
+// U groups of a lane under way together
+template <int TH, int MODE>
+__device__ __forceinline__ void stage_input(const Image &I, __bf16 *tile, unsigned rc8, int y0,
+                                            int x0, int cs)
+{
+    constexpr int U = MODE == kModePool ? 2 : 4;
+    const int c8 = I.c >> 3, total = (TH + 2) * kHaloW * c8;
+    constexpr unsigned rw = div_recip(kHaloW);
+    for (int q0 = threadIdx.x; q0 < total; q0 += 256 * U) {
+        bf16x8 v[U];
+        int at[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int q = q0 + 256 * u;
+            const int px = div_small(q, rc8), cg = q - px * c8;
+            const int ty = div_small(px, rw), tx = px - ty * kHaloW;
+            at[u] = px * cs + 8 * cg;
+            v[u] = load_at<MODE>(I, 8 * cg, y0 + ty - 1, x0 + tx - 1, q < total);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (q0 + 256 * u < total) *reinterpret_cast<bf16x8 *>(tile + at[u]) = v[u];
     }
 }
 
-template <int NT, int MT, int WP, int WC>
+template <int TH>
+__device__ __forceinline__ void stage_tile(const ConvArgs &A, __bf16 *tile, int n, int y0, int x0,
+                                           int cs)
+{
+    const Image I = image_of(A.in1, n, A.h, A.w_);
+    if (A.in1.mode == kModePool)
+        stage_input<TH, kModePool>(I, tile, A.rc1, y0, x0, cs);
+    else if (A.in1.mode == kModeUp)
+        stage_input<TH, kModeUp>(I, tile, A.rc1, y0, x0, cs);
+    else
+        stage_input<TH, kMode0>(I, tile, A.rc1, y0, x0, cs);
+    if (A.in2.c)
+        stage_input<TH, kMode0>(image_of(A.in2, n, A.h, A.w_), tile + A.in1.c, A.rc2, y0, x0, cs);
+}
+
+// C8 > 0: input channels / 8 known when compiled, so the taps' places in the
+// tile are constants (with C8 a multiple of four the same for the whole
+// wave, else one of four by the lane's group); 0: from A, computed for every
+// 32 k.
+template <int NT, int MT, int WP, int WC, int C8>
 __global__ __launch_bounds__(256) void k_conv3x3_tile(ConvArgs A)
 {
     static_assert(WP * WC == 4, "four waves");
@@ -209,12 +275,11 @@ __global__ __launch_bounds__(256) void k_conv3x3_tile(ConvArgs A)
     const int wp = wave % WP, wc = wave / WP;
     const int row = blockIdx.x / A.tiles_x, x0 = (blockIdx.x - row * A.tiles_x) * kTileW;
     const int n = row / A.tiles_y, y0 = (row - n * A.tiles_y) * TH;
-    const int cin = A.in1.c + A.in2.c, c8 = cin >> 3, cs = stage_stride(cin);
+    const int c8 = C8 ? C8 : (A.in1.c + A.in2.c) >> 3, cs = stage_stride(8 * c8);
     const int zero_at = (TH + 2) * kHaloW * cs;
     const int co0 = (blockIdx.y * WC + wc) * 16 * NT;
     if (threadIdx.x == 0) *reinterpret_cast<bf16x8 *>(tile + zero_at) = zero8();
-    stage_tile(A, tile, TH, n, y0, x0, cs);
-    __syncthreads();
+    stage_tile<TH>(A, tile, n, y0, x0, cs);
 
     const int px = lane & 15, kg = lane >> 4;
     f32x4 acc[NT][MT];
@@ -224,24 +289,63 @@ __global__ __launch_bounds__(256) void k_conv3x3_tile(ConvArgs A)
         for (int m = 0; m < MT; ++m) acc[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
     const __bf16 *wrow = A.w + (long)(co0 + px) * A.kpad + 8 * kg;
     const __bf16 *base = tile + (wp * MT * kHaloW + px) * cs;
-#pragma unroll 2
-    for (int kb = 0; kb < A.kpad; kb += 32) {
-        // the eight k of this lane: one tap, eight channels
-        const int k8 = (kb >> 3) + kg;
-        const int tap = div_small(k8, A.rc8);
-        const int ky = (tap * 11) >> 5;  // tap / 3 for tap < 16
-        const int off = ((ky * kHaloW + (tap - 3 * ky)) * cs) + 8 * (k8 - tap * c8);
-        bf16x8 w[NT], x[MT];
+    // place of the eight channels k = 8 k8 .. in the tile, from base
+    auto place = [&](int k8) {
+        const int tap = C8 ? k8 / (C8 ? C8 : 1) : div_small(k8, A.rc8);
+        const int ky = C8 ? tap / 3 : (tap * 11) >> 5;  // tap / 3 for tap < 16
+        return ((ky * kHaloW + (tap - 3 * ky)) * cs) + 8 * (k8 - tap * c8);
+    };
+    // weights are read AHEAD steps of 32 k before their products
+    constexpr int AHEAD = 4;
+    bf16x8 w[AHEAD][NT];
+    auto fetch = [&](int slot, int kb) {
 #pragma unroll
-        for (int t = 0; t < NT; ++t) w[t] = ld8(wrow + (long)t * 16 * A.kpad + kb);
+        for (int t = 0; t < NT; ++t) w[slot][t] = ld8(wrow + (long)t * 16 * A.kpad + kb);
+    };
+    auto step = [&](int slot, int off, bool some) {
+        bf16x8 x[MT];
 #pragma unroll
-        for (int m = 0; m < MT; ++m)
-            x[m] = ld8(tap < 9 ? base + m * kHaloW * cs + off : tile + zero_at);
+        for (int m = 0; m < MT; ++m) x[m] = ld8(some ? base + m * kHaloW * cs + off : tile + zero_at);
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
             for (int m = 0; m < MT; ++m)
-                acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t], x[m], acc[t][m], 0, 0, 0);
+                acc[t][m] =
+                    __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[slot][t], x[m], acc[t][m], 0, 0, 0);
+    };
+    if constexpr (C8 == 0) {
+        const int last = A.kpad - 32;
+#pragma unroll
+        for (int s = 0; s < AHEAD; ++s) fetch(s, 32 * s < last ? 32 * s : last);
+        __syncthreads();
+        for (int kb = 0; kb < A.kpad; kb += 32 * AHEAD) {
+#pragma unroll
+            for (int s = 0; s < AHEAD; ++s) {
+                const int k = kb + 32 * s, k8 = (k >> 3) + kg;
+                if (k < A.kpad) step(s, place(k8), k8 < 9 * c8);
+                fetch(s, k + 32 * AHEAD < last ? k + 32 * AHEAD : last);
+            }
+        }
+    } else {
+        constexpr int STEPS = (72 * C8 + 31) / 32;
+#pragma unroll
+        for (int s = 0; s < AHEAD && s < STEPS; ++s) fetch(s, 32 * s);
+        __syncthreads();
+        if constexpr (C8 % 4 == 0) base += 8 * kg;
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s) {
+            const int k8 = 4 * s;
+            if constexpr (C8 % 4 == 0) {
+                step(s % AHEAD, place(k8), true);
+            } else {
+                const int off = kg < 2 ? (kg == 0 ? place(k8) : place(k8 + 1))
+                                       : (kg == 2 ? place(k8 + 2) : place(k8 + 3));
+                step(s % AHEAD, off, k8 + 4 <= 9 * C8 || k8 + kg < 9 * C8);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (s + AHEAD < STEPS) fetch(s % AHEAD, 32 * (s + AHEAD));
+            __builtin_amdgcn_sched_barrier(0);
+        }
     }
 
     const int xo = x0 + px;
@@ -293,17 +397,39 @@ __global__ __launch_bounds__(256) void k_conv3x3_tile(ConvArgs A)
 // channels, N = k, K = pixels, so both operands want eight neighbouring
 // pixels of one channel where the tensors hold eight channels of one pixel.
 // A workgroup owns 16 input channels (all nine taps of them) and 16 MF output
-// channels and goes through its share of the tiles of 16 x 8 pixels: it
-// stages the input transposed into LDS, once per tap column so that every
-// read is eight aligned pixels, and the gradient transposed, and each wave
-// adds two of the tile's rows (32 pixels) into 9 MF accumulators.  At the end
-// the four waves' sums meet in LDS and leave with one FP32 atomic each.
+// channels and goes through its share of the tiles of 16 x 16 pixels: it
+// stages input and gradient transposed into LDS, and each wave adds two of the
+// tile's rows (32 pixels) into 9 MF accumulators.  The three taps of a row
+// come from one read of ten pixels, shifted in registers.  The next tile's
+// loads are under way while a tile is computed.  At the end the waves'
+// sums meet in LDS and leave with one FP32 atomic each.
 //   bound: the staging's two-byte LDS writes; before, every lane fetched
 // every element of both operands from memory by itself.
-constexpr int kGradH = 8;
+constexpr int kGradH = 16, kGradWaves = kGradH / 2, kGradThreads = 64 * kGradWaves;
 constexpr int kGradRow = 16 + 8;                      // pixels between two staged rows
 constexpr int kGradX = (kGradH + 2) * kGradRow + 8;   // ... two channels (input)
 constexpr int kGradG = kGradH * kTileW + 8;           // ... two channels (gradient)
+
+// pixels p + 1 .. p + 8 of eight pixels p .. and the two after them
+__device__ __forceinline__ bf16x8 shift_one(bf16x8 v, unsigned next)
+{
+    typedef __attribute__((__vector_size__(16))) unsigned u32x4;
+    const u32x4 a = (u32x4)v;
+    u32x4 r;
+    r[0] = __builtin_amdgcn_alignbit(a[1], a[0], 16);
+    r[1] = __builtin_amdgcn_alignbit(a[2], a[1], 16);
+    r[2] = __builtin_amdgcn_alignbit(a[3], a[2], 16);
+    r[3] = __builtin_amdgcn_alignbit(next, a[3], 16);
+    return (bf16x8)r;
+}
+// pixels p + 2 .. p + 9
+__device__ __forceinline__ bf16x8 shift_two(bf16x8 v, unsigned next)
+{
+    typedef __attribute__((__vector_size__(16))) unsigned u32x4;
+    const u32x4 a = (u32x4)v;
+    const u32x4 r = {a[1], a[2], a[3], next};
+    return (bf16x8)r;
+}
 
 struct WgradArgs {
     ConvArgs c;          // inputs and geometry of the forward convolution
@@ -311,16 +437,16 @@ struct WgradArgs {
     float *dw;           // [cout_pad][kpad]
     float *db;           // cout values, or null
     int tiles_x, tiles_y, tiles;
-    int gvec;            // g can be read eight channels at a time
 };
 
-template <int MF>
-__global__ __launch_bounds__(256) void k_conv3x3_wgrad(WgradArgs W)
+// MODE: the first input's; VEC: cout a multiple of eight, g aligned
+template <int MF, int MODE, bool VEC>
+__global__ __launch_bounds__(kGradThreads) void k_conv3x3_wgrad(WgradArgs W)
 {
-    constexpr int kLds = 3 * 16 * kGradX + 16 * MF * kGradG;
-    static_assert(kLds * 2 >= 9 * MF * 64 * 16, "a wave's sums pass through the same LDS");
+    constexpr int kStage = 16 * kGradX + 16 * MF * kGradG, kSums = 9 * MF * 64 * 8;
+    constexpr int kLds = kStage > kSums ? kStage : kSums;
     __shared__ __attribute__((aligned(16))) __bf16 lds[kLds];
-    __bf16 *const xt = lds, *const gt = lds + 3 * 16 * kGradX;
+    __bf16 *const xt = lds, *const gt = lds + 16 * kGradX;
     const ConvArgs &A = W.c;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int ci0 = blockIdx.x * 16, co0 = blockIdx.y * 16 * MF;
@@ -336,46 +462,80 @@ __global__ __launch_bounds__(256) void k_conv3x3_wgrad(WgradArgs W)
     for (int m = 0; m < MF; ++m) bsum[m] = 0.0f;
     const bool bias = W.db && blockIdx.x == 0;
 
-    for (int tile = blockIdx.z; tile < W.tiles; tile += gridDim.z) {
+    // what this thread stages of every tile: up to NX groups of eight input
+    // channels of a halo pixel and NG of eight gradient channels of a pixel
+    constexpr int kHalo = (kGradH + 2) * kHaloW;
+    constexpr int NX = (2 * kHalo + kGradThreads - 1) / kGradThreads, NG = 2 * MF * kGradH * kTileW / kGradThreads;
+    bf16x8 vx[NX], vg[NG];
+    // the input that holds this workgroup's two groups: each thread's group
+    // may lie in the first or in the second input
+    auto fetch_x = [&](auto mode, int k, int n, int y0, int x0) {
+        const int q = threadIdx.x + kGradThreads * k;
+        const int cg = q / kHalo, px = q - cg * kHalo;
+        const int sy = px / kHaloW, sx = px - sy * kHaloW;
+        const int ci = ci0 + 8 * cg;
+        const bool ok = q < 2 * kHalo && ci < cin;
+        const int y = y0 + sy - 1, x = x0 + sx - 1;
+        if (ci0 + 8 < A.in1.c || !A.in2.c) {
+            vx[k] = load_at<decltype(mode)::value>(image_of(A.in1, n, A.h, A.w_), ci, y, x,
+                                                   ok && ci < A.in1.c);
+        } else if (ci0 >= A.in1.c) {
+            vx[k] = load_at<kMode0>(image_of(A.in2, n, A.h, A.w_), ci - A.in1.c, y, x, ok);
+        } else {  // one group of each
+            const bf16x8 a = load_at<decltype(mode)::value>(image_of(A.in1, n, A.h, A.w_), ci, y, x,
+                                                            ok && cg == 0);
+            const bf16x8 b = load_at<kMode0>(image_of(A.in2, n, A.h, A.w_), 0, y, x, ok && cg == 1);
+            vx[k] = cg == 0 ? a : b;
+        }
+    };
+    auto fetch = [&](int tile) {
         const int n = tile / (W.tiles_x * W.tiles_y), r = tile - n * W.tiles_x * W.tiles_y;
         const int ty = r / W.tiles_x, y0 = ty * kGradH, x0 = (r - ty * W.tiles_x) * kTileW;
-        __syncthreads();
-        for (int q = threadIdx.x; q < 2 * (kGradH + 2) * kHaloW; q += 256) {
-            const int cg = q / ((kGradH + 2) * kHaloW), px = q - cg * (kGradH + 2) * kHaloW;
-            const int sy = px / kHaloW, sx = px - sy * kHaloW;
-            const int y = y0 + sy - 1, x = x0 + sx - 1, ci = ci0 + 8 * cg;
-            bf16x8 v = zero8();
-            if (ci < cin && y >= 0 && y < A.h && x >= 0 && x < A.w_)
-                v = ci < A.in1.c ? load_in(A.in1, ci, n, y, x, A.h, A.w_)
-                                 : load_in(A.in2, ci - A.in1.c, n, y, x, A.h, A.w_);
 #pragma unroll
-            for (int kx = 0; kx < 3; ++kx) {
-                const int p = sx - kx;
-                if (p < 0 || p >= kTileW) continue;
-                __bf16 *d = xt + (kx * 16 + 8 * cg) * kGradX + sy * kGradRow + p;
+        for (int k = 0; k < NX; ++k) fetch_x(std::integral_constant<int, MODE>{}, k, n, y0, x0);
+        const Image G = image_of(In{W.g, A.cout, kMode0}, n, A.h, A.w_);
 #pragma unroll
-                for (int i = 0; i < 8; ++i) d[i * kGradX] = v[i];
-            }
-        }
-        for (int q = threadIdx.x; q < 2 * MF * kGradH * kTileW; q += 256) {
+        for (int k = 0; k < NG; ++k) {
+            const int q = threadIdx.x + kGradThreads * k;
             const int cg = q / (kGradH * kTileW), px = q - cg * kGradH * kTileW;
             const int y = y0 + px / kTileW, x = x0 + px % kTileW, co = co0 + 8 * cg;
-            bf16x8 v = zero8();
-            if (y < A.h && x < A.w_ && co < A.cout) {
-                const __bf16 *g = W.g + (((long)n * A.h + y) * A.w_ + x) * A.cout + co;
-                if (W.gvec) {
-                    v = ld8(g);
-                } else {
+            if constexpr (VEC) {
+                vg[k] = load_at<kMode0>(G, co, y, x, co < A.cout);
+            } else {
+                vg[k] = zero8();
+                if (y < A.h && x < A.w_) {
+                    const __bf16 *g = W.g + (((long)n * A.h + y) * A.w_ + x) * A.cout + co;
 #pragma unroll
                     for (int i = 0; i < 8; ++i)
-                        if (co + i < A.cout) v[i] = g[i];
+                        if (co + i < A.cout) vg[k][i] = g[i];
                 }
             }
+        }
+    };
+    fetch(blockIdx.z);  // gridDim.z <= tiles
+    for (int tile = blockIdx.z; tile < W.tiles; tile += gridDim.z) {
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < NX; ++k) {
+            const int q = threadIdx.x + kGradThreads * k;
+            const int cg = q / kHalo, px = q - cg * kHalo;
+            const int sy = px / kHaloW, sx = px - sy * kHaloW;
+            if (q < 2 * kHalo) {
+                __bf16 *d = xt + 8 * cg * kGradX + sy * kGradRow + sx;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) d[i * kGradX] = vx[k][i];
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < NG; ++k) {
+            const int q = threadIdx.x + kGradThreads * k;
+            const int cg = q / (kGradH * kTileW), px = q - cg * kGradH * kTileW;
             __bf16 *d = gt + 8 * cg * kGradG + px;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) d[i * kGradG] = v[i];
+            for (int i = 0; i < 8; ++i) d[i * kGradG] = vg[k][i];
         }
         __syncthreads();
+        if (tile + gridDim.z < W.tiles) fetch(tile + gridDim.z);
         // this wave's rows 2 wave and 2 wave + 1; the lane's eight pixels
         const int row = 2 * wave + (kg >> 1), col = 8 * (kg & 1);
         bf16x8 g[MF];
@@ -388,16 +548,25 @@ __global__ __launch_bounds__(256) void k_conv3x3_wgrad(WgradArgs W)
             }
         }
 #pragma unroll
-        for (int t = 0; t < 9; ++t) {
-            const bf16x8 x = ld8(xt + ((t % 3) * 16 + l16) * kGradX + (row + t / 3) * kGradRow + col);
+        for (int ky = 0; ky < 3; ++ky) {
+            const __bf16 *p = xt + l16 * kGradX + (row + ky) * kGradRow + col;
+            const bf16x8 x0 = ld8(p);
+            const unsigned next = *reinterpret_cast<const unsigned *>(p + 8);
+            const bf16x8 x1 = shift_one(x0, next), x2 = shift_two(x0, next);
 #pragma unroll
-            for (int m = 0; m < MF; ++m)
-                acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(g[m], x, acc[t][m], 0, 0, 0);
+            for (int m = 0; m < MF; ++m) {
+                acc[3 * ky][m] =
+                    __builtin_amdgcn_mfma_f32_16x16x32_bf16(g[m], x0, acc[3 * ky][m], 0, 0, 0);
+                acc[3 * ky + 1][m] =
+                    __builtin_amdgcn_mfma_f32_16x16x32_bf16(g[m], x1, acc[3 * ky + 1][m], 0, 0, 0);
+                acc[3 * ky + 2][m] =
+                    __builtin_amdgcn_mfma_f32_16x16x32_bf16(g[m], x2, acc[3 * ky + 2][m], 0, 0, 0);
+            }
         }
     }
     // the other waves' sums into wave 0's
     f32x4 *const red = reinterpret_cast<f32x4 *>(lds);
-    for (int src = 1; src < 4; ++src) {
+    for (int src = 1; src < kGradWaves; ++src) {
         __syncthreads();
         if (wave == src) {
 #pragma unroll
@@ -426,15 +595,22 @@ __global__ __launch_bounds__(256) void k_conv3x3_wgrad(WgradArgs W)
                         atomicAdd(&W.dw[(long)co * A.kpad + t * cin + ci0 + l16], acc[t][m][i]);
                 }
     }
-    if (bias) {
+    if (W.db && blockIdx.x == 0) {
         // lanes l, l+16, l+32, l+48 hold partial sums of channel co0 + l%16
+        float *const rb = reinterpret_cast<float *>(lds);
+        __syncthreads();
 #pragma unroll
         for (int m = 0; m < MF; ++m) {
             float s = bsum[m];
             s += __shfl_xor(s, 16);
             s += __shfl_xor(s, 32);
-            const int co = co0 + 16 * m + l16;
-            if (lane < 16 && co < A.cout) atomicAdd(&W.db[co], s);
+            if (lane < 16) rb[wave * 16 * MF + 16 * m + lane] = s;
+        }
+        __syncthreads();
+        if (threadIdx.x < 16 * MF && co0 + (int)threadIdx.x < A.cout) {
+            float s = 0.0f;
+            for (int k = 0; k < kGradWaves; ++k) s += rb[k * 16 * MF + threadIdx.x];
+            atomicAdd(&W.db[co0 + threadIdx.x], s);
         }
     }
 }
@@ -614,6 +790,51 @@ namespace {
 unsigned blocks256(long n) { return (unsigned)((n + 255) / 256); }
 int rc_of(hipError_t e) { return e == hipSuccess ? M2D_OK : M2D_ERR_HIP; }
 bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
+
+template <int MF, int MODE>
+void launch_wgrad_mode(const WgradArgs &W, bool vec, dim3 grid, hipStream_t s)
+{
+    if (vec)
+        hipLaunchKernelGGL((k_conv3x3_wgrad<MF, MODE, true>), grid, dim3(kGradThreads), 0, s, W);
+    else
+        hipLaunchKernelGGL((k_conv3x3_wgrad<MF, MODE, false>), grid, dim3(kGradThreads), 0, s, W);
+}
+template <int MF>
+void launch_wgrad(const WgradArgs &W, bool vec, dim3 grid, hipStream_t s)
+{
+    if (W.c.in1.mode == kModePool)
+        launch_wgrad_mode<MF, kModePool>(W, vec, grid, s);
+    else if (W.c.in1.mode == kModeUp)
+        launch_wgrad_mode<MF, kModeUp>(W, vec, grid, s);
+    else
+        launch_wgrad_mode<MF, kMode0>(W, vec, grid, s);
+}
+
+// Rows of a tile with 16, 32, 64 output channels per workgroup (nt = 1, 2,
+// 4): mt for each of the waves along the rows
+constexpr int tile_rows(int nt, int mt) { return nt == 4 ? 2 * mt : 4 * mt; }
+
+template <int NT, int MT, int WP, int WC, int C8, int... More>
+void launch_conv_c8(const ConvArgs &A, dim3 grid, int lds, hipStream_t s)
+{
+    if constexpr (sizeof...(More) > 0)
+        if (A.in1.c + A.in2.c != 8 * C8)
+            return launch_conv_c8<NT, MT, WP, WC, More...>(A, grid, lds, s);
+    hipLaunchKernelGGL((k_conv3x3_tile<NT, MT, WP, WC, C8>), grid, dim3(256), lds, s, A);
+}
+
+// the channel counts of the network's layers and their input gradients, any
+// other with computed places
+template <int MT>
+void launch_conv_tile(const ConvArgs &A, int nt, dim3 grid, int lds, hipStream_t s)
+{
+    if (nt == 4)
+        launch_conv_c8<2, MT, 2, 2, 4, 8, 16, 24, 0>(A, grid, lds, s);
+    else if (nt == 2)
+        launch_conv_c8<2, MT, 4, 1, 2, 4, 8, 12, 0>(A, grid, lds, s);
+    else
+        launch_conv_c8<1, MT, 4, 1, 1, 2, 4, 6, 0>(A, grid, lds, s);
+}
 }  // namespace
 
 // ---------------------------------------------------------------------------
@@ -653,23 +874,26 @@ extern "C" int m2d_unet_conv3x3(const void *in1, int c1, int mode1, const void *
     const int cpad = (cout + 15) / 16 * 16;  // weight rows available: cout rounded to 16
     const hipStream_t s = (hipStream_t)stream;
     // 64 channels per workgroup where the weights have them (the input is
-    // staged once for all of them), else 32, else 16; fewer rows per tile with
-    // 64, whose tensors are the small ones
+    // staged once for all of them), else 32, else 16
     const int nt = cpad % 64 == 0 ? 4 : cpad % 32 == 0 ? 2 : 1;
-    const int th = nt == 4 ? 4 : 8;
-    const int lds = stage_bytes(th, cin);
-    if (lds <= 64 * 1024) {
-        A.tiles_x = (w_ + kTileW - 1) / kTileW;
+    // Four rows of the tile per wave where its LDS allows and that leaves two
+    // workgroups for every CU (one with 64 channels, whose weights' reads
+    // from L2 are what the taller tile halves), else two
+    const long fill = nt == 4 ? 256 : 512;
+    A.tiles_x = (w_ + kTileW - 1) / kTileW;
+    for (int mt = 4; mt >= 2; mt -= 2) {
+        const int th = tile_rows(nt, mt), lds = stage_bytes(th, cin);
         A.tiles_y = (h + th - 1) / th;
-        A.rc8 = div_recip(cin / 8);
         const long tiles = (long)A.tiles_x * A.tiles_y * n;  // below npix
-        const dim3 grid((unsigned)tiles, (unsigned)(cpad / (16 * nt)));
-        if (nt == 4)
-            hipLaunchKernelGGL((k_conv3x3_tile<2, 2, 2, 2>), grid, dim3(256), lds, s, A);
-        else if (nt == 2)
-            hipLaunchKernelGGL((k_conv3x3_tile<2, 2, 4, 1>), grid, dim3(256), lds, s, A);
+        const dim3 g((unsigned)tiles, (unsigned)(cpad / (16 * nt)));
+        if (lds > 64 * 1024 || (mt == 4 && (long)g.x * g.y < fill)) continue;
+        A.rc8 = div_recip(cin / 8);
+        A.rc1 = div_recip(c1 / 8);
+        A.rc2 = c2 ? div_recip(c2 / 8) : 0;
+        if (mt == 4)
+            launch_conv_tile<4>(A, nt, g, lds, s);
         else
-            hipLaunchKernelGGL((k_conv3x3_tile<1, 2, 4, 1>), grid, dim3(256), lds, s, A);
+            launch_conv_tile<2>(A, nt, g, lds, s);
         return rc_of(hipGetLastError());
     }
     dim3 grid((unsigned)((npix + 63) / 64), (unsigned)(cpad / (16 * nt)));
@@ -702,27 +926,27 @@ extern "C" int m2d_unet_conv3x3_wgrad(const void *in1, int c1, int mode1, const 
     W.g = (const __bf16 *)g;
     W.dw = dw;
     W.db = db;
-    W.gvec = cout % 8 == 0 && aligned16(g);
     W.tiles_x = (w_ + kTileW - 1) / kTileW;
     W.tiles_y = (h + kGradH - 1) / kGradH;
     const long tiles = (long)W.tiles_x * W.tiles_y * n;
     if (tiles > 0x7fffffffL) return M2D_ERR_ARG;
     W.tiles = (int)tiles;
-    // 64 output channels per workgroup where there are as many, and enough
-    // shares of the tiles for about four workgroups per CU: fewer leave CUs
-    // idle, more only add atomics
-    const int mf = cout > 32 ? 4 : cout > 16 ? 2 : 1;
+    // 32 output channels per workgroup where there are as many (64 took 312
+    // registers a lane: one wave per SIMD), and a workgroup of eight waves
+    // for every CU: their atomics meet on the same addresses (2304 of them for
+    // 16 x 16 channels: 61 us with 1024 workgroups, 113 us with 2048) and
+    // each adds a rounding
+    const int mf = cout > 16 ? 2 : 1;
     const int gx = (cin + 15) / 16, gy = (cout + 16 * mf - 1) / (16 * mf);
-    long gz = (1024 + gx * gy - 1) / (gx * gy);
+    long gz = (256 + gx * gy - 1) / (gx * gy);
     gz = gz < tiles ? gz : tiles;
     const dim3 grid((unsigned)gx, (unsigned)gy, (unsigned)gz);
     const hipStream_t s = (hipStream_t)stream;
-    if (mf == 4)
-        hipLaunchKernelGGL(k_conv3x3_wgrad<4>, grid, dim3(256), 0, s, W);
-    else if (mf == 2)
-        hipLaunchKernelGGL(k_conv3x3_wgrad<2>, grid, dim3(256), 0, s, W);
+    const bool vec = cout % 8 == 0 && aligned16(g);
+    if (mf == 2)
+        launch_wgrad<2>(W, vec, grid, s);
     else
-        hipLaunchKernelGGL(k_conv3x3_wgrad<1>, grid, dim3(256), 0, s, W);
+        launch_wgrad<1>(W, vec, grid, s);
     return rc_of(hipGetLastError());
 }
 

@@ -435,3 +435,60 @@ def test_simplec_pairs_match_reference_fixture(gpu, tmp_path):
             assert np.array_equal(u, v), q
         assert list(got.meta[q][:3]) == list(want.meta[q][:3])
         assert got.meta[q][3] == pytest.approx(want.meta[q][3], rel=1e-3)
+
+
+# (n, h, w, c1, mode, c2, cout): tiles cut by the image's edge in both
+# directions, output channels that leave a group of four or of 16, 32, 64
+# open, channel counts of the network's layers and others (their taps' places
+# are computed), and a staged input beyond 64 KB of LDS
+TILE_CASES = [
+    (1, 1, 1, 8, 0, 0, 8), (1, 9, 17, 8, 0, 0, 16), (2, 17, 33, 16, 0, 0, 16),
+    (1, 7, 15, 16, 0, 0, 5), (1, 10, 18, 24, 0, 0, 12), (1, 16, 30, 32, 2, 16, 16),
+    (1, 9, 31, 32, 0, 0, 48), (3, 5, 19, 16, 1, 0, 32), (1, 8, 16, 40, 0, 8, 32),
+    (1, 12, 34, 64, 2, 32, 32), (1, 5, 17, 32, 0, 0, 64), (2, 3, 21, 64, 1, 0, 128),
+    (1, 6, 18, 128, 2, 64, 64), (1, 5, 33, 64, 0, 0, 96), (1, 4, 16, 64, 0, 0, 192),
+    (1, 6, 20, 392, 0, 0, 64), (1, 9, 20, 240, 0, 0, 16)]
+
+
+@pytest.mark.parametrize("case", TILE_CASES)
+def test_conv3x3_tiles_match_torch(gpu, case):
+    """Forward convolution and weight gradient at the edges of their tiles
+    against PyTorch in FP32 (exact products of bf16 values, sums in another
+    order: 1e-4 of the largest value, as above)."""
+    import ctypes as C
+
+    import torch
+
+    from mach2d import unet as U
+    L = U._bind()
+    n, h, w, c1, mode, c2, cout = case
+    g = torch.Generator().manual_seed(11 + sum(case))
+    sh1 = {0: (n, h, w, c1), 1: (n, 2 * h, 2 * w, c1), 2: (n, h // 2, w // 2, c1)}[mode]
+    x1 = _bf(torch.randn(*sh1, generator=g))
+    x2 = _bf(torch.randn(n, h, w, c2, generator=g)) if c2 else None
+    cin = c1 + c2
+    kpad, cpad = (9 * cin + 31) // 32 * 32, (cout + 15) // 16 * 16
+    wf = torch.zeros(cpad, kpad)
+    wf[:cout, :9 * cin] = _bf(torch.randn(cout, 9 * cin, generator=g) * 0.2)
+    b = torch.randn(cout, generator=g)
+    dx1, dx2 = _dev(x1), _dev(x2) if c2 else None
+    got = _conv_gpu(L, dx1, c1, mode, dx2, c2, _dev(wf), _dev(b, torch.float32), cout, kpad,
+                    n, h, w, 1)
+    xe = _effective(x1, mode, x2)
+    wr = wf[:cout, :9 * cin].clone().requires_grad_(True)
+    want = _ref_conv(xe, wr, b, cin, cout, False)
+    scale = want.abs().max().item()
+    assert torch.allclose(got, torch.relu(want).detach(), atol=1e-4 * scale, rtol=0), case
+    G = _bf(torch.randn(n, h, w, cout, generator=g))
+    (want * G).sum().backward()
+    dw, db, dG = torch.zeros(cpad, kpad, device="cuda"), torch.zeros(cout, device="cuda"), _dev(G)
+    assert L.m2d_unet_conv3x3_wgrad(C.c_void_p(dx1.data_ptr()), c1, mode,
+                                    C.c_void_p(dx2.data_ptr()) if c2 else None, c2,
+                                    C.c_void_p(dG.data_ptr()), cout, kpad, n, h, w,
+                                    C.c_void_p(dw.data_ptr()), C.c_void_p(db.data_ptr()),
+                                    None) == 0
+    torch.cuda.synchronize()
+    sw = max(wr.grad.abs().max().item(), 1e-3)
+    assert torch.allclose(dw.cpu()[:cout, :9 * cin], wr.grad, atol=1e-4 * sw, rtol=0), case
+    assert not dw.cpu()[:, 9 * cin:].any() and not dw.cpu()[cout:].any()
+    assert torch.allclose(db.cpu(), G.sum(dim=(0, 1, 2)), atol=1e-4 * G.abs().sum().item() / cout)
