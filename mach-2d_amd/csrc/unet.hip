@@ -441,7 +441,7 @@ struct WgradArgs {
 
 // MODE: the first input's; VEC: cout a multiple of eight, g aligned
 template <int MF, int MODE, bool VEC>
-__global__ __launch_bounds__(kGradThreads) void k_conv3x3_wgrad(WgradArgs W)
+__global__ __launch_bounds__(kGradThreads, 4) void k_conv3x3_wgrad(WgradArgs W)
 {
     constexpr int kStage = 16 * kGradX + 16 * MF * kGradG, kSums = 9 * MF * 64 * 8;
     constexpr int kLds = kStage > kSums ? kStage : kSums;
@@ -886,7 +886,7 @@ extern "C" int m2d_unet_conv3x3(const void *in1, int c1, int mode1, const void *
         A.tiles_y = (h + th - 1) / th;
         const long tiles = (long)A.tiles_x * A.tiles_y * n;  // below npix
         const dim3 g((unsigned)tiles, (unsigned)(cpad / (16 * nt)));
-        if (lds > 64 * 1024 || (mt == 4 && (long)g.x * g.y < fill)) continue;
+        if (lds > (mt == 4 ? 80 : 64) * 1024 || (mt == 4 && (long)g.x * g.y < fill)) continue;
         A.rc8 = div_recip(cin / 8);
         A.rc1 = div_recip(c1 / 8);
         A.rc2 = c2 ? div_recip(c2 / 8) : 0;
@@ -932,13 +932,14 @@ extern "C" int m2d_unet_conv3x3_wgrad(const void *in1, int c1, int mode1, const 
     if (tiles > 0x7fffffffL) return M2D_ERR_ARG;
     W.tiles = (int)tiles;
     // 32 output channels per workgroup where there are as many (64 took 312
-    // registers a lane: one wave per SIMD), and a workgroup of eight waves
-    // for every CU: their atomics meet on the same addresses (2304 of them for
-    // 16 x 16 channels: 61 us with 1024 workgroups, 113 us with 2048) and
-    // each adds a rounding
+    // registers a lane: one wave per SIMD), and two workgroups of eight waves
+    // for every CU, but at most 256 on the same outputs: their atomics meet
+    // there (16 x 16 channels: 29 us with 256, 61 with 1024, 113 with 2048)
+    // and each adds a rounding
     const int mf = cout > 16 ? 2 : 1;
     const int gx = (cin + 15) / 16, gy = (cout + 16 * mf - 1) / (16 * mf);
-    long gz = (256 + gx * gy - 1) / (gx * gy);
+    long gz = (512 + gx * gy - 1) / (gx * gy);
+    gz = gz < 256 ? gz : 256;
     gz = gz < tiles ? gz : tiles;
     const dim3 grid((unsigned)gx, (unsigned)gy, (unsigned)gz);
     const hipStream_t s = (hipStream_t)stream;
