@@ -666,8 +666,28 @@ int m2d_unet_adam(float *w, float *m, float *v, const float *g, long count, floa
  * (taps rotated by 180 degrees, channels transposed) from FP32 w. */
 int m2d_unet_pack_weights(const float *w, int cout, int cin, int kpad, void *wb, void *wr,
                           int kpad_r, int cin_pad, void *stream);
+/* m2d_unet_pack_weights for `count` layers in one launch (per 24 layers). */
+typedef struct m2d_unet_layer {
+    const float *w;
+    void *wb, *wr;  /* wr may be NULL */
+    int cout, cin, kpad, kpad_r, cin_pad;
+} m2d_unet_layer;
+int m2d_unet_pack_weights_many(int count, const m2d_unet_layer *layers, void *stream);
+/* out = bf16 gradient (n, h, w, c) through the ReLU of activation y (bf16):
+ * the sum of g1 and g2 (g2 may be NULL), FP32 gradients of the inputs of the
+ * convolutions y went into (channels c0.. of cs), each carried back through
+ * its mode to y's resolution h x w, zero where y <= 0: m2d_unet_mode_bwd per
+ * input, m2d_unet_to_bf16 and m2d_unet_relu_bwd in one pass.  c % 8 == 0, c0
+ * and cs multiples of 4, pointers 16-byte aligned. */
+int m2d_unet_grad_in(const float *g1, int cs1, int c01, int mode1, const float *g2, int cs2,
+                     int c02, int mode2, const void *y, int c, int n, int h, int w, void *out,
+                     void *stream);
 /* 0.5*sum(mask*(pred - target)^2)*inv_count: per-256-pixel partial sums and
- * the bf16 gradient (gs channels, value in channel 0). */
+ * the bf16 gradient (gs channels, value in channel 0).  _count: 1 / *count, a
+ * device value, for inv_count. */
+int m2d_unet_mse_count(const float *pred, int ps, const float *target, const float *mask,
+                       long npix, const float *count, void *grad, int gs, float *partial,
+                       void *stream);
 int m2d_unet_mse(const float *pred, int ps, const float *target, const float *mask, long npix,
                  float inv_count, void *grad, int gs, float *partial, void *stream);
 /* Network input of nb systems (a: 9-diagonal FP64 per system, b: rhs) on an

@@ -667,6 +667,77 @@ __global__ __launch_bounds__(256) void k_to_bf16(const float *src, __bf16 *dst, 
     if (i < n) dst[i] = (__bf16)src[i];
 }
 
+// Gradient of a layer's pre-activation output (bf16) from the FP32 gradients
+// of the one or two convolution inputs its activation y went into, each
+// carried back through its mode to y's resolution h x w as k_mode_bwd does,
+// added in their order, rounded and cut where y is not positive.  One pass
+// over memory where zeroing, adding, rounding and the ReLU were four; a
+// thread takes eight channels.
+struct GradSrc {
+    const float *g;  // null: none
+    int cs, c0, mode;
+};
+struct GradArgs {
+    GradSrc src[2];
+    const __bf16 *y;
+    __bf16 *out;
+    int c, h, w;
+    long groups;  // pixels * c / 8
+};
+__global__ __launch_bounds__(256) void k_grad_in(GradArgs A)
+{
+    const long q = (long)blockIdx.x * 256 + threadIdx.x;
+    if (q >= A.groups) return;
+    const int c8 = A.c >> 3;
+    const long px = q / c8;
+    const int ch = 8 * (int)(q - px * c8);
+    const long row = px / A.w;
+    const int x = (int)(px - row * A.w);
+    const long n = row / A.h;
+    const int y = (int)(row - n * A.h);
+    float v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = 0.0f;
+    auto add = [&](const float *p, float f) {
+        const f32x4 a = *reinterpret_cast<const f32x4 *>(p), b = *reinterpret_cast<const f32x4 *>(p + 4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            v[i] += f * a[i];
+            v[4 + i] += f * b[i];
+        }
+    };
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const GradSrc &S = A.src[k];
+        if (!S.g) continue;
+        const float *g = S.g + S.c0 + ch;
+        if (S.mode == kModePool) {
+            add(g + ((n * (A.h >> 1) + (y >> 1)) * (A.w >> 1) + (x >> 1)) * S.cs, 0.25f);
+        } else if (S.mode == kModeUp) {
+            const float *p = g + ((n * 2 * A.h + 2 * y) * 2 * A.w + 2 * x) * S.cs;
+            float t[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                t[i] = v[i];
+                v[i] = 0.0f;
+            }
+            add(p, 1.0f);
+            add(p + S.cs, 1.0f);
+            add(p + 2l * A.w * S.cs, 1.0f);
+            add(p + 2l * A.w * S.cs + S.cs, 1.0f);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] = t[i] + v[i];
+        } else {
+            add(g + px * S.cs, 1.0f);
+        }
+    }
+    const bf16x8 act = ld8(A.y + px * A.c + ch);
+    bf16x8 r;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) r[i] = (float)act[i] > 0.0f ? (__bf16)v[i] : (__bf16)0.0f;
+    *reinterpret_cast<bf16x8 *>(A.out + px * A.c + ch) = r;
+}
+
 // Adam on FP32 master weights w[cout_pad][kpad] (and bias), then the bf16
 // copies the kernels read: wb (same layout) and wr, the input-gradient
 // weights [cin_pad][kpad_r] with wr[ci][tap' * cout + co] = w[co][(8 - tap') * cin + ci].
@@ -689,31 +760,39 @@ __global__ __launch_bounds__(256) void k_adam(AdamArgs a)
     a.w[i] -= a.lr * (m / a.c1) / (sqrtf(v / a.c2) + a.eps);
 }
 
-__global__ __launch_bounds__(256) void k_pack_weights(const float *w, int cout, int cin, int kpad,
-                                                      __bf16 *wb, __bf16 *wr, int kpad_r,
-                                                      int cin_pad)
+// one layer per grid row
+constexpr int kPackLayers = 24;
+struct PackArgs {
+    m2d_unet_layer l[kPackLayers];
+};
+__global__ __launch_bounds__(256) void k_pack_weights(PackArgs A)
 {
+    const m2d_unet_layer &P = A.l[blockIdx.y];
     const long i = (long)blockIdx.x * 256 + threadIdx.x;
-    const long nw = (long)cout * kpad;
-    if (i < nw) wb[i] = (__bf16)w[i];
-    if (wr && i < (long)cin_pad * kpad_r) {
-        const int ci = (int)(i / kpad_r), k = (int)(i % kpad_r);
+    const long nw = (long)P.cout * P.kpad;
+    __bf16 *const wb = (__bf16 *)P.wb, *const wr = (__bf16 *)P.wr;
+    if (i < nw) wb[i] = (__bf16)P.w[i];
+    if (wr && i < (long)P.cin_pad * P.kpad_r) {
+        const int ci = (int)(i / P.kpad_r), k = (int)(i % P.kpad_r);
         float v = 0.0f;
-        if (ci < cin && k < 9 * cout) {
-            const int tr = k / cout, co = k - tr * cout;
-            v = w[(long)co * kpad + (8 - tr) * cin + ci];
+        if (ci < P.cin && k < 9 * P.cout) {
+            const int tr = k / P.cout, co = k - tr * P.cout;
+            v = P.w[(long)co * P.kpad + (8 - tr) * P.cin + ci];
         }
         wr[i] = (__bf16)v;
     }
 }
 
-// Loss 0.5 * sum over masked pixels of (pred - target)^2 / count, its
+// Loss 0.5 * sum over masked pixels of (pred - target)^2 / count (1 / count
+// from inv_count, or from the count in device memory), its
 // gradient (bf16, `cs` channels with the value in channel 0) and per-block
 // partial sums of the loss.
 __global__ __launch_bounds__(256) void k_mse(const float *pred, int ps, const float *target,
                                              const float *mask, long npix, float inv_count,
-                                             __bf16 *grad, int gs, float *partial)
+                                             const float *count, __bf16 *grad, int gs,
+                                             float *partial)
 {
+    if (count) inv_count = (float)(1.0 / (double)*count);
     const long i = (long)blockIdx.x * 256 + threadIdx.x;
     float l = 0.0f;
     if (i < npix) {
@@ -992,16 +1071,70 @@ extern "C" int m2d_unet_adam(float *w, float *m, float *v, const float *g, long 
     return rc_of(hipGetLastError());
 }
 
+extern "C" int m2d_unet_pack_weights_many(int count, const m2d_unet_layer *layers, void *stream)
+{
+    if (count < 0 || (count && !layers)) return M2D_ERR_ARG;
+    for (int k = 0; k < count; ++k) {
+        const m2d_unet_layer &l = layers[k];
+        if (!l.w || !l.wb || l.cout <= 0 || l.cin <= 0 || l.kpad < 9 * l.cin ||
+            (l.wr && (l.kpad_r < 9 * l.cout || l.cin_pad < l.cin)))
+            return M2D_ERR_ARG;
+    }
+    for (int k0 = 0; k0 < count; k0 += kPackLayers) {
+        const int m = count - k0 < kPackLayers ? count - k0 : kPackLayers;
+        PackArgs A;
+        long most = 1;
+        for (int k = 0; k < m; ++k) {
+            const m2d_unet_layer &l = A.l[k] = layers[k0 + k];
+            const long nw = (long)l.cout * l.kpad, nr = l.wr ? (long)l.cin_pad * l.kpad_r : 0;
+            most = nw > most ? nw : most;
+            most = nr > most ? nr : most;
+        }
+        hipLaunchKernelGGL(k_pack_weights, dim3(blocks256(most), (unsigned)m), dim3(256), 0,
+                           (hipStream_t)stream, A);
+    }
+    return rc_of(hipGetLastError());
+}
+
 extern "C" int m2d_unet_pack_weights(const float *w, int cout, int cin, int kpad, void *wb,
                                      void *wr, int kpad_r, int cin_pad, void *stream)
 {
-    if (!w || !wb || cout <= 0 || cin <= 0 || kpad < 9 * cin ||
-        (wr && (kpad_r < 9 * cout || cin_pad < cin)))
+    const m2d_unet_layer l = {w, wb, wr, cout, cin, kpad, kpad_r, cin_pad};
+    return m2d_unet_pack_weights_many(1, &l, stream);
+}
+
+extern "C" int m2d_unet_grad_in(const float *g1, int cs1, int c01, int mode1, const float *g2,
+                                int cs2, int c02, int mode2, const void *y, int c, int n, int h,
+                                int w, void *out, void *stream)
+{
+    if (!g1 || !y || !out || c <= 0 || c % 8 || n <= 0 || h <= 0 || w <= 0) return M2D_ERR_ARG;
+    GradArgs A;
+    A.src[0] = GradSrc{g1, cs1, c01, mode1};
+    A.src[1] = GradSrc{g2, cs2, c02, mode2};
+    for (const GradSrc &S : A.src)
+        if (S.g && (S.mode < 0 || S.mode > 2 || S.c0 < 0 || S.c0 % 4 || S.cs % 4 ||
+                    S.c0 + c > S.cs || !aligned16(S.g) ||
+                    (S.mode == kModePool && (h % 2 || w % 2))))
+            return M2D_ERR_ARG;
+    if (!aligned16(y) || !aligned16(out)) return M2D_ERR_ARG;
+    A.y = (const __bf16 *)y;
+    A.out = (__bf16 *)out;
+    A.c = c;
+    A.h = h;
+    A.w = w;
+    A.groups = (long)n * h * w * (c / 8);
+    hipLaunchKernelGGL(k_grad_in, dim3(blocks256(A.groups)), dim3(256), 0, (hipStream_t)stream, A);
+    return rc_of(hipGetLastError());
+}
+
+static int mse(const float *pred, int ps, const float *target, const float *mask, long npix,
+               float inv_count, const float *count, void *grad, int gs, float *partial,
+               void *stream)
+{
+    if (!pred || !target || !mask || !grad || !partial || npix <= 0 || ps < 1 || gs < 1)
         return M2D_ERR_ARG;
-    const long nw = (long)cout * kpad, nr = wr ? (long)cin_pad * kpad_r : 0;
-    const long tot = nw > nr ? nw : nr;
-    hipLaunchKernelGGL(k_pack_weights, dim3(blocks256(tot)), dim3(256), 0, (hipStream_t)stream, w,
-                       cout, cin, kpad, (__bf16 *)wb, (__bf16 *)wr, kpad_r, cin_pad);
+    hipLaunchKernelGGL(k_mse, dim3(blocks256(npix)), dim3(256), 0, (hipStream_t)stream, pred, ps,
+                       target, mask, npix, inv_count, count, (__bf16 *)grad, gs, partial);
     return rc_of(hipGetLastError());
 }
 
@@ -1009,11 +1142,15 @@ extern "C" int m2d_unet_mse(const float *pred, int ps, const float *target, cons
                             long npix, float inv_count, void *grad, int gs, float *partial,
                             void *stream)
 {
-    if (!pred || !target || !mask || !grad || !partial || npix <= 0 || ps < 1 || gs < 1)
-        return M2D_ERR_ARG;
-    hipLaunchKernelGGL(k_mse, dim3(blocks256(npix)), dim3(256), 0, (hipStream_t)stream, pred, ps,
-                       target, mask, npix, inv_count, (__bf16 *)grad, gs, partial);
-    return rc_of(hipGetLastError());
+    return mse(pred, ps, target, mask, npix, inv_count, nullptr, grad, gs, partial, stream);
+}
+
+extern "C" int m2d_unet_mse_count(const float *pred, int ps, const float *target,
+                                  const float *mask, long npix, const float *count, void *grad,
+                                  int gs, float *partial, void *stream)
+{
+    if (!count) return M2D_ERR_ARG;
+    return mse(pred, ps, target, mask, npix, 0.0f, count, grad, gs, partial, stream);
 }
 
 extern "C" int m2d_unet_pack_input(const double *a, const double *b, int nx, int ny, int h, int w,

@@ -74,6 +74,7 @@ EXPORTS = [
     "m2d_unet_to_bf16", "m2d_unet_adam", "m2d_unet_pack_weights", "m2d_unet_mse",
     "m2d_unet_pack_input", "m2d_unet_unpack_output", "m2d_solve_msi9d_noalloc",
     "m2d_tdma2d9_device_many", "m2d_set_tdma_mode",
+    "m2d_unet_pack_weights_many", "m2d_unet_grad_in", "m2d_unet_mse_count",
 ]
 
 _lib = None

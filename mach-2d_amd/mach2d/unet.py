@@ -77,15 +77,24 @@ def _bind():
     L.m2d_unet_to_bf16.argtypes = [vp, vp, lg, vp]
     L.m2d_unet_adam.argtypes = [vp, vp, vp, vp, lg, f, f, f, f, i, vp]
     L.m2d_unet_pack_weights.argtypes = [vp, i, i, i, vp, vp, i, i, vp]
+    L.m2d_unet_pack_weights_many.argtypes = [i, vp, vp]
+    L.m2d_unet_grad_in.argtypes = [vp, i, i, i, vp, i, i, i, vp, i, i, i, i, vp, vp]
     L.m2d_unet_mse.argtypes = [vp, i, vp, vp, lg, f, vp, i, vp, vp]
+    L.m2d_unet_mse_count.argtypes = [vp, i, vp, vp, lg, vp, vp, i, vp, vp]
     L.m2d_unet_pack_input.argtypes = [vp, vp, i, i, i, i, d, vp, i, vp]
     L.m2d_unet_unpack_output.argtypes = [vp, i, i, i, i, d, vp, vp]
     for name in ("m2d_unet_conv3x3", "m2d_unet_conv3x3_wgrad", "m2d_unet_relu_bwd",
                  "m2d_unet_mode_bwd", "m2d_unet_to_bf16", "m2d_unet_adam",
-                 "m2d_unet_pack_weights", "m2d_unet_mse", "m2d_unet_pack_input",
+                 "m2d_unet_pack_weights", "m2d_unet_pack_weights_many", "m2d_unet_grad_in",
+                 "m2d_unet_mse", "m2d_unet_mse_count", "m2d_unet_pack_input",
                  "m2d_unet_unpack_output"):
         getattr(L, name).restype = C.c_int
     return L
+
+
+class PackLayer(C.Structure):
+    _fields_ = ([(k, C.c_void_p) for k in ("w", "wb", "wr")] +
+                [(k, C.c_int) for k in ("cout", "cin", "kpad", "kpad_r", "cin_pad")])
 
 
 class Layer:
@@ -113,32 +122,43 @@ class UNet:
             lay = Layer(name, src, mode, skip, chans[src], chans[skip] if skip else 0, cout, relu)
             chans[name] = cout
             self.layers.append(lay)
+        # the weights and biases of all layers in one buffer (lay.w, lay.b are
+        # views of it), likewise their gradients and Adam moments, so that a
+        # step zeroes and updates them all at once
+        sizes = [k for lay in self.layers for k in (lay.cpad * lay.kpad, _r(lay.cout, 4))]
+        self._flat = {k: torch.zeros(sum(sizes), device=device) for k in ("p", "g", "m", "v")}
+        for k, (wn, bn) in (("p", ("w", "b")), ("g", ("gw", "gb")), ("m", ("mw", "mb")),
+                            ("v", ("vw", "vb"))):
+            parts = iter(torch.split(self._flat[k], sizes))
+            for lay in self.layers:
+                setattr(lay, wn, next(parts).view(lay.cpad, lay.kpad))
+                setattr(lay, bn, next(parts)[:lay.cout])
+        self._views = [(lay, k, getattr(lay, k)) for lay in self.layers
+                       for k in ("w", "b", "gw", "gb", "mw", "mb", "vw", "vb")]
+        for lay in self.layers:
+            lay.wb = torch.zeros(lay.cpad, lay.kpad, dtype=torch.bfloat16, device=device)
+            lay.wr = torch.zeros(lay.cin_pad, lay.kpad_r, dtype=torch.bfloat16, device=device)
         g = torch.Generator().manual_seed(seed)
         for lay in self.layers:       # He initialisation on the real (tap, channel) entries
             w = torch.zeros(lay.cpad, lay.kpad)
             std = (2.0 / (9 * lay.cin)) ** 0.5 if lay.relu else (1.0 / (9 * lay.cin)) ** 0.5
             w[:lay.cout, :9 * lay.cin] = torch.randn(lay.cout, 9 * lay.cin, generator=g) * std
-            lay.w = w.to(device)
-            lay.b = torch.zeros(lay.cout, device=device)
-        self._alloc_train_state()
+            lay.w.copy_(w)
         self.step_count = 0
         self.pack()
 
-    def _alloc_train_state(self):
-        t = self.torch
-        for lay in self.layers:
-            lay.mw, lay.vw = t.zeros_like(lay.w), t.zeros_like(lay.w)
-            lay.mb, lay.vb = t.zeros_like(lay.b), t.zeros_like(lay.b)
-            lay.gw, lay.gb = t.zeros_like(lay.w), t.zeros_like(lay.b)
-            lay.wb = t.zeros(lay.cpad, lay.kpad, dtype=t.bfloat16, device=self.dev)
-            lay.wr = t.zeros(lay.cin_pad, lay.kpad_r, dtype=t.bfloat16, device=self.dev)
+    def _one_buffer(self):
+        """The layers' tensors are still the views of the one buffer (a caller
+        may have put others in their place)."""
+        return all(getattr(lay, k) is v for lay, k, v in self._views)
 
     def pack(self, stream=None):
         """bf16 copies of the weights (forward and input-gradient forms)."""
-        for lay in self.layers:
-            _check(self.L.m2d_unet_pack_weights(_ptr(lay.w), lay.cout, lay.cin, lay.kpad,
-                                                _ptr(lay.wb), _ptr(lay.wr), lay.kpad_r,
-                                                lay.cin_pad, stream), "pack_weights")
+        ls = (PackLayer * len(self.layers))(
+            *[PackLayer(lay.w.data_ptr(), lay.wb.data_ptr(), lay.wr.data_ptr(), lay.cout, lay.cin,
+                        lay.kpad, lay.kpad_r, lay.cin_pad) for lay in self.layers])
+        _check(self.L.m2d_unet_pack_weights_many(len(self.layers), C.addressof(ls), stream),
+               "pack_weights")
 
     # -- inputs --------------------------------------------------------------
     @staticmethod
@@ -190,57 +210,59 @@ class UNet:
         out = self.forward(x, stream, keep=True)
         acts = self._acts
         npix = n * h * w
-        cnt = float(mask.sum().item())
+        cnt = mask.sum(dtype=t.float32)     # stays on the device
         head = self.layers[-1]
         g = t.empty(n, h, w, head.cout, dtype=t.bfloat16, device=self.dev)
         partial = t.empty((npix + 255) // 256, dtype=t.float32, device=self.dev)
-        _check(self.L.m2d_unet_mse(_ptr(out), head.cout, _ptr(target), _ptr(mask), npix,
-                                   1.0 / cnt, _ptr(g), head.cout, _ptr(partial), stream), "mse")
+        _check(self.L.m2d_unet_mse_count(_ptr(out), head.cout, _ptr(target), _ptr(mask), npix,
+                                         _ptr(cnt), _ptr(g), head.cout, _ptr(partial), stream),
+               "mse")
         loss = partial.sum()
-        grads32 = {}   # FP32 gradient accumulators of the activations
-        gpre = {"head": g}
+        if self._one_buffer():
+            self._flat["g"].zero_()
+        else:
+            for lay in self.layers:
+                lay.gw.zero_()
+                lay.gb.zero_()
+        into = {}   # activation: the gradients of the convolution inputs it went into
         for lay in reversed(self.layers):
             lv = LEVEL[lay.name]
             hh, ww = h >> lv, w >> lv
             if lay.name != "head":
-                gb = t.empty_like(acts[lay.name])
-                _check(self.L.m2d_unet_to_bf16(_ptr(grads32[lay.name]), _ptr(gb), gb.numel(),
-                                               stream), "to_bf16")
-                if lay.relu:
-                    _check(self.L.m2d_unet_relu_bwd(_ptr(gb), _ptr(acts[lay.name]), gb.numel(),
-                                                    stream), "relu_bwd")
-                gpre[lay.name] = gb
-            gl = gpre[lay.name]
+                g = t.empty_like(acts[lay.name])
+                srcs = into.pop(lay.name)
+                (g1, cs1, c01, m1), (g2, cs2, c02, m2) = (srcs + [(None, 0, 0, 0)])[:2]
+                _check(self.L.m2d_unet_grad_in(_ptr(g1), cs1, c01, m1, _ptr(g2), cs2, c02, m2,
+                                               _ptr(acts[lay.name]), lay.cout, n, hh, ww, _ptr(g),
+                                               stream), "grad_in")
             src, skip = acts[lay.src], acts[lay.skip] if lay.skip else None
-            lay.gw.zero_()
-            lay.gb.zero_()
             _check(self.L.m2d_unet_conv3x3_wgrad(_ptr(src), lay.c1, lay.mode, _ptr(skip), lay.c2,
-                                                 _ptr(gl), lay.cout, lay.kpad, n, hh, ww,
+                                                 _ptr(g), lay.cout, lay.kpad, n, hh, ww,
                                                  _ptr(lay.gw), _ptr(lay.gb), stream),
                    "wgrad " + lay.name)
             if lay.src == "x":
                 continue
             gi = t.empty(n, hh, ww, lay.cin, dtype=t.float32, device=self.dev)
-            _check(self.L.m2d_unet_conv3x3(_ptr(gl), lay.cout, DIRECT, None, 0, _ptr(lay.wr),
+            _check(self.L.m2d_unet_conv3x3(_ptr(g), lay.cout, DIRECT, None, 0, _ptr(lay.wr),
                                            None, lay.cin, lay.cin, lay.kpad_r, n, hh, ww, 0,
                                            None, _ptr(gi), 0, stream), "dgrad " + lay.name)
-            for name, c0, c, mode in ((lay.src, 0, lay.c1, lay.mode),
-                                      (lay.skip, lay.c1, lay.c2, DIRECT)):
-                if not name:
-                    continue
-                if name not in grads32:
-                    grads32[name] = t.zeros(acts[name].shape, dtype=t.float32, device=self.dev)
-                _check(self.L.m2d_unet_mode_bwd(_ptr(gi), lay.cin, c0, c, mode, n, hh, ww,
-                                                _ptr(grads32[name]), stream), "mode_bwd")
+            for name, c0, mode in ((lay.src, 0, lay.mode), (lay.skip, lay.c1, DIRECT)):
+                if name:
+                    into.setdefault(name, []).append((gi, lay.cin, c0, mode))
         self._acts = None
         return loss
 
     def adam_step(self, lr=1e-3, b1=0.9, b2=0.999, eps=1e-8, stream=None):
         self.step_count += 1
-        for lay in self.layers:
-            for p, m, v, gr in ((lay.w, lay.mw, lay.vw, lay.gw), (lay.b, lay.mb, lay.vb, lay.gb)):
-                _check(self.L.m2d_unet_adam(_ptr(p), _ptr(m), _ptr(v), _ptr(gr), p.numel(), lr,
-                                            b1, b2, eps, self.step_count, stream), "adam")
+        f = self._flat
+        if self._one_buffer():
+            sets = [(f["p"], f["m"], f["v"], f["g"])]
+        else:
+            sets = [x for lay in self.layers for x in ((lay.w, lay.mw, lay.vw, lay.gw),
+                                                       (lay.b, lay.mb, lay.vb, lay.gb))]
+        for p, m, v, gr in sets:
+            _check(self.L.m2d_unet_adam(_ptr(p), _ptr(m), _ptr(v), _ptr(gr), p.numel(), lr,
+                                        b1, b2, eps, self.step_count, stream), "adam")
         self.pack(stream)
 
     # -- guesses ---------------------------------------------------------------

@@ -492,3 +492,37 @@ def test_conv3x3_tiles_match_torch(gpu, case):
     assert torch.allclose(dw.cpu()[:cout, :9 * cin], wr.grad, atol=1e-4 * sw, rtol=0), case
     assert not dw.cpu()[:, 9 * cin:].any() and not dw.cpu()[cout:].any()
     assert torch.allclose(db.cpu(), G.sum(dim=(0, 1, 2)), atol=1e-4 * G.abs().sum().item() / cout)
+
+
+@pytest.mark.parametrize("n,h,w,c,m1,m2", [(1, 2, 2, 8, 1, None), (2, 6, 10, 16, 1, 0), (1, 3, 5, 24, 0, None),
+                                           (1, 5, 3, 8, 2, None), (2, 4, 8, 32, 0, 2), (1, 8, 6, 40, 2, 1)])
+def test_grad_in_is_its_pieces(gpu, n, h, w, c, m1, m2):
+    """m2d_unet_grad_in against mode_bwd per input, to_bf16 and relu_bwd: the
+    same bits, for every mode, one and two inputs, channel offsets."""
+    import ctypes as C
+
+    import torch
+
+    from mach2d import unet as U
+    L = U._bind()
+    gen = torch.Generator().manual_seed(h * w + c)
+    p = lambda t: C.c_void_p(t.data_ptr()) if t is not None else None  # noqa: E731
+    src, ref = [], torch.zeros(n, h, w, c, device="cuda")
+    for k, m in enumerate((m1, m2)):
+        if m is None:
+            src += [None, 0, 0, 0]
+            continue
+        hh, ww = {0: (h, w), 1: (h // 2, w // 2), 2: (2 * h, 2 * w)}[m]
+        cs, c0 = c + 8 * k, 8 * k
+        g = torch.randn(n, hh, ww, cs, generator=gen).to("cuda")
+        src += [g, cs, c0, m]
+        assert L.m2d_unet_mode_bwd(p(g), cs, c0, c, m, n, hh, ww, p(ref), None) == 0
+    y = _dev(torch.relu(torch.randn(n, h, w, c, generator=gen)))
+    want = torch.empty(n, h, w, c, dtype=torch.bfloat16, device="cuda")
+    assert L.m2d_unet_to_bf16(p(ref), p(want), want.numel(), None) == 0
+    assert L.m2d_unet_relu_bwd(p(want), p(y), want.numel(), None) == 0
+    got = torch.empty_like(want)
+    assert L.m2d_unet_grad_in(p(src[0]), *src[1:4], p(src[4]), *src[5:8], p(y), c, n, h, w, p(got),
+                              None) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
