@@ -28,7 +28,7 @@ tdma_258x130 times the device TDMA of the u and v systems with the lines
 solved by the Thomas recurrence and by parallel cyclic reduction.
 
 Prints one JSON line.  gbps = algorithmic bytes of the solve over its time
-(FP64: 8 N (18 + 11 + 24 K); refinement: 4 N (18 + 24 K_inner) +
+(FP64: 8 N (18 + 11 + 24 K); refinement: 4 N (18 + 46 K_inner) +
 8 N (11 (outer + 1) + 3 outer)); roofline = the dominant kernel's
 algorithmic bytes per launch over its average launch duration (HIP events on
 the solver's stream around each launch, in a repeat of the timed steps: the
@@ -60,6 +60,10 @@ BYTES_PER_POINT = {
     "sweeps": 13,    # forward: read r, dl (5), write w; backward: read w, du (4), write z
     "backward": 6,   # staged sweeps only: the backward sweep alone
     "residual": 14,  # one launch: read z, var, a (9), rhs; write var, r
+    # refinement, two launches: A z and its products (read a (9), z, r and 4
+    # kept q; write q), the step (read z, r, c, q, 4 p, 4 q; write p, q, c, r
+    # and the next sweep's input)
+    "residual32": 33,
 }
 
 
@@ -70,7 +74,7 @@ BYTES_PER_POINT = {
 # residual of one launch.
 MEASURED_TRAFFIC = {
     "sweeps": 84.95e6, "residual": 67.13e6, "factor": 111.72e6,
-    "sweeps32": 39.25e6, "residual32": 33.75e6, "factor32": 55.94e6,
+    "sweeps32": 39.25e6, "factor32": 55.94e6,
 }
 
 
@@ -220,7 +224,7 @@ def msi5_run(steps, warmup):
             nbytes = 8 * s.N * (12 + 7 + 18 * st.nit) if nd == 5 else \
                 8 * s.N * (18 + 11 + 24 * st.nit)
         else:
-            nbytes = 4 * s.N * (12 + 18 * st.nit) + 8 * s.N * (7 * (st.outer + 1) + 3 * st.outer)
+            nbytes = 4 * s.N * (12 + 40 * st.nit) + 8 * s.N * (7 * (st.outer + 1) + 3 * st.outer)
         e = {"solves_per_s": round(1.0 / per, 4), "ms_per_solve": round(per * 1e3, 3),
              "nit": st.nit, "outer": st.outer, "gbps": round(nbytes / per / 1e9, 2),
              "correct": bool(all(x.status == 0 and x.rn < x.gammarp for x in sts))}
@@ -577,7 +581,7 @@ def cpu_baseline(s, nit, budget_s=15.0):
 def solve_bytes(mode, N, st):
     if mode == "fp64":
         return 8 * N * (18 + 11 + 24 * st.nit)
-    return 4 * N * (18 + 24 * st.nit) + 8 * N * (11 * (st.outer + 1) + 3 * st.outer)
+    return 4 * N * (18 + 46 * st.nit) + 8 * N * (11 * (st.outer + 1) + 3 * st.outer)
 
 
 def roofline(kt, N, traffic_known=True):
@@ -586,7 +590,7 @@ def roofline(kt, N, traffic_known=True):
     dom = max(kt, key=lambda k: kt[k][0])
     base = dom.replace("32", "")
     size = 4 if dom.endswith("32") else 8
-    per_launch = BYTES_PER_POINT[base] * size * N
+    per_launch = BYTES_PER_POINT.get(dom, BYTES_PER_POINT[base]) * size * N
     avg_ms = kt[dom][0] / kt[dom][1]
     ach = per_launch / (avg_ms * 1e-3) / 1e9
     traffic = MEASURED_TRAFFIC.get(dom) if traffic_known else None

@@ -173,10 +173,11 @@ int m2d_factor(m2d_system *s, const double *d_a);
  * stopping rule of fb2d9: ||r||_2 < gamma*||r0||_2 or nitm iterations.
  * d_hist, if not NULL, receives ||r_k||_2 for k = 1..nit (capacity hist_cap).
  * In FP32_IR mode, gamma and nitm bound the FP64 outer residual; inner FP32
- * sweeps run until their own residual drops by `inner_gamma` (set with
- * m2d_set_inner) or `inner_nitm` iterations (defaults 1e-4 and 25: short
- * inner runs between FP64 residuals converge in about as many iterations as
- * plain FP64 MSI). */
+ * iterations (MSI sweeps, each result taken as the direction of a
+ * residual-minimising step) run until their own residual drops by
+ * `inner_gamma` (set with m2d_set_inner), or to a tenth of what the outer rule
+ * still asks for where that is less of a drop, or for `inner_nitm` iterations (defaults
+ * 1e-4 and 25). */
 int m2d_solve(m2d_system *s, const double *d_a, const double *d_rhs,
               double *d_var, double gamma, int nitm, double *d_hist,
               int hist_cap, m2d_status *st);

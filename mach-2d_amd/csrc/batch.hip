@@ -255,20 +255,121 @@ __global__ __launch_bounds__(kPts) void k_a32_batch(const BatchSys<double> *__re
     for (int k = 0; k < 9; ++k) a32[k * N + p] = (float)a[k * N + p];
 }
 
-// Refinement step: right-hand side -r (FP32) and c = 0 for the correction.
-__global__ __launch_bounds__(kPts) void k_ir_prepare_batch(const BatchSys<double> *__restrict__ s64,
-                                                           const BatchSys<float> *__restrict__ s32,
-                                                           const int2 *__restrict__ map)
+// ---- the accelerated FP32 correction solves (krylov.h) ---------------------
+// kPts * R points per workgroup, R per thread (256 apart).  What bounds them:
+// 16 and 17 vectors streamed; 256 systems of 64s x 32s points, s in [1, 8] (7.9
+// million points): apply 98 us, step 70 us (5.2 and 7.2 TB/s, the last-level
+// cache helping), of 360 per iteration; 112 and 75 us with one point per
+// thread, 97 and 72 with four.
+template <int R>
+__global__ __launch_bounds__(kPts) void k_krylov_start_batch(
+    const BatchSys<double> *__restrict__ s64, const BatchSys<float> *__restrict__ s32,
+    const int2 *__restrict__ map)
 {
     const int2 m = map[blockIdx.x];
     if (m.x < 0) return;
     const BatchSys<double> &o = s64[m.x];
     if (o.st->done) return;
-    const long N = (long)o.sk.nx * o.sk.ny;
-    const long p = (long)m.y * kPts + threadIdx.x;
-    if (p >= N) return;
-    const_cast<float *>(s32[m.x].rrhs)[p] = (float)(-o.r[p]);
-    s32[m.x].rx[p] = 0.f;
+    const BatchSys<float> &d = s32[m.x];
+    const Skew sk = d.sk;
+    const int N = sk.nx * sk.ny;
+    double s[1] = {0.0};
+    for (int t = 0; t < R; ++t) {
+        const BlockPoint q = block_point(m.y * R + t, sk.nx);
+        if (q.p >= N) break;
+        const float v = (float)o.r[q.p];
+        d.r[sk.template of_point_c<16>(q.i, q.j)] = v;
+        d.kry.r[q.p] = v;
+        d.rx[q.p] = 0.f;
+        s[0] += (double)v * (double)v;
+    }
+    block_sums(s);
+    if (threadIdx.x == 0) d.partial[m.y] = s[0];
+}
+
+// q = A z into its slot, and the workgroup's share of the products.
+template <int R>
+__global__ __launch_bounds__(kPts) void k_krylov_apply_batch(
+    const BatchSys<float> *__restrict__ sys, const int2 *__restrict__ map)
+{
+    const int2 m = map[blockIdx.x];
+    if (m.x < 0) return;
+    const BatchSys<float> &d = sys[m.x];
+    if (d.st->done) return;
+    const Skew sk = d.sk;
+    const KrylovVec v = d.kry;
+    const KrylovSlots k(v, d.st->iter);
+    const int N = sk.nx * sk.ny;
+    float *qc = v.q + k.q(0) * v.n;
+    double s[kKrySums] = {};
+    float q[R];
+#pragma unroll
+    for (int t = 0; t < R; ++t) {
+        const BlockPoint w = block_point(m.y * R + t, sk.nx);
+        if (w.p >= N) continue;
+        KrylovKept o;
+        o.load(v, k, w.p);
+        q[t] = krylov_apply<9>(d.ra, d.w, sk, w.i, w.j);
+        o.dots(q[t], v.r[w.p], s);
+    }
+#pragma unroll
+    for (int t = 0; t < R; ++t) {
+        const int e = (m.y * R + t) * kPts + (int)threadIdx.x;
+        if (e < N) qc[e] = q[t];
+    }
+    block_sums(s);
+    if (threadIdx.x == 0)
+        for (int c = 0; c < kKrySums; ++c) d.partial[(long)c * d.np + m.y] = s[c];
+}
+
+// One workgroup per system: beta and alpha from the products.
+__global__ __launch_bounds__(256) void k_krylov_coef_batch(const BatchSys<float> *__restrict__ sys)
+{
+    const BatchSys<float> &d = sys[blockIdx.x];
+    if (d.st->done) return;
+    const KrylovSlots k(d.kry, d.st->iter);
+    double s[kKrySums] = {};
+    for (int b = threadIdx.x; b < d.np; b += 256)
+#pragma unroll
+        for (int c = 0; c < kKrySums; ++c) s[c] += d.partial[(long)c * d.np + b];
+    block_sums(s);
+    if (threadIdx.x == 0) krylov_coef(d.kry, k, s, d.st->rn);
+}
+
+// z', q', the step, the next sweep's input and the workgroup's share of ||r||^2.
+template <int R>
+__global__ __launch_bounds__(kPts) void k_krylov_step_batch(
+    const BatchSys<float> *__restrict__ sys, const int2 *__restrict__ map)
+{
+    const int2 m = map[blockIdx.x];
+    if (m.x < 0) return;
+    const BatchSys<float> &d = sys[m.x];
+    if (d.st->done) return;
+    const Skew sk = d.sk;
+    const KrylovVec v = d.kry;
+    const KrylovSlots k(v, d.st->iter);
+    const KrylovCoef coef = *v.c;
+    const int N = sk.nx * sk.ny;
+    float *in = d.r, *c = d.rx;
+    double s[1] = {0.0};
+    KrylovStep w[R];
+    long f[R];
+#pragma unroll
+    for (int t = 0; t < R; ++t) {
+        const BlockPoint q = block_point(m.y * R + t, sk.nx);
+        if (q.p >= N) continue;
+        f[t] = sk.template of_point_c<16>(q.i, q.j);
+        w[t].load(v, k, q.p, d.w[f[t]], c);
+    }
+#pragma unroll
+    for (int t = 0; t < R; ++t) {
+        const int e = (m.y * R + t) * kPts + (int)threadIdx.x;
+        if (e >= N) continue;
+        const float x = w[t].finish(v, k, coef, e, c, in[f[t]]);
+        s[0] += (double)x * (double)x;
+    }
+    block_sums(s);
+    if (threadIdx.x == 0) d.partial[m.y] = s[0];
 }
 
 // x += c in FP64.
@@ -304,9 +405,11 @@ __global__ __launch_bounds__(kPts) void k_ir_update_batch(const BatchSys<double>
 namespace {
 
 struct Maps {
-    int2 *d = nullptr;  // one allocation: sweep (forward/factor), backward, points, skew
-    int nf = 0, nb = 0, np = 0, ns = 0;
-    int2 *fwd = nullptr, *bwd = nullptr, *pts = nullptr, *skw = nullptr;
+    // one allocation: sweep (forward/factor), backward, points, skew, points
+    // of the correction solves (refinement only)
+    int2 *d = nullptr;
+    int nf = 0, nb = 0, np = 0, ns = 0, nk = 0;
+    int2 *fwd = nullptr, *bwd = nullptr, *pts = nullptr, *skw = nullptr, *kry = nullptr;
 };
 
 // One chunk of MSI iterations captured in a graph.
@@ -343,6 +446,7 @@ struct m2d_batch {
     // iterations (an outer step of a batch costs more than a single system's)
     double inner_gamma = 1e-4;
     int inner_nitm = 50;
+    int kry_r = 1;  // points per thread of the correction solves' kernels (1 or 2)
     bool factored = false;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
 };
@@ -420,44 +524,52 @@ void drop_graph(m2d_batch *b)
     b->graph.iters = 0;
 }
 
+// Point blocks of `per_block` points: XCD x (workgroups g with g mod 8 = x)
+// takes the x-th contiguous eighth of the list, so the rows a block's stencil
+// reaches (the blocks about nx / per_block before and after it) are mostly
+// read on the same XCD and meet in its L2.  Holes of the ragged end are
+// (-1, 0).
+std::vector<int2> point_map(const m2d_batch *b, long per_block)
+{
+    std::vector<int2> nat;
+    for (int q = 0; q < b->n; ++q)
+        for (long k = 0; k < blocks_of(b->N[q], per_block); ++k)
+            nat.push_back(make_int2(q, (int)k));
+    constexpr int kXcd = 8;
+    const size_t per = (nat.size() + kXcd - 1) / kXcd;
+    std::vector<int2> pts(per * kXcd, make_int2(-1, 0));
+    for (size_t k = 0; k < nat.size(); ++k) pts[(k % per) * kXcd + k / per] = nat[k];
+    return pts;
+}
+
 int build_maps(m2d_batch *b, int layout)
 {
     std::vector<int2> fwd, bwd, pts, skw;
     sweep_maps(b, layout % 3, fwd, bwd);
-    std::vector<int2> nat;
-    for (int q = 0; q < b->n; ++q) {
-        for (long k = 0; k < blocks_of(b->N[q], kPts); ++k) nat.push_back(make_int2(q, (int)k));
+    for (int q = 0; q < b->n; ++q)
         for (long k = 0; k < blocks_of(b->sk[q].size(), 256); ++k)
             skw.push_back(make_int2(q, (int)k));
-    }
-    // Point blocks: XCD x (workgroups g with g mod 8 = x) takes the x-th
-    // contiguous eighth of the list, so the rows a block's stencil reaches
-    // (the blocks about nx / 256 before and after it) are mostly read on
-    // the same XCD and meet in its L2.  Holes of the ragged end are (-1, 0).
-    constexpr int kXcd = 8;
-    const size_t per = (nat.size() + kXcd - 1) / kXcd;
-    pts.assign(per * kXcd, make_int2(-1, 0));
-    for (size_t k = 0; k < nat.size(); ++k) pts[(k % per) * kXcd + k / per] = nat[k];
+    pts = point_map(b, kPts);
+    std::vector<int2> kry;
+    if (!b->h32.empty()) kry = point_map(b, (long)kPts * b->kry_r);
     Maps &m = b->maps;
     if (m.d) (void)hipFree(m.d);
     m.d = nullptr;
-    const size_t tot = fwd.size() + bwd.size() + pts.size() + skw.size();
-    HIP_OK(hipMalloc((void **)&m.d, sizeof(int2) * tot));
     std::vector<int2> all;
-    all.reserve(tot);
-    all.insert(all.end(), fwd.begin(), fwd.end());
-    all.insert(all.end(), bwd.begin(), bwd.end());
-    all.insert(all.end(), pts.begin(), pts.end());
-    all.insert(all.end(), skw.begin(), skw.end());
-    HIP_OK(hipMemcpy(m.d, all.data(), sizeof(int2) * tot, hipMemcpyHostToDevice));
+    for (const std::vector<int2> *v : {&fwd, &bwd, &pts, &skw, &kry})
+        all.insert(all.end(), v->begin(), v->end());
+    HIP_OK(hipMalloc((void **)&m.d, sizeof(int2) * all.size()));
+    HIP_OK(hipMemcpy(m.d, all.data(), sizeof(int2) * all.size(), hipMemcpyHostToDevice));
     m.nf = (int)fwd.size();
     m.nb = (int)bwd.size();
     m.np = (int)pts.size();
     m.ns = (int)skw.size();
+    m.nk = (int)kry.size();
     m.fwd = m.d;
     m.bwd = m.fwd + m.nf;
     m.pts = m.bwd + m.nb;
     m.skw = m.pts + m.np;
+    m.kry = m.skw + m.ns;
     b->layout = layout;
     drop_graph(b);
     return M2D_OK;
@@ -499,15 +611,60 @@ void begin_msi(m2d_batch *b, SolveState *st, const SolveState *outer)
 }
 
 template <typename T>
-void enqueue_iteration(m2d_batch *b)
+void enqueue_sweeps(m2d_batch *b)
 {
-    const BatchSys<T> *d = dsys<T>(b);
     const Maps &m = b->maps;
-    launch_forward_batch<T>(d, m.fwd, m.nf, b->stream, b->layout >= 3);
-    launch_backward_batch<T>(d, m.bwd, m.nb, b->stream, b->layout >= 3);
-    hipLaunchKernelGGL(k_update_residual_batch<T>, dim3(m.np), dim3(kPts), 0, b->stream, d,
-                       m.pts);
-    hipLaunchKernelGGL(k_finalize_batch<T>, dim3(b->n), dim3(256), 0, b->stream, d, 0);
+    launch_forward_batch<T>(dsys<T>(b), m.fwd, m.nf, b->stream, b->layout >= 3);
+    launch_backward_batch<T>(dsys<T>(b), m.bwd, m.nb, b->stream, b->layout >= 3);
+}
+
+// One MSI iteration: FP64 plain, FP32 (correction solves) accelerated.
+template <typename T>
+void enqueue_iteration(m2d_batch *b);
+template <>
+void enqueue_iteration<double>(m2d_batch *b)
+{
+    const Maps &m = b->maps;
+    enqueue_sweeps<double>(b);
+    hipLaunchKernelGGL(k_update_residual_batch<double>, dim3(m.np), dim3(kPts), 0, b->stream,
+                       b->d64, m.pts);
+    hipLaunchKernelGGL(k_finalize_batch<double>, dim3(b->n), dim3(256), 0, b->stream, b->d64, 0);
+}
+
+template <int R>
+void enqueue_krylov(m2d_batch *b)
+{
+    const Maps &m = b->maps;
+    hipLaunchKernelGGL(k_krylov_apply_batch<R>, dim3(m.nk), dim3(kPts), 0, b->stream, b->d32,
+                       m.kry);
+    hipLaunchKernelGGL(k_krylov_coef_batch, dim3(b->n), dim3(256), 0, b->stream, b->d32);
+    hipLaunchKernelGGL(k_krylov_step_batch<R>, dim3(m.nk), dim3(kPts), 0, b->stream, b->d32,
+                       m.kry);
+}
+template <>
+void enqueue_iteration<float>(m2d_batch *b)
+{
+    enqueue_sweeps<float>(b);
+    b->kry_r == 2 ? enqueue_krylov<2>(b) : enqueue_krylov<1>(b);
+    hipLaunchKernelGGL(k_finalize_batch<float>, dim3(b->n), dim3(256), 0, b->stream, b->d32, 0);
+}
+
+// The state an MSI run starts from: FP64 the residual of the iterate; FP32
+// the right-hand side -r of the outer FP64 residual and c = 0.
+template <typename T>
+void enqueue_start(m2d_batch *b);
+template <>
+void enqueue_start<double>(m2d_batch *b)
+{
+    hipLaunchKernelGGL(k_residual_batch<double>, dim3(b->maps.np), dim3(kPts), 0, b->stream,
+                       b->d64, b->maps.pts, 1);
+}
+template <>
+void enqueue_start<float>(m2d_batch *b)
+{
+    const Maps &m = b->maps;
+    auto go = b->kry_r == 2 ? k_krylov_start_batch<2> : k_krylov_start_batch<1>;
+    hipLaunchKernelGGL(go, dim3(m.nk), dim3(kPts), 0, b->stream, b->d64, b->d32, m.kry);
 }
 
 // Capture chunk_iters iterations of precision T once; replays stay valid
@@ -550,8 +707,7 @@ int run_msi(m2d_batch *b, SolveState *st, SolveState *host, const SolveState *ou
 {
     begin_msi<T>(b, st, outer);
     const BatchSys<T> *d = dsys<T>(b);
-    hipLaunchKernelGGL(k_residual_batch<T>, dim3(b->maps.np), dim3(kPts), 0, b->stream, d,
-                       b->maps.pts, 1);
+    enqueue_start<T>(b);
     hipLaunchKernelGGL(k_finalize_batch<T>, dim3(b->n), dim3(256), 0, b->stream, d, 1);
     HIP_OK(hipGetLastError());
     int rc = chunk_graph<T>(b);
@@ -563,8 +719,9 @@ int run_msi(m2d_batch *b, SolveState *st, SolveState *host, const SolveState *ou
         if (all_done(b, host)) break;
         if (rep * b->chunk_iters > 2L * kIterCap) return M2D_ERR_ITER_CAP;  // not reached
     }
-    hipLaunchKernelGGL(k_settle_batch<T>, dim3(b->maps.np), dim3(kPts), 0, b->stream, d,
-                       b->maps.pts);
+    if (sizeof(T) == 8)  // the FP64 iterate alternates between two arrays
+        hipLaunchKernelGGL(k_settle_batch<double>, dim3(b->maps.np), dim3(kPts), 0, b->stream,
+                           b->d64, b->maps.pts);
     HIP_OK(hipGetLastError());
     return M2D_OK;
 }
@@ -647,7 +804,7 @@ extern "C" int m2d_batch_create(int count, const int *nx, const int *ny, int pre
     b->precision = precision;
     const bool fp64 = precision == M2D_FP64;
     const int vb = fp64 ? 8 : 4;
-    long L = 0, NN = 0, NP = 0;
+    long L = 0, NN = 0, NP = 0, NK = 0;
     for (int q = 0; q < count; ++q) {
         b->nx.push_back(nx[q]);
         b->ny.push_back(ny[q]);
@@ -658,6 +815,9 @@ extern "C" int m2d_batch_create(int count, const int *nx, const int *ny, int pre
         NP += blocks_of(b->N[q], kPts);
         b->nwords += boundary_words(nx[q], ny[q]) + scratch_words(ny[q]);
     }
+    // two points per thread once that leaves two workgroups per CU
+    b->kry_r = NN >= 512L * 2 * kPts ? 2 : 1;
+    for (int q = 0; q < count; ++q) NK += blocks_of(b->N[q], (long)kPts * b->kry_r);
     bool ok = true;
     double *part = nullptr;
     ok = ok && balloc(b, &b->st, count) == hipSuccess && balloc(b, &b->st_in, count) == hipSuccess;
@@ -676,12 +836,23 @@ extern "C" int m2d_batch_create(int count, const int *nx, const int *ny, int pre
     }
     // skewed pool of the sweep precision: a 9, dl 6, du 4, r, w
     double *p64 = nullptr, *r64 = nullptr, *alt64 = nullptr;
-    float *p32 = nullptr, *ref32 = nullptr;
+    float *p32 = nullptr, *ref32 = nullptr, *kry = nullptr;
+    double *kpart = nullptr;
+    KrylovCoef *kcoef = nullptr;
+    int win = 0;
     if (fp64) {
         ok = balloc(b, &p64, 21 * L) == hipSuccess && balloc(b, &alt64, NN) == hipSuccess;
     } else {
-        ok = balloc(b, &p32, 21 * L) == hipSuccess && balloc(b, &ref32, 12 * NN) == hipSuccess &&
-             balloc(b, &r64, NN) == hipSuccess && balloc(b, &b->d32, count) == hipSuccess;
+        ok = balloc(b, &p32, 21 * L) == hipSuccess && balloc(b, &ref32, 10 * NN) == hipSuccess &&
+             balloc(b, &r64, NN) == hipSuccess && balloc(b, &b->d32, count) == hipSuccess &&
+             balloc(b, &kpart, kKrySums * NK) == hipSuccess &&
+             balloc(b, &kcoef, count) == hipSuccess;
+        // a shorter window where the full one does not fit the memory
+        for (win = kKryWin; ok; --win) {
+            if (balloc(b, &kry, (2L * win + 2) * NN) == hipSuccess) break;
+            (void)hipGetLastError();
+            ok = win > 0;
+        }
     }
     if (!ok) {
         m2d_batch_destroy(b);
@@ -693,7 +864,7 @@ extern "C" int m2d_batch_create(int count, const int *nx, const int *ny, int pre
         ok = hipMemset(p32, 0, sizeof(float) * 21 * L) == hipSuccess;
     b->h64.resize(count);
     if (!fp64) b->h32.resize(count);
-    long ls = 0, ln = 0, lp = 0, lw = 0;
+    long ls = 0, ln = 0, lp = 0, lw = 0, lk = 0;
     for (int q = 0; q < count && ok; ++q) {
         const Skew &k = b->sk[q];
         const long Lq = k.size(), Nq = b->N[q];
@@ -728,13 +899,19 @@ extern "C" int m2d_batch_create(int count, const int *nx, const int *ny, int pre
             i.bnd = b->words + lw;
             i.scratch = i.bnd + boundary_words(nx[q], ny[q]);
             i.st = b->st_in + q;
-            float *rf = ref32 + 12 * ln;
-            i.ra = rf;             // FP32 A, 9 diagonals
-            i.rrhs = rf + 9 * Nq;  // -r in FP32
-            i.rx = rf + 10 * Nq;   // correction c
-            i.rx2 = rf + 11 * Nq;  // its alternate
-            i.partial = o.partial;
-            i.np = np;
+            float *rf = ref32 + 10 * ln;
+            i.ra = rf;           // FP32 A, 9 diagonals
+            i.rx = rf + 9 * Nq;  // correction c
+            float *rk = kry + (2L * win + 2) * ln;
+            i.kry.n = Nq;
+            i.kry.win = win;
+            i.kry.q = rk;
+            i.kry.r = rk + (win + 1) * Nq;
+            i.kry.p = rk + (win + 2) * Nq;
+            i.kry.c = kcoef + q;
+            i.partial = kpart + kKrySums * lk;
+            i.np = (int)blocks_of(Nq, (long)kPts * b->kry_r);
+            lk += i.np;
             i.gamma = b->inner_gamma;
             i.nitm = b->inner_nitm;
         }
@@ -872,13 +1049,23 @@ static int batch_solve(m2d_batch *b, const double *const *d_a, const double *con
         rc = read_states(b, b->st, b->h_st);
         if (rc) return rc;
         const int kmax = nitm > 0 ? nitm : kIterCap;
+        std::vector<KrylovChoice> choice(b->n);
+        std::vector<double> before(b->n);
+        std::vector<int> its(b->n);
         for (int k = 1; k <= kmax && !all_done(b, b->h_st); ++k) {
-            hipLaunchKernelGGL(k_ir_prepare_batch, dim3(m.np), dim3(kPts), 0, b->stream, b->d64,
-                               b->d32, m.pts);
+            for (int q = 0; q < b->n; ++q) {
+                b->h32[q].kry.plain = choice[q].plain;
+                b->h32[q].gamma = correction_drop(b->inner_gamma, b->h_st[q]);
+                before[q] = b->h_st[q].rn;
+            }
+            rc = upload_desc(b);
+            if (rc) return rc;
             rc = run_msi<float>(b, b->st_in, b->h_in, b->st);
             if (rc) return rc;
-            for (int q = 0; q < b->n; ++q)
-                if (!b->h_st[q].done) inner_total[q] += b->h_in[q].nit;
+            for (int q = 0; q < b->n; ++q) {
+                its[q] = b->h_st[q].done ? 0 : b->h_in[q].nit;
+                inner_total[q] += its[q];
+            }
             hipLaunchKernelGGL(k_ir_update_batch, dim3(m.np), dim3(kPts), 0, b->stream, b->d64,
                                b->d32, m.pts);
             hipLaunchKernelGGL(k_residual_batch<double>, dim3(m.np), dim3(kPts), 0, b->stream,
@@ -892,6 +1079,7 @@ static int batch_solve(m2d_batch *b, const double *const *d_a, const double *con
                 const int s = b->h_in[q].status;
                 if (!b->h_st[q].done && (s == M2D_ERR_NONFINITE || s == M2D_ERR_SYNC_TIMEOUT))
                     return s;
+                choice[q].after(before[q], b->h_st[q].rn, its[q]);
             }
         }
     }
@@ -947,11 +1135,10 @@ extern "C" int m2d_batch_tune(m2d_batch *b, const double *const *d_a, const doub
                                    0, b->stream, b->st, b->n, (const SolveState *)nullptr);
                 hipLaunchKernelGGL(k_residual_batch<double>, dim3(m.np), dim3(kPts), 0,
                                    b->stream, b->d64, m.pts, 0);
-                hipLaunchKernelGGL(k_ir_prepare_batch, dim3(m.np), dim3(kPts), 0, b->stream,
-                                   b->d64, b->d32, m.pts);
                 for (auto &i : b->h32) {
                     i.gamma = 0.0;
                     i.nitm = n_it;
+                    i.kry.plain = 0;
                 }
                 rc = upload_desc(b);
                 if (rc) break;

@@ -16,6 +16,7 @@
 #include <mutex>
 #include <vector>
 
+#include "krylov.h"
 #include "m2d_internal.h"
 #include "msi_stencil.h"
 #include "skew.h"
@@ -54,7 +55,7 @@ struct Work {
             if (p) (void)hipFree(p);
         a = dl = du = r = w = x2 = nullptr;
     }
-    bool alloc(int nx, int ny)
+    bool alloc(int nx, int ny, bool alternate)
     {
         sk = skew_for(nx, ny, (int)sizeof(T));
         const long L = sk.size();
@@ -63,7 +64,8 @@ struct Work {
                   hipMalloc((void **)&dl, 6 * z) == hipSuccess &&
                   hipMalloc((void **)&du, 4 * z) == hipSuccess &&
                   hipMalloc((void **)&r, z) == hipSuccess && hipMalloc((void **)&w, z) == hipSuccess &&
-                  hipMalloc((void **)&x2, sizeof(T) * (size_t)nx * ny) == hipSuccess;
+                  (!alternate ||
+                   hipMalloc((void **)&x2, sizeof(T) * (size_t)nx * ny) == hipSuccess);
         // padding entries are never consumed; start them finite.  dl5 and
         // du4 stay zero for a 5-diagonal system (its factorization writes
         // neither)
@@ -117,18 +119,22 @@ struct m2d_system {
     // register ring's prefetch suffices and the ring's extra LDS pass costs
     bool staged = false;
     int chunk = 8;
-    // inner FP32 MSI: short runs between FP64 residuals; measured on the
-    // 1026x514 system, a refresh every 25 inner iterations needs 650 inner
-    // iterations in all (plain FP64: 646), every 200 needs 734
+    // inner FP32 MSI: short runs between FP64 residuals; on the 1026x514
+    // system a refresh every 25 inner iterations needs 100 of them in all
+    // (plain FP64 MSI: 646)
     double inner_gamma = 1e-4;
     int inner_nitm = 25;
 
     Work<double> w64;
     Work<float> w32;
     // mixed precision: FP32 A (reference layout), outer FP64 residual, FP32
-    // correction and its right-hand side
-    float *a32 = nullptr, *c32 = nullptr, *rr32 = nullptr;
+    // correction; the accelerated iteration's vectors (kry_mem: kry.q,
+    // kry.r, kry.p), scalars and partial sums
+    float *a32 = nullptr, *c32 = nullptr;
     double *r64 = nullptr;
+    float *kry_mem = nullptr;
+    KrylovVec kry{};
+    u64 *kry_partial = nullptr;
 
     u64 *partial = nullptr;  // residual partial sums (tagged words)
     int np = 0;
@@ -260,7 +266,8 @@ extern "C" int m2d_destroy(m2d_system *s)
     if (!s) return M2D_OK;
     s->w64.release();
     s->w32.release();
-    void *bufs[] = {s->a32, s->c32, s->rr32, s->r64, s->partial, s->bnd, s->st, s->st_in};
+    void *bufs[] = {s->a32, s->c32, s->r64, s->partial, s->bnd, s->st, s->st_in,
+                    s->kry_mem, s->kry.c, s->kry_partial};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
     for (hipEvent_t e : s->pool) (void)hipEventDestroy(e);
@@ -307,10 +314,24 @@ extern "C" int m2d_create_stencil(int nx, int ny, int precision, int ndiag, m2d_
               dalloc(&s->bnd, s->nbnd) == hipSuccess &&
               dalloc(&s->st, 1) == hipSuccess && dalloc(&s->st_in, 1) == hipSuccess &&
               dalloc(&s->r64, N) == hipSuccess;
-    if (ok && precision == M2D_FP64) ok = s->w64.alloc(nx, ny);
+    if (ok && precision == M2D_FP64) ok = s->w64.alloc(nx, ny, true);
     if (ok && precision == M2D_FP32_IR) {
-        ok = s->w32.alloc(nx, ny) && dalloc(&s->a32, (long)ndiag * N) == hipSuccess &&
-             dalloc(&s->c32, N) == hipSuccess && dalloc(&s->rr32, N) == hipSuccess;
+        const long nk = krylov_partial_words(nx, ny);
+        ok = s->w32.alloc(nx, ny, false) && dalloc(&s->a32, (long)ndiag * N) == hipSuccess &&
+             dalloc(&s->c32, N) == hipSuccess && dalloc(&s->kry.c, 1) == hipSuccess &&
+             dalloc(&s->kry_partial, nk) == hipSuccess &&
+             hipMemset(s->kry_partial, 0, sizeof(u64) * (size_t)nk) == hipSuccess;
+        // a shorter window where the full one does not fit the memory
+        s->kry.n = N;
+        for (s->kry.win = kKryWin; ok && !s->kry_mem; --s->kry.win) {
+            if (dalloc(&s->kry_mem, (2L * s->kry.win + 2) * N) == hipSuccess) break;
+            (void)hipGetLastError();
+            s->kry_mem = nullptr;
+            ok = s->kry.win > 0;
+        }
+        s->kry.q = s->kry_mem;
+        s->kry.r = s->kry_mem + (s->kry.win + 1) * N;
+        s->kry.p = s->kry_mem + (s->kry.win + 2) * N;
     }
     ok = ok && hipHostMalloc((void **)&s->h_st, sizeof(SolveState), hipHostMallocDefault) ==
                    hipSuccess;
@@ -456,10 +477,9 @@ static int put_factor(m2d_system *s, const double *d_dl, const double *d_du)
     return M2D_OK;
 }
 
-// One MSI iteration (k >= 1) in precision T.
+// The two sweeps of MSI iteration k >= 1 in precision T: z in W.w from W.r.
 template <typename T>
-static void enqueue_iteration(m2d_system *s, Work<T> &W, SolveState *st, const T *a, const T *rhs,
-                              T *x, double *hist, int hist_cap, int k, double gamma, int nitm)
+static void enqueue_sweeps(m2d_system *s, Work<T> &W, SolveState *st, int k)
 {
     const int off = sizeof(T) == 4 ? KT_FP32 : 0;
     if (!s->staged) {  // both sweeps in one launch, timed as the forward sweep
@@ -477,34 +497,37 @@ static void enqueue_iteration(m2d_system *s, Work<T> &W, SolveState *st, const T
                                       s->stream, s->nd == 5);
         });
     }
-    timed(s, KT_RESIDUAL + off, k, [&] {
-        launch_update_residual_norm<T>(a, x, W.x2, W.w, rhs, W.r, W.sk, s->partial, st,
-                                       NormRule{hist, hist_cap, 0, gamma, nitm}, s->stream,
-                                       s->nd);
+}
+
+// One MSI iteration (k >= 1) of the FP64 solve.
+static void enqueue_iteration(m2d_system *s, Work<double> &W, SolveState *st, const double *a,
+                              const double *rhs, double *x, double *hist, int hist_cap, int k,
+                              double gamma, int nitm)
+{
+    enqueue_sweeps(s, W, st, k);
+    timed(s, KT_RESIDUAL, k, [&] {
+        launch_update_residual_norm<double>(a, x, W.x2, W.w, rhs, W.r, W.sk, s->partial, st,
+                                            NormRule{hist, hist_cap, 0, gamma, nitm}, s->stream,
+                                            s->nd);
     });
 }
 
-// fb2d9 on the device, in precision T, from the current x (reference
-// layout); returns after the stopping rule fired (state in s->h_st).
-// Iterations go out in chunks (2, 4, ... up to s->chunk), each followed by
+// Iterations 1, 2, ... (enqueue_k(k) enqueues one) until the device's
+// stopping rule on st fired or nitm of them went out; returns with the state
+// in s->h_st.  Iterations go out in chunks (2, 4, ... up to s->chunk), each followed by
 // a copy of the state; the next chunk is enqueued before the host waits for
 // the previous one's state, so the device never waits for the host, and a
 // chunk enqueued after the stopping rule fired turns into no-ops.
-template <typename T>
-static int run_msi(m2d_system *s, Work<T> &W, SolveState *st, const T *a, const T *rhs, T *x,
-                   double gamma, int nitm, double *hist, int hist_cap)
+template <typename F>
+static int run_chunks(m2d_system *s, SolveState *st, int nitm, F enqueue_k)
 {
-    begin(s, st);
-    launch_residual_norm<T, T, T>(a, x, rhs, W.r, s->nx, s->ny, s->partial, st, &W.sk,
-                                  NormRule{nullptr, 0, 1, gamma, nitm}, s->stream, s->nd);
     const int kmax = nitm > 0 ? nitm : kIterCap;
     const bool piped = s->h_chunk && s->ev_chunk[0] && s->ev_chunk[1];
     int k = 1;
     int chunk = 2;  // grows geometrically up to s->chunk
     auto enqueue_chunk = [&](int slot) -> int {
         const int kend = std::min(kmax, k + chunk - 1);
-        for (; k <= kend; ++k)
-            enqueue_iteration<T>(s, W, st, a, rhs, x, hist, hist_cap, k, gamma, nitm);
+        for (; k <= kend; ++k) enqueue_k(k);
         chunk = std::min(chunk * 2, s->chunk);
         HIP_OK(hipMemcpyAsync(s->h_chunk + slot, st, sizeof(SolveState), hipMemcpyDeviceToHost,
                               s->stream));
@@ -514,8 +537,7 @@ static int run_msi(m2d_system *s, Work<T> &W, SolveState *st, const T *a, const 
     if (!piped) {
         while (k <= kmax) {
             const int kend = std::min(kmax, k + chunk - 1);
-            for (; k <= kend; ++k)
-                enqueue_iteration<T>(s, W, st, a, rhs, x, hist, hist_cap, k, gamma, nitm);
+            for (; k <= kend; ++k) enqueue_k(k);
             HIP_OK(hipGetLastError());
             int rc = read_state(s, st);
             if (rc) return rc;
@@ -540,7 +562,25 @@ static int run_msi(m2d_system *s, Work<T> &W, SolveState *st, const T *a, const 
             if (s->h_st->done) break;
         }
     }
-    launch_settle<T>(x, W.x2, s->N, st, s->stream);
+    HIP_OK(hipGetLastError());
+    return M2D_OK;
+}
+
+// fb2d9 on the device from the current x (reference layout); returns after
+// the stopping rule fired (state in s->h_st).
+static int run_msi(m2d_system *s, Work<double> &W, SolveState *st, const double *a,
+                   const double *rhs, double *x, double gamma, int nitm, double *hist,
+                   int hist_cap)
+{
+    begin(s, st);
+    launch_residual_norm<double, double, double>(a, x, rhs, W.r, s->nx, s->ny, s->partial, st,
+                                                 &W.sk, NormRule{nullptr, 0, 1, gamma, nitm},
+                                                 s->stream, s->nd);
+    const int rc = run_chunks(s, st, nitm, [&](int k) {
+        enqueue_iteration(s, W, st, a, rhs, x, hist, hist_cap, k, gamma, nitm);
+    });
+    if (rc) return rc;
+    launch_settle<double>(x, W.x2, s->N, st, s->stream);
     HIP_OK(hipGetLastError());
     harvest(s, s->h_st->nit);
     return M2D_OK;
@@ -563,7 +603,7 @@ static int solve_fp64(m2d_system *s, const double *d_a, const double *d_rhs, dou
                       double gamma, int nitm, double *d_hist, int hist_cap, m2d_status *out)
 {
     HIP_OK(hipEventRecord(s->ev0, s->stream));
-    int rc = run_msi<double>(s, s->w64, s->st, d_a, d_rhs, d_var, gamma, nitm, d_hist, hist_cap);
+    int rc = run_msi(s, s->w64, s->st, d_a, d_rhs, d_var, gamma, nitm, d_hist, hist_cap);
     if (rc) return rc;
     HIP_OK(hipEventRecord(s->ev1, s->stream));
     HIP_OK(hipEventSynchronize(s->ev1));
@@ -578,18 +618,31 @@ static int solve_fp64(m2d_system *s, const double *d_a, const double *d_rhs, dou
 // refinement.  Outer step: r = A x - rhs in FP64 (the stopping rule of fb2d9
 // on this FP64 residual), then the correction c solves A c = -r
 // approximately by FP32 MSI iterations from c = 0 (A, its factor, residuals
-// and sweeps in FP32) until its own residual drops by inner_gamma, then
-// x += c in FP64.
+// and sweeps in FP32), each taken as a step of krylov.h, until its own
+// residual drops by inner_gamma, or to a tenth of what the outer rule asks
+// for where that takes less (correction_drop), or after inner_nitm of them,
+// then x += c in FP64.
 // ---------------------------------------------------------------------------
-__global__ void k_ir_prepare(const double *__restrict__ r64, float *__restrict__ rr32,
-                             float *__restrict__ c32, long n, const SolveState *st)
+// One correction solve for the FP64 residual in s->r64 (state in s->h_st).
+static int run_correction(m2d_system *s, int plain, double gamma)
 {
-    if (st->done) return;
-    const long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q < n) {
-        rr32[q] = (float)(-r64[q]);
-        c32[q] = 0.f;
-    }
+    Work<float> &W = s->w32;
+    KrylovVec v = s->kry;
+    v.plain = plain;
+    const int nitm = s->inner_nitm;
+    begin(s, s->st_in);
+    launch_krylov_start(s->r64, W.r, s->c32, W.sk, v, s->kry_partial, s->st_in,
+                        NormRule{nullptr, 0, 1, gamma, nitm}, s->stream);
+    const int rc = run_chunks(s, s->st_in, nitm, [&](int k) {
+        enqueue_sweeps(s, W, s->st_in, k);
+        timed(s, KT_RESIDUAL + KT_FP32, k, [&] {
+            launch_krylov_iteration(s->a32, W.w, W.r, s->c32, W.sk, v, s->kry_partial, s->st_in,
+                                    NormRule{nullptr, 0, 0, gamma, nitm}, s->stream, s->nd);
+        });
+    });
+    if (rc) return rc;
+    harvest(s, s->h_st->nit);
+    return M2D_OK;
 }
 
 __global__ void k_ir_update(double *__restrict__ x, const float *__restrict__ c32, long n,
@@ -616,14 +669,13 @@ static int solve_fp32_ir(m2d_system *s, const double *d_a, const double *d_rhs, 
     if (rc) return rc;
     SolveState outer = *s->h_st;
     int total_inner = 0;
+    KrylovChoice choice;
     const int kmax = nitm > 0 ? nitm : kIterCap;
     for (int k = 1; k <= kmax && !outer.done; ++k) {
-        hipLaunchKernelGGL(k_ir_prepare, dim3(nblk), dim3(256), 0, s->stream, s->r64, s->rr32,
-                           s->c32, N, s->st);
-        rc = run_msi<float>(s, s->w32, s->st_in, s->a32, s->rr32, s->c32, s->inner_gamma,
-                            s->inner_nitm, nullptr, 0);
+        rc = run_correction(s, choice.plain, correction_drop(s->inner_gamma, outer));
         if (rc) return rc;
-        total_inner += s->h_st->nit;
+        const int its = s->h_st->nit;
+        total_inner += its;
         const int inner_status = s->h_st->status;
         hipLaunchKernelGGL(k_ir_update, dim3(nblk), dim3(256), 0, s->stream, d_var, s->c32, N,
                            s->st);
@@ -634,6 +686,7 @@ static int solve_fp32_ir(m2d_system *s, const double *d_a, const double *d_rhs, 
         HIP_OK(hipGetLastError());
         rc = read_state(s, s->st);
         if (rc) return rc;
+        choice.after(outer.rn, s->h_st->rn, its);
         outer = *s->h_st;
         if (inner_status == M2D_ERR_NONFINITE || inner_status == M2D_ERR_SYNC_TIMEOUT) {
             outer.status = inner_status;
@@ -980,7 +1033,7 @@ static void enqueue_solve64(m2d_system *s, const double *a, const double *rhs, d
                                                  s->stream, s->nd);
     const int n = enq < 0 ? nitm : std::min(enq, nitm);
     for (int k = 1; k <= n; ++k)
-        enqueue_iteration<double>(s, W, s->st, a, rhs, x, nullptr, 0, k, gamma, nitm);
+        enqueue_iteration(s, W, s->st, a, rhs, x, nullptr, 0, k, gamma, nitm);
     launch_settle<double>(x, W.x2, s->N, s->st, s->stream);
 }
 
@@ -1540,7 +1593,7 @@ extern "C" int m2d_solve_msi9d_noalloc(const int *nx, const int *ny, const int *
         set_last(rc);
         return rc;
     }
-    rc = run_msi<double>(&s, s.w64, s.st, d_a, d_b, d_sol, *tol, *nitm, nullptr, 0);
+    rc = run_msi(&s, s.w64, s.st, d_a, d_b, d_sol, *tol, *nitm, nullptr, 0);
     if (rc) {
         set_last(rc);
         return rc;

@@ -35,6 +35,7 @@ struct SolveState {
 
 struct Link;
 struct Skew;
+struct KrylovVec;
 
 // ---- wavefront kernels and layout (sweep.hip) --------------------------------
 long boundary_words(int nx, int ny);
@@ -118,6 +119,18 @@ void launch_update_residual_norm(const T *a, T *x, T *x2, const T *z, const T *r
                                  const NormRule &rule, hipStream_t s, int nd = 9);
 template <typename T>
 void launch_settle(T *x, const T *x2, long n, const SolveState *st, hipStream_t s);
+// the accelerated FP32 correction solve (krylov.h): r and the sweeps' input
+// in (skewed) = r64, c = 0, ||r|| and the rule; then, after each sweep pair
+// left z, the step along its direction, the next input, ||r|| and the rule.
+// partial: krylov_partial_words words, zero
+// when first used
+long krylov_partial_words(int nx, int ny);
+void launch_krylov_start(const double *r64, float *in, float *c, const Skew &sk,
+                         const KrylovVec &v, unsigned long long *partial, SolveState *st, const NormRule &rule,
+                         hipStream_t s);
+void launch_krylov_iteration(const float *a, const float *z, float *in, float *c, const Skew &sk,
+                             const KrylovVec &v, unsigned long long *partial, SolveState *st,
+                             const NormRule &rule, hipStream_t s, int nd);
 int residual_blocks(int nx, int ny);
 long residual_partial_words(int nx, int ny);
 void launch_check_outside(const double *a, int nx, int ny, SolveState *st, hipStream_t s,

@@ -11,6 +11,7 @@
 #include <assert.h>
 #include <math.h>
 
+#include "krylov.h"
 #include "m2d_internal.h"
 #include "msi_stencil.h"
 #include "skew.h"
@@ -33,6 +34,22 @@ constexpr int kResThreads = 256;
 long residual_partial_words(int nx, int ny)
 {
     return 2L * residual_blocks(nx, ny) + 1;
+}
+
+// Partial sum q of a launch, waiting for its tag (v: its words, loaded
+// before); one that never arrives sets *lost.
+__device__ __forceinline__ double wait_partial(Raw<double> &v, const u64 *pw, unsigned tag,
+                                               int *lost)
+{
+    for (int spin = 0; !raw_ok<double>(v, tag); ++spin) {
+        if (spin == kMaxSpin) {
+            *lost = 1;
+            break;
+        }
+        __builtin_amdgcn_s_sleep(1);
+        raw_load<double>(v, pw);
+    }
+    return raw_value(v);
 }
 
 // One workgroup of 256 threads: ||r||_2 from the np partial sums (each
@@ -60,15 +77,7 @@ __device__ void norm_rule_block(const u64 *__restrict__ pw, int np, unsigned tag
         for (int g = 0; g < G; ++g) {
             const int q = q0 + 256 * g;
             if (q >= np) break;
-            for (int spin = 0; !raw_ok<double>(v[g], tag); ++spin) {
-                if (spin == kMaxSpin) {
-                    lost = 1;
-                    break;
-                }
-                __builtin_amdgcn_s_sleep(1);
-                raw_load<double>(v[g], pw + 2L * q);
-            }
-            acc += raw_value(v[g]);
+            acc += wait_partial(v[g], pw + 2L * q, tag, &lost);
         }
     }
     red[threadIdx.x] = acc;
@@ -196,6 +205,174 @@ __global__ __launch_bounds__(kResThreads) void k_residual(const TA *__restrict__
         __hip_atomic_store(pw + 2L * np, (u64)tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// --------------------------------------------------------------------------
+// The accelerated FP32 correction solve (krylov.h): three kernels around the
+// sweeps.  Points are taken in the reference order, R at a time per thread
+// (256 apart, so loads stay coalesced), 256 R per workgroup; partial sums
+// and the workgroup that finishes last work as in k_residual, kKrySums words
+// per workgroup for the products (region 0 of the buffer) and one for the
+// norm (region 1).
+//
+// What bounds them: the 16 and 17 vectors of N floats each that they stream, from
+// the last-level cache, and on smaller grids the launch and the last
+// workgroup's wait.  Measured (apply + step): 1026x514, 9 diagonals, 17.7 +
+// 10.7 us (the residual kernel of plain MSI: 12; a sweep pair: 158); 515x259,
+// 5 diagonals, 12.6 + 6.6 us of 105 per iteration.
+// --------------------------------------------------------------------------
+template <int R>
+__host__ __device__ inline int krylov_blocks(long n)
+{
+    return (int)((n + 256L * R - 1) / (256L * R));
+}
+
+// Points per thread: 2 once that leaves two workgroups per CU (half the
+// partial sums for the last workgroup to add up), else 1, so that more CUs
+// have work.  apply + step with 1, 2 and 4 points: 1026x514 33.8, 28.5 and
+// 29.6 us; 515x259 19.3, 20.0 and 23.5 us.
+static bool krylov_two(long n) { return n >= 512L * 512; }
+
+long krylov_partial_words(int nx, int ny)
+{
+    return (2L * kKrySums + 2L) * krylov_blocks<1>((long)nx * ny) + 2;
+}
+
+// Workgroup g of the grid takes block (g mod 8) * per + g / 8: each XCD a
+// contiguous run (see k_residual).
+__device__ __forceinline__ int krylov_block(int per)
+{
+    return (int)(blockIdx.x % 8u) * per + (int)(blockIdx.x / 8u);
+}
+
+// r = -(right-hand side) = the FP64 residual, c = 0, ||r|| and the rule.
+template <int R>
+__global__ __launch_bounds__(256) void k_krylov_start(const double *__restrict__ r64,
+                                                      float *__restrict__ in,
+                                                      float *__restrict__ c, Skew sk,
+                                                      KrylovVec w, u64 *pw, SolveState *st,
+                                                      int np, int per, NormRule rule)
+{
+    const int lg = krylov_block(per);
+    const unsigned tag = (unsigned)tag_load(pw + 2L * np) + 1u;
+    if (lg < np) {
+        const long n = (long)sk.nx * sk.ny;
+        double s[1] = {0.0};
+        for (int t = 0; t < R; ++t) {
+            const long e = ((long)lg * R + t) * 256 + threadIdx.x;
+            if (e < n) {
+                const int j = (int)(e / sk.nx), i = (int)(e - (long)j * sk.nx);
+                const float v = (float)r64[e];
+                in[sk.template of_point_c<16>(i, j)] = v;
+                w.r[e] = v;
+                c[e] = 0.f;
+                s[0] += (double)v * (double)v;
+            }
+        }
+        block_sums(s);
+        if (threadIdx.x == 0) put_tagged(pw + 2L * lg, tag, s[0]);
+    }
+    if (blockIdx.x != gridDim.x - 1) return;
+    norm_rule_block(pw, np, tag, st, rule);
+    if (threadIdx.x == 0)
+        __hip_atomic_store(pw + 2L * np, (u64)tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// q = A z into its slot, the products, and beta and alpha.
+template <int ND, int R>
+__global__ __launch_bounds__(256) void k_krylov_apply(const float *__restrict__ ra,
+                                                      const float *__restrict__ z, Skew sk,
+                                                      KrylovVec v, u64 *pw, SolveState *st,
+                                                      int np, int per)
+{
+    if (st->done) return;
+    const int lg = krylov_block(per);
+    const KrylovSlots k(v, st->iter);
+    const unsigned tag = (unsigned)tag_load(pw + 2L * kKrySums * np) + 1u;
+    if (lg < np) {
+        float *qc = v.q + k.q(0) * v.n;
+        double s[kKrySums] = {};
+        float q[R];
+#pragma unroll
+        for (int t = 0; t < R; ++t) {
+            const long e = ((long)lg * R + t) * 256 + threadIdx.x;
+            if (e >= v.n) continue;
+            const int j = (int)(e / sk.nx), i = (int)(e - (long)j * sk.nx);
+            KrylovKept o;
+            o.load(v, k, e);
+            q[t] = krylov_apply<ND>(ra, z, sk, i, j);
+            o.dots(q[t], v.r[e], s);
+        }
+#pragma unroll
+        for (int t = 0; t < R; ++t) {
+            const long e = ((long)lg * R + t) * 256 + threadIdx.x;
+            if (e < v.n) qc[e] = q[t];
+        }
+        block_sums(s);
+        if (threadIdx.x == 0)
+            for (int d = 0; d < kKrySums; ++d)
+                put_tagged(pw + 2L * ((long)lg * kKrySums + d), tag, s[d]);
+    }
+    if (blockIdx.x != gridDim.x - 1) return;
+    __shared__ int lost;
+    if (threadIdx.x == 0) lost = 0;
+    __syncthreads();
+    double s[kKrySums] = {};
+    for (int b = threadIdx.x; b < np; b += 256) {
+        Raw<double> w[kKrySums];
+        const u64 *pb = pw + 2L * kKrySums * b;
+#pragma unroll
+        for (int d = 0; d < kKrySums; ++d) raw_load<double>(w[d], pb + 2 * d);
+#pragma unroll
+        for (int d = 0; d < kKrySums; ++d) s[d] += wait_partial(w[d], pb + 2 * d, tag, &lost);
+    }
+    block_sums(s);
+    if (threadIdx.x != 0) return;
+    if (lost) st->abort = 1;  // the norm's rule ends the solve
+    krylov_coef(v, k, s, st->rn);
+    __hip_atomic_store(pw + 2L * kKrySums * np, (u64)tag, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// z', q', the step, the next sweep's input, ||r|| and the rule.
+template <int R>
+__global__ __launch_bounds__(256) void k_krylov_step(const float *__restrict__ z,
+                                                     float *__restrict__ in,
+                                                     float *__restrict__ c, Skew sk, KrylovVec v,
+                                                     u64 *pw, SolveState *st, int np, int per,
+                                                     NormRule rule)
+{
+    if (st->done) return;
+    const int lg = krylov_block(per);
+    const KrylovSlots k(v, st->iter);
+    const unsigned tag = (unsigned)tag_load(pw + 2L * np) + 1u;
+    if (lg < np) {
+        double s[1] = {0.0};
+        const KrylovCoef coef = *v.c;
+        KrylovStep w[R];
+        long f[R];
+#pragma unroll
+        for (int t = 0; t < R; ++t) {
+            const long e = ((long)lg * R + t) * 256 + threadIdx.x;
+            if (e >= v.n) continue;
+            const int j = (int)(e / sk.nx), i = (int)(e - (long)j * sk.nx);
+            f[t] = sk.template of_point_c<16>(i, j);
+            w[t].load(v, k, e, z[f[t]], c);
+        }
+#pragma unroll
+        for (int t = 0; t < R; ++t) {
+            const long e = ((long)lg * R + t) * 256 + threadIdx.x;
+            if (e >= v.n) continue;
+            const float x = w[t].finish(v, k, coef, e, c, in[f[t]]);
+            s[0] += (double)x * (double)x;
+        }
+        block_sums(s);
+        if (threadIdx.x == 0) put_tagged(pw + 2L * lg, tag, s[0]);
+    }
+    if (blockIdx.x != gridDim.x - 1) return;
+    norm_rule_block(pw, np, tag, st, rule);
+    if (threadIdx.x == 0)
+        __hip_atomic_store(pw + 2L * np, (u64)tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // After an MSI run: an iterate left in x2 (an odd number of iterations)
 // goes back to x.
 template <typename T>
@@ -305,6 +482,49 @@ void launch_update_residual_norm(const T *a, T *x, T *x2, const T *z, const T *r
                            a, x, x2, z, rhs, r, nx, ny, partial, st, sk, nbx, per, rule);
 }
 
+// region 1 of the partial sums: the norms' words
+static u64 *krylov_norm_words(u64 *pw, int np) { return pw + 2L * kKrySums * np + 1; }
+
+void launch_krylov_start(const double *r64, float *in, float *c, const Skew &sk,
+                         const KrylovVec &v, u64 *partial, SolveState *st, const NormRule &rule,
+                         hipStream_t s)
+{
+    const long n = (long)sk.nx * sk.ny;
+    const bool two = krylov_two(n);
+    const int np = two ? krylov_blocks<2>(n) : krylov_blocks<1>(n), per = (np + 7) / 8;
+    assert(sk.S == 16);
+    u64 *pn = krylov_norm_words(partial, np);
+    if (two)
+        hipLaunchKernelGGL(k_krylov_start<2>, dim3(8 * per), dim3(256), 0, s, r64, in, c, sk, v,
+                           pn, st, np, per, rule);
+    else
+        hipLaunchKernelGGL(k_krylov_start<1>, dim3(8 * per), dim3(256), 0, s, r64, in, c, sk, v,
+                           pn, st, np, per, rule);
+}
+
+template <int ND, int R>
+static void krylov_iteration(const float *a, const float *z, float *in, float *c, const Skew &sk,
+                             const KrylovVec &v, u64 *partial, SolveState *st,
+                             const NormRule &rule, hipStream_t s)
+{
+    const int np = krylov_blocks<R>(v.n), per = (np + 7) / 8;
+    hipLaunchKernelGGL((k_krylov_apply<ND, R>), dim3(8 * per), dim3(256), 0, s, a, z, sk, v,
+                       partial, st, np, per);
+    hipLaunchKernelGGL(k_krylov_step<R>, dim3(8 * per), dim3(256), 0, s, z, in, c, sk, v,
+                       krylov_norm_words(partial, np), st, np, per, rule);
+}
+
+void launch_krylov_iteration(const float *a, const float *z, float *in, float *c, const Skew &sk,
+                             const KrylovVec &v, u64 *partial, SolveState *st,
+                             const NormRule &rule, hipStream_t s, int nd)
+{
+    assert(sk.S == 16 && v.n == (long)sk.nx * sk.ny);
+    const bool two = krylov_two(v.n);
+    auto go = nd == 5 ? (two ? krylov_iteration<5, 2> : krylov_iteration<5, 1>)
+                      : (two ? krylov_iteration<9, 2> : krylov_iteration<9, 1>);
+    go(a, z, in, c, sk, v, partial, st, rule, s);
+}
+
 template <typename T>
 void launch_settle(T *x, const T *x2, long n, const SolveState *st, hipStream_t s)
 {
@@ -339,17 +559,8 @@ template void launch_update_residual_norm<double>(const double *, double *, doub
                                                   const double *, const double *, double *,
                                                   const Skew &, u64 *, SolveState *,
                                                   const NormRule &, hipStream_t, int);
-template void launch_update_residual_norm<float>(const float *, float *, float *, const float *,
-                                                 const float *, float *, const Skew &, u64 *,
-                                                 SolveState *, const NormRule &, hipStream_t,
-                                                 int);
 template void launch_settle<double>(double *, const double *, long, const SolveState *,
                                     hipStream_t);
-template void launch_settle<float>(float *, const float *, long, const SolveState *, hipStream_t);
-template void launch_residual_norm<float, float, float>(const float *, const float *,
-                                                        const float *, float *, int, int,
-                                                        u64 *, SolveState *, const Skew *,
-                                                        const NormRule &, hipStream_t, int);
 template void launch_convert<double, float>(const double *, float *, long, hipStream_t);
 template void launch_convert<float, double>(const float *, double *, long, hipStream_t);
 

@@ -1,0 +1,135 @@
+"""The accelerated FP32 correction solves of the FP64 refinement: edges of
+their point blocks (256 and 512 points), of the window of kept directions,
+and the return to plain MSI steps, against the FP64 oracle.  Bound: both
+solutions have a residual of 1e-10 of the first; the oracle's is within 5e-9
+of the exact one on these systems and the refinement's is closer: 1e-8."""
+import numpy as np
+import pytest
+
+from mach2d import problems as P
+
+pytestmark = pytest.mark.gpu
+
+
+def _oracle(orc, s, nd):
+    if nd == 5:
+        dl, du = orc.lu2d5(s.a, s.nx, s.ny)
+        return orc.fb2d5(s.a, dl, du, s.nx, s.ny, np.zeros(s.N), 1e-10, 20000, s.rhs)[:2]
+    dl, du = orc.lu2d9(s.a, s.nx, s.ny)
+    return orc.fb2d9(s.a, dl, du, s.nx, s.ny, np.zeros(s.N), 1e-10, 20000, s.rhs)[:2]
+
+
+def _solve(gpu, s, nd, inner=None, staged=False, rhs=None, nitm=20000):
+    import torch
+    dev = gpu.DeviceMSI(s.nx, s.ny, "fp32_ir", ndiag=nd)
+    if inner:
+        dev.set_inner(*inner)
+    if staged:
+        dev.set_staging(True)
+    a = torch.tensor(s.a, device="cuda")
+    b = torch.tensor(s.rhs if rhs is None else rhs, device="cuda")
+    x = torch.zeros(s.N, dtype=torch.float64, device="cuda")
+    dev.factor(a)
+    st = dev.solve(a, b, x, 1e-10, nitm)
+    x = x.cpu().numpy()
+    dev.close()
+    return st, x
+
+
+def _check(st, x, ox):
+    assert st.status == 0 and st.rn < 1e-10 * st.r0
+    assert np.linalg.norm(x - ox) <= 1e-8 * np.linalg.norm(ox)
+
+
+@pytest.mark.parametrize("nd", [9, 5])
+@pytest.mark.parametrize("nx,ny", [(3, 3), (17, 15), (16, 16), (257, 3), (3, 257), (65, 63),
+                                   (129, 66), (640, 410)])
+def test_point_blocks(gpu, orc, nx, ny, nd):
+    s = (P.pcorr_system if nd == 9 else P.pcorr_system5)(nx, ny, seed=nx + ny, q=1.05)
+    st, x = _solve(gpu, s, nd)
+    _check(st, x, _oracle(orc, s, nd)[0])
+
+
+@pytest.mark.parametrize("inner", [(1e-4, 1), (1e-4, 4), (1e-4, 6), (1e-2, 25), (1e-4, 200)])
+def test_window(gpu, orc, inner):
+    """Correction solves shorter than the window of kept directions, just
+    past it, and long ones; never more sweeps than plain MSI."""
+    s = P.pcorr_system(66, 34, seed=2, rhs="gauss")
+    ox, onit = _oracle(orc, s, 9)
+    st, x = _solve(gpu, s, 9, inner)
+    _check(st, x, ox)
+    assert st.nit <= onit + inner[1]
+
+
+def test_staged_sweeps(gpu, orc):
+    s = P.pcorr_system(130, 130, seed=4, rhs="gauss")
+    st, x = _solve(gpu, s, 9, staged=True)
+    _check(st, x, _oracle(orc, s, 9)[0])
+
+
+def _recirculating(nx, ny):
+    """Upwind convection around the middle of the grid added to a p' system:
+    far from symmetric, slow for the accelerated steps, which hand over to
+    plain ones."""
+    s = P.pcorr_system(nx, ny, seed=3, aspect=1e2, rhs="gauss")
+    a = s.a.reshape(9, ny, nx)
+    i, j = np.meshgrid(np.arange(nx) / nx - 0.5, np.arange(ny) / ny - 0.5)
+    add = np.zeros_like(a)
+    add[3], add[5] = -np.maximum(-j, 0.0), -np.maximum(j, 0.0)
+    add[1], add[7] = -np.maximum(i, 0.0), -np.maximum(-i, 0.0)
+    add[3][:, 0] = add[5][:, -1] = add[1][0] = add[7][-1] = 0.0
+    add[4] = -(add[1] + add[3] + add[5] + add[7])
+    s.a = np.ascontiguousarray((a + add * a[4].mean()).reshape(9, -1))
+    return s
+
+
+def test_far_from_symmetric(gpu, orc):
+    s = _recirculating(130, 66)
+    ox, onit = _oracle(orc, s, 9)
+    st, x = _solve(gpu, s, 9)
+    assert st.status == 0 and st.rn < 1e-10 * st.r0
+    # the oracle's own solution is 1.0e-8 off at this residual: its slowest
+    # components, the worst amplified ones, are what is left of it
+    assert np.linalg.norm(x - ox) <= 5e-8 * np.linalg.norm(ox)
+    print("recirculating: %d iterations, plain %d" % (st.nit, onit))
+    assert st.nit <= onit
+
+
+def test_stalled_window(gpu, orc):
+    """A system on which the residual turns orthogonal to its own direction
+    at 2e-3: the sweep of the direction itself carries on (about 66
+    iterations; 275 where it does not)."""
+    s = P.pcorr_system5(130, 60, seed=3, aspect=1e3, rhs="smooth")
+    st, x = _solve(gpu, s, 5)
+    _check(st, x, _oracle(orc, s, 5)[0])
+    assert st.nit <= 100
+
+
+def test_zero_right_hand_side(gpu):
+    """Nothing to solve: a zero residual leaves the iterate as it is."""
+    s = P.pcorr_system(40, 20, seed=1)
+    st, x = _solve(gpu, s, 9, rhs=np.zeros(s.N), nitm=2)
+    assert st.status == 0 and st.r0 == 0.0 and not x.any()
+
+
+def test_batch_two_points_per_thread(gpu, orc):
+    """A batch large enough for two points per thread, with systems smaller
+    than one workgroup's share, against the FP64 batch."""
+    import torch
+    sizes = [(3, 3), (33, 31), (32, 32), (20, 12)] + [(258, 130)] * 16
+    sys_ = [P.pcorr_system(nx, ny, seed=q, q=1.05, rhs="gauss")
+            for q, (nx, ny) in enumerate(sizes)]
+    sys_[3] = _recirculating(20, 12)
+    a = [torch.tensor(s.a, device="cuda") for s in sys_]
+    b = [torch.tensor(s.rhs, device="cuda") for s in sys_]
+    xs = []
+    for prec in ("fp64", "fp32_ir"):
+        x = [torch.zeros(s.N, dtype=torch.float64, device="cuda") for s in sys_]
+        bt = gpu.BatchMSI(sizes, precision=prec)
+        bt.factor(a)
+        _, st = bt.solve(a, b, x, 1e-12 if prec == "fp64" else 1e-10, 20000)
+        assert all(t.status == 0 for t in st)
+        xs.append(x)
+        bt.close()
+    for u, v in zip(*xs):
+        assert float((u - v).norm()) <= 1e-8 * float(u.norm())
