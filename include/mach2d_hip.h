@@ -219,13 +219,14 @@ int m2d_get_factor(m2d_system *s, double *d_dl, double *d_du);
 /* Launch-shape tuning of the wavefront kernels (autotuner hook):
  * publish_every = columns between progress publications of a band;
  * xcd_stride = 1 (bands on consecutive XCDs) or 8 (bands of one system on
- * one XCD).  Default: 8 for systems of five or more 64-row bands (ny > 256),
- * else 1. */
+ * one XCD).  Default: 1. */
 int m2d_set_tuning(m2d_system *s, int publish_every, int xcd_stride);
 
 /* Sweep operand path: 1 = the LDS-staged sweeps (a second wave loads each
- * chunk's operands into an LDS ring ahead of use), 0 (default) = operands
- * loaded into registers by the computing wave.  Same results either way. */
+ * chunk's operands into an LDS ring ahead of use), 0 (default) = one
+ * launch for both sweeps, operands from an LDS ring where the bands have CUs
+ * of their own, else loaded into registers by the computing wave.  Same
+ * results either way. */
 int m2d_set_staging(m2d_system *s, int staged);
 
 /* ---- 3. Batched API (device pointers) ---------------------------------- */

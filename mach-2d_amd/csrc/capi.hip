@@ -110,13 +110,13 @@ struct m2d_system {
     hipStream_t stream = nullptr;
     // 8: the bands of the system on one XCD (workgroups are dealt to the
     // XCDs round robin, every eighth runs a band); 1: on consecutive XCDs.
-    // The default (m2d_create_stencil) follows measurement: 8 from five
-    // bands up (1026x514 solves 5-6 % faster), 1 below (258x130 time step
-    // 1-2 % faster)
+    // 1 by default: the fed sweeps of 1026x514 (9 bands, FP64, 9 diagonals)
+    // take 324 us a pair on consecutive XCDs; 8 leaves them too few CUs, and
+    // the register sweeps take 362 us on one XCD, which also holds no more
+    // than 64 bands at once
     int xcd_stride = 1;
-    // sweep operands through the LDS ring (m2d_set_staging); off by default:
-    // a single system's working set sits in the last-level cache, where the
-    // register ring's prefetch suffices and the ring's extra LDS pass costs
+    // the two-wave LDS-staged sweeps, one launch each (m2d_set_staging); off
+    // by default: the fed sweeps do the same with a wave for each duty
     bool staged = false;
     int chunk = 8;
     // inner FP32 MSI: short runs between FP64 residuals; on the 1026x514
@@ -303,7 +303,6 @@ extern "C" int m2d_create_stencil(int nx, int ny, int precision, int ndiag, m2d_
     s->nx = nx;
     s->ny = ny;
     s->N = (long)nx * ny;
-    s->xcd_stride = (ny + 63) / 64 >= 5 ? 8 : 1;
     s->precision = precision;
     s->np = residual_blocks(nx, ny);
     s->nbnd = boundary_words(nx, ny) + scratch_words(ny);
@@ -1558,7 +1557,6 @@ extern "C" int m2d_solve_msi9d_noalloc(const int *nx, const int *ny, const int *
     SolveState h_st;
     s.nx = *nx;
     s.ny = *ny;
-    s.xcd_stride = (*ny + 63) / 64 >= 5 ? 8 : 1;  // as m2d_create_stencil
     s.N = (long)*nx * *ny;
     s.nd = 9;
     s.precision = M2D_FP64;

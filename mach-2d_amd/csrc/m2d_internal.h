@@ -54,7 +54,8 @@ void launch_forward_staged(const T *r, const T *dl, T *w, const Skew &sk, Link l
 template <typename T>
 void launch_backward_staged(T *wz, const T *du, const Skew &sk, Link lk, int xcd_stride,
                             hipStream_t s, bool five = false);
-// both sweeps of one iteration in one launch (w from r, then z over w)
+// both sweeps of one iteration in one launch (w from r, then z over w); the
+// fed sweeps where the bands have CUs of their own
 template <typename T>
 void launch_sweeps(const T *r, const T *dl, T *w, const T *du, const Skew &sk, Link lk,
                    int xcd_stride, hipStream_t s, bool five = false);

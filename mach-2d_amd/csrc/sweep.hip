@@ -896,6 +896,315 @@ __device__ __forceinline__ void backward_band_staged(T *__restrict__ wz, const T
 }
 
 // --------------------------------------------------------------------------
+// Fed sweeps: the single system's (k_sweeps).  Four waves, one on each SIMD
+// of the CU: wave 0 computes, wave 1 copies the operands of later chunks into
+// an LDS ring (direct-to-LDS loads), wave 2 stores finished chunks and
+// publishes the edge row, wave 3 polls the neighbour's edge row and keeps its
+// values in LDS.  What bounds them is the computing wave: it issues one
+// instruction every 4.7 cycles, dependent or not, so every instruction that
+// another wave can issue for it counts, and its chunk is shorter than the
+// round trip of a load from the last-level cache or of a boundary word,
+// so neither may be waited for a chunk after its issue.  Loads that share a
+// wave with stores wait for the stores before them (one in-order counter):
+// hence a wave each.  Instructions of the computing wave per chunk (FP64, 5
+// diagonals): forward 240 -> 164, backward 200 -> 118.  A sweep pair, register
+// sweeps and fed: FP64 258x130, 5 diagonals 88.5 -> 73 us, 9 diagonals 97.6 ->
+// 78; 1026x514, 9 diagonals 362 -> 325; FP32 1026x514, 9 diagonals 167 -> 147,
+// 515x259, 5 diagonals 84 -> 74.  Five slots: a chunk's loads have two to
+// three chunks (1 us) to arrive, what the LDS holds for 9 diagonals in FP64.
+//
+// Barriers (c = -1 .. nf-1), passed by all four: barrier c follows chunk c;
+// before it chunk c + 2's operands and chunk c + 1's edge values are in LDS;
+// after it wave 2 stores out-slot c & 1 and wave 1 overwrites chunk c's
+// operand slot.
+// --------------------------------------------------------------------------
+constexpr int kFedSlots = 5;
+constexpr int kEdgeCols = 256;  // columns of the neighbour's row kept in LDS (a power of two)
+template <typename T, int F, int NA>
+struct alignas(16) FedRing {
+    static constexpr int NQ = F * (int)sizeof(T) / 16;  // 16-byte vectors per lane and array
+    uint4 in[kFedSlots][NA * NQ * kWave];               // [slot][(a * NQ + q) * 64 + lane]
+    T out[2][kWave * F];
+    T edge[kEdgeCols];  // column number u (0 = the first one a band reads) at u - 1
+};
+
+// Wave 3.  Column number u = 0 .. nf*F of the neighbour's row is in_col(u),
+// its words at bin + in_col * NW; outside the grid, and without a neighbour,
+// it is zero.  A poll covers 64 columns; whatever prefix of them has arrived
+// goes to LDS.  One poll is in flight and is looked at when the next chunk
+// needs it, so a band that lags far enough behind its neighbour never waits.
+// The wait is bounded; on failure (or another band's) the abort flag is set
+// and zeros follow, so that all waves run to their end.
+template <typename T, int F, typename Ring, typename FIN>
+struct EdgeFeed {
+    Ring &ring;
+    const Link &lk;
+    const u64 *bin;
+    int nx, lane;
+    FIN in_col;
+    bool dead;     // no neighbour, or given up: zeros
+    int have = 0;  // columns in LDS
+    Raw<T> w{};
+    int base = 0;
+
+    __device__ EdgeFeed(Ring &ring_, const Link &lk_, const u64 *bin_, int nx_, bool has_in,
+                        FIN in_col_)
+        : ring(ring_), lk(lk_), bin(bin_), nx(nx_), lane((int)threadIdx.x & (kWave - 1)),
+          in_col(in_col_), dead(!has_in)
+    {
+        if (has_in) poll();
+    }
+    __device__ void poll()
+    {
+        raw_load<T>(w, bin + (long)min(max(in_col(base + lane), 0), nx - 1) * TagWords<T>::n);
+    }
+    __device__ void accept(int limit)
+    {
+        const int u = base + lane, col = in_col(u);
+        const bool need = !dead && col >= 0 && col < nx;
+        const u64 missing = __ballot((need && !raw_ok<T>(w, lk.gen)) || u >= limit);
+        const int n = missing ? __builtin_ctzll(missing) : kWave;
+        if (lane < n) ring.edge[(u - 1) & (kEdgeCols - 1)] = need ? raw_value(w) : T(0);
+        have = max(have, base + n);
+    }
+    // chunk c's columns in LDS (chunk c - 1 is still being read); w is the
+    // poll in flight, of the columns from `base` on
+    __device__ void ensure(int c)
+    {
+        const int limit = (c - 1) * F + kEdgeCols;
+        for (int spin = 0; have < (c + 1) * F + 1; ++spin) {
+            accept(limit);
+            base = have;
+            if (dead) continue;
+            poll();
+            if (spin == kMaxSpin || (spin & 15) == 15) {
+                const bool stop = spin == kMaxSpin ||
+                                  __hip_atomic_load(&lk.st->abort, __ATOMIC_RELAXED,
+                                                    __HIP_MEMORY_SCOPE_AGENT);
+                if (!stop) continue;
+                __hip_atomic_store(&lk.st->abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                dead = true;
+            }
+        }
+    }
+};
+
+template <typename T, int F, typename Ring, typename FIN>
+__device__ __forceinline__ void feed_edges(Ring &ring, const Link &lk, const u64 *bin,
+                                           const Skew &sk, int nf, bool has_in, FIN in_col)
+{
+    EdgeFeed<T, F, Ring, FIN> feed(ring, lk, bin, sk.nx, has_in, in_col);
+    for (int c = -1; c < nf; ++c) {
+        feed.ensure(c + 1);
+        handoff();
+    }
+}
+
+// Wave 2: chunk c from out-slot c & 1 to dst at chunk stored(c), and the edge
+// lane's F values to the neighbouring band: lane q < F takes its element q
+// (F-1-q if reversed) as column col_of(c, q).
+template <typename T, int F, typename Ring, typename FSTORED, typename FCOL>
+__device__ __forceinline__ void store_fed(Ring &ring, T *__restrict__ dst, const Skew &sk,
+                                          int band, int nf, u64 *bout, bool has_out,
+                                          unsigned gen, int edge, bool reversed, FSTORED stored,
+                                          FCOL col_of)
+{
+    const int lane = threadIdx.x & (kWave - 1);
+    const unsigned lofs = (unsigned)lane * F;
+    handoff();
+    for (int c = 0; c < nf; ++c) {
+        handoff();
+        const T *slot = ring.out[c & 1];
+        const int q = lane < F ? lane : 0;
+        const T pv = slot[edge * F + (reversed ? F - 1 - q : q)];
+        T vals[F];
+        vload<T, F>(vals, slot + lofs);
+        const int col = col_of(c, lane);
+        if (has_out && lane < F && col >= 0 && col < sk.nx)  // the neighbour waits for it
+            put_tagged(bout + (long)col * TagWords<T>::n, gen, pv);
+        vstore<T, F>(dst + sk.chunk_base(band, stored(c), 0), lofs, vals);
+    }
+}
+
+// Wave 1: base(a, c) is the wave-uniform start of array a's block of
+// processing chunk c.  Past the last chunk it re-reads that one, which keeps
+// the count of loads in flight fixed.
+template <typename T, int F, int NA, typename Ring, typename FBASE>
+__device__ __forceinline__ void load_fed(Ring &ring, int nf, FBASE base)
+{
+    constexpr int D = kFedSlots, NQ = Ring::NQ, V = 16 / (int)sizeof(T);
+    const unsigned lofs = (unsigned)(threadIdx.x & (kWave - 1)) * F;
+    auto stage = [&](int c) {
+        const int cc = min(c, nf - 1);
+        uint4 *slot = ring.in[c % D];
+#pragma unroll
+        for (int a = 0; a < NA; ++a) {
+            const T *g = base(a, cc);
+#pragma unroll
+            for (int q = 0; q < NQ; ++q)
+                __builtin_amdgcn_global_load_lds((global_cvoid *)(g + (lofs + q * V)),
+                                                 (local_void *)(slot + (a * NQ + q) * kWave), 16,
+                                                 0, 0);
+        }
+    };
+    for (int c = 0; c < D - 1; ++c) stage(c);
+    wait_vmem<(D - 3) * NA * NQ>();  // chunks 0 and 1 complete
+    handoff();
+    for (int c = 0; c < nf; ++c) {
+        stage(c + D - 1);
+        wait_vmem<(D - 3) * NA * NQ>();  // chunk c + 2 complete
+        handoff();
+    }
+    wait_vmem<0>();
+}
+
+template <typename T, int F, int NA, int H, typename Ring>
+__device__ __forceinline__ void read_fed(Halves<T, NA, H> &b, const Ring &ring, int slot, int q0,
+                                         int lane)
+{
+    constexpr int NQ = Ring::NQ, V = 16 / (int)sizeof(T);
+    const uint4 *p = ring.in[slot] + lane;
+    __builtin_amdgcn_sched_barrier(0);  // the reads stay ahead of the half before theirs
+#pragma unroll
+    for (int a = 0; a < NA; ++a)
+#pragma unroll
+        for (int q = 0; q < H / V; ++q) {
+            const uint4 v = p[(a * NQ + q0 + q) * kWave];
+            __builtin_memcpy(&b.v[a][q * V], &v, 16);
+        }
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// forward sweep L w = -r, fed (the arithmetic of forward_band).
+template <typename T, int F, bool Five, typename Ring>
+__device__ __forceinline__ void forward_band_fed(Ring &ring, const T *__restrict__ r,
+                                                 const T *__restrict__ dl, T *__restrict__ w,
+                                                 const Skew &sk, const Link &lk, int band)
+{
+    typedef SweepOps<T, Five> Ops;
+    constexpr int NA = Ops::NF, H = F / 2, NQ = Ring::NQ, NW = TagWords<T>::n;
+    const int lane = threadIdx.x & (kWave - 1), role = (int)threadIdx.x / kWave;
+    const int nx = sk.nx, pad = sk.pad(band);
+    const int nf = sk.nst / F;
+    const long L = sk.size();
+    if (role == 1) {
+        load_fed<T, F, NA>(ring, nf, [=](int a, int c) {
+            return (a == 0 ? r : dl + (long)Ops::fslot(a) * L) + sk.chunk_base(band, c, 0);
+        });
+        return;
+    }
+    if (role == 2) {  // edge = lane 63, columns c*F + q - pad - 126
+        store_fed<T, F>(
+            ring, w, sk, band, nf, lk.bnd + (long)band * nx * NW, band < sk.nb - 1, lk.gen,
+            kWave - 1, false, [](int c) { return c; },
+            [=](int c, int q) { return c * F + q - pad - 2 * (kWave - 1); });
+        return;
+    }
+    if (role == 3) {
+        feed_edges<T, F>(ring, lk, lk.bnd + (long)(band > 0 ? band - 1 : 0) * nx * NW, sk, nf,
+                         band > 0, [=](int u) { return u - pad; });
+        return;
+    }
+    const unsigned lofs = (unsigned)lane * F;
+    Halves<T, NA, H> A, B;
+    T cur = 0, se = 0, sv = 0, sw = 0;
+    auto half = [&](const Halves<T, NA, H> &cb, const T *bv, T *op) {
+        T outv[H];
+#pragma unroll
+        for (int t = 0; t < H; ++t) {
+            const T up = lane_from_below_or(cur, bv[t]);  // lane 0: column i+1 above
+            sw = sv;
+            sv = se;
+            se = up;
+            outv[t] = cur = forward_step<Five>(cb, t, cur, se, sv, sw);
+        }
+        vstore<T, H>(op, outv);
+    };
+    handoff();
+    se = lane == 0 ? ring.edge[kEdgeCols - 1] : T(0);  // column -pad above (used only if pad = 0)
+    read_fed<T, F, NA, H>(A, ring, 0, 0, lane);
+    int slot = 0;
+    for (int c = 0; c < nf; ++c) {
+        T bv[F];  // the neighbour's values, one per step, read first: LDS answers in order
+        vload<T, F>(bv, ring.edge + ((unsigned)(c * F) & (unsigned)(kEdgeCols - 1)));
+        T *op = ring.out[c & 1] + lofs;
+        read_fed<T, F, NA, H>(B, ring, slot, NQ / 2, lane);
+        half(A, bv, op);
+        slot = slot == kFedSlots - 1 ? 0 : slot + 1;
+        read_fed<T, F, NA, H>(A, ring, slot, 0, lane);
+        half(B, bv + H, op + H);
+        handoff();
+    }
+}
+
+// backward sweep U z = w, fed (the arithmetic of backward_band); processing
+// chunk c is stored chunk nf-1-c, visited from its upper half down.
+template <typename T, int F, bool Five, typename Ring>
+__device__ __forceinline__ void backward_band_fed(Ring &ring, T *__restrict__ wz,
+                                                  const T *__restrict__ du, const Skew &sk,
+                                                  const Link &lk, int band)
+{
+    constexpr int NA = SweepOps<T, Five>::NB, H = F / 2, NQ = Ring::NQ, NW = TagWords<T>::n;
+    const int lane = threadIdx.x & (kWave - 1), role = (int)threadIdx.x / kWave;
+    const int nx = sk.nx, pad = sk.pad(band);
+    const int nf = sk.nst / F;
+    const long L = sk.size();
+    const bool has_above = band < sk.nb - 1;
+    if (role == 1) {
+        load_fed<T, F, NA>(ring, nf, [=](int a, int c) {
+            return (a == 0 ? (const T *)wz : du + (long)(a - 1) * L) +
+                   sk.chunk_base(band, nf - 1 - c, 0);
+        });
+        return;
+    }
+    if (role == 2) {  // edge = lane 0, step q = column sc*F + F-1-q - pad of stored chunk sc
+        store_fed<T, F>(
+            ring, wz, sk, band, nf, lk.bnd + (long)(band > 0 ? band - 1 : 0) * nx * NW, band > 0,
+            lk.gen, 0, true, [=](int c) { return nf - 1 - c; },
+            [=](int c, int q) { return (nf - 1 - c) * F + F - 1 - q - pad; });
+        return;
+    }
+    if (role == 3) {
+        feed_edges<T, F>(ring, lk, lk.bnd + (long)(has_above ? band : 0) * nx * NW, sk, nf,
+                         has_above, [=](int u) { return nx - 1 - u; });
+        return;
+    }
+    const unsigned lofs = (unsigned)lane * F;
+    Halves<T, NA, H> A, B;
+    T cur = 0, nw = 0, nv = 0, ne = 0;
+    auto half = [&](const Halves<T, NA, H> &cb, const T *bv, T *op) {
+        T outv[H];
+#pragma unroll
+        for (int t = 0; t < H; ++t) {
+            const int q = H - 1 - t;  // element in the half
+            // lane 63: column i-1 of the band above; the top lane of a
+            // partial band reads a padding row above it (zero couplings)
+            const T dn = lane_from_above_or(cur, bv[t]);
+            ne = nv;
+            nv = nw;
+            nw = dn;
+            outv[q] = cur = backward_step<Five>(cb, q, cur, nw, nv, ne);
+        }
+        vstore<T, H>(op, outv);
+    };
+    handoff();
+    nw = lane == kWave - 1 ? ring.edge[kEdgeCols - 1] : T(0);  // column nx-1 of the row above
+    read_fed<T, F, NA, H>(A, ring, 0, NQ / 2, lane);  // upper half first
+    int slot = 0;
+    for (int c = 0; c < nf; ++c) {
+        T bv[F];  // the neighbour's values, one per step, read first: LDS answers in order
+        vload<T, F>(bv, ring.edge + ((unsigned)(c * F) & (unsigned)(kEdgeCols - 1)));
+        T *op = ring.out[c & 1] + lofs;
+        read_fed<T, F, NA, H>(B, ring, slot, 0, lane);
+        half(A, bv, op + H);
+        slot = slot == kFedSlots - 1 ? 0 : slot + 1;
+        read_fed<T, F, NA, H>(A, ring, slot, NQ / 2, lane);
+        half(B, bv + H, op);
+        handoff();
+    }
+}
+
+// --------------------------------------------------------------------------
 // lu2d9 factorization: A (skewed copy) -> dl, du (skewed).  The edge row
 // carries the four du values of each column.
 //
@@ -1122,11 +1431,15 @@ __device__ __forceinline__ void factor_band(const T *__restrict__ a, T *__restri
 // band s, each under its own sweep's generation; band s+1 writes its
 // backward words only after its forward sweep has read every forward word of
 // the slot, so no forward word lands on a backward one.
-template <typename T, int F, bool Five>
-__global__ __launch_bounds__(2 * kWave) void k_sweeps(const T *__restrict__ r,
-                                                  const T *__restrict__ dl, T *__restrict__ w,
-                                                  const T *__restrict__ du, Skew sk, Link lk0,
-                                                  int xcd_stride)
+//
+// Fed: the fed sweeps (four waves); else the sweeps that load their operands
+// into registers (two waves).
+template <typename T, int F, bool Five, bool Fed>
+__global__ __launch_bounds__((Fed ? 4 : 2) * kWave) void k_sweeps(const T *__restrict__ r,
+                                                               const T *__restrict__ dl,
+                                                               T *__restrict__ w,
+                                                               const T *__restrict__ du, Skew sk,
+                                                               Link lk0, int xcd_stride)
 {
     if (lk0.st->done) return;
     const int blk = blockIdx.x;
@@ -1135,11 +1448,17 @@ __global__ __launch_bounds__(2 * kWave) void k_sweeps(const T *__restrict__ r,
     Link lk = lk0;
     lk.phase = 1;
     lk.gen = launch_gen(lk);
-    forward_band<T, F, Five>(r, dl, w, sk, lk, band);
+    // the forward sweep has the more arrays
+    typedef std::conditional_t<Fed, FedRing<T, F, SweepOps<T, Five>::NF>, int> Ring;
+    __shared__ Ring ring;
+    if constexpr (Fed)
+        forward_band_fed<T, F, Five>(ring, r, dl, w, sk, lk, band);
+    else
+        forward_band<T, F, Five>(r, dl, w, sk, lk, band);
     // the band's w is stored (the storing wave's last chunk included) before
-    // the backward sweep loads it: the two waves share the CU, so waiting for
+    // the backward sweep loads it: the waves share the CU, so waiting for
     // the stores to complete is enough (no cache write-back); a band that
-    // gave up skips the backward sweep, on both waves alike
+    // gave up skips the backward sweep, on all waves alike
     __shared__ int stop;
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     __builtin_amdgcn_s_waitcnt(0);
@@ -1150,7 +1469,10 @@ __global__ __launch_bounds__(2 * kWave) void k_sweeps(const T *__restrict__ r,
     if (stop) return;
     lk.phase = 2;
     lk.gen = launch_gen(lk);
-    backward_band<T, F, Five>(w, du, sk, lk, band);
+    if constexpr (Fed)
+        backward_band_fed<T, F, Five>(ring, w, du, sk, lk, band);
+    else
+        backward_band<T, F, Five>(w, du, sk, lk, band);
 }
 
 template <typename T, int F, bool Five>
@@ -1485,16 +1807,31 @@ void launch_backward_staged(T *wz, const T *du, const Skew &sk, Link lk, int xcd
                            xcd_stride);
 }
 
+// Fed sweeps fill a CU's LDS with one band, and a band holds its CU until its
+// backward sweep ends, which needs every band above it: they are taken where
+// the bands of four such launches (the process's hardware queues) have CUs at
+// once, counting only those the placement uses.  Other systems take the
+// register sweeps, two to four bands to a CU.  Both measured: see the fed
+// sweeps' comment.
+static bool sweeps_fed(int nb, int xcd_stride)
+{
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+        return false;
+    return 4L * nb * xcd_stride <= cus;
+}
+
 template <typename T>
 void launch_sweeps(const T *r, const T *dl, T *w, const T *du, const Skew &sk, Link lk,
                    int xcd_stride, hipStream_t s, bool five)
 {
     constexpr int F = sweep_steps<T>();
-    const dim3 g(sk.nb * xcd_stride), b(2 * kWave);
-    if (five)
-        hipLaunchKernelGGL((k_sweeps<T, F, true>), g, b, 0, s, r, dl, w, du, sk, lk, xcd_stride);
-    else
-        hipLaunchKernelGGL((k_sweeps<T, F, false>), g, b, 0, s, r, dl, w, du, sk, lk, xcd_stride);
+    const bool fed = sweeps_fed(sk.nb, xcd_stride);
+    auto k = five ? (fed ? k_sweeps<T, F, true, true> : k_sweeps<T, F, true, false>)
+                  : (fed ? k_sweeps<T, F, false, true> : k_sweeps<T, F, false, false>);
+    hipLaunchKernelGGL(k, dim3(sk.nb * xcd_stride), dim3((fed ? 4 : 2) * kWave), 0, s, r, dl, w,
+                       du, sk, lk, xcd_stride);
 }
 
 template <typename T>
