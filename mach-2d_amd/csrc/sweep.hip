@@ -1083,7 +1083,7 @@ __device__ __forceinline__ void forward_band_fed(Ring &ring, const T *__restrict
 {
     typedef SweepOps<T, Five> Ops;
     constexpr int NA = Ops::NF, H = F / 2, NQ = Ring::NQ, NW = TagWords<T>::n;
-    const int lane = threadIdx.x & (kWave - 1), role = (int)threadIdx.x / kWave;
+    const int lane = threadIdx.x & (kWave - 1), role = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
     const int nx = sk.nx, pad = sk.pad(band);
     const int nf = sk.nst / F;
     const long L = sk.size();
@@ -1145,7 +1145,7 @@ __device__ __forceinline__ void backward_band_fed(Ring &ring, T *__restrict__ wz
                                                   const Link &lk, int band)
 {
     constexpr int NA = SweepOps<T, Five>::NB, H = F / 2, NQ = Ring::NQ, NW = TagWords<T>::n;
-    const int lane = threadIdx.x & (kWave - 1), role = (int)threadIdx.x / kWave;
+    const int lane = threadIdx.x & (kWave - 1), role = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
     const int nx = sk.nx, pad = sk.pad(band);
     const int nf = sk.nst / F;
     const long L = sk.size();

@@ -26,9 +26,10 @@
 //     an addition back.
 //
 // A chain runs on lane l < R of the first wave of its workgroup, one line
-// per lane.  Its operands stream through an LDS ring: the wave itself
-// issues direct-to-LDS loads (no registers) three chunks ahead and waits on
-// its vector-memory counter for the chunk it needs.  Its results (Q, then x
+// per lane.  Its operands stream through an LDS ring, filled by
+// direct-to-LDS loads (no registers) three chunks ahead: in k_tdma_pre by the
+// wave itself, which waits on its vector-memory counter for the chunk it
+// needs, in k_tdma_line by a wave beside it.  Its results (Q, then x
 // over it; den and P in k_tdma_pre) stay in an LDS tile that every thread
 // of the workgroup stores once the chain has ended, so the chain issues no
 // global store (a store ahead of a load in the in-order vector-memory
@@ -36,11 +37,14 @@
 // a "pass layout" where the lanes' lines are adjacent in memory: element
 // (t, l) of line l at step t sits at t*LP + l (LP = the pass's lines padded
 // to a multiple of 64), written once per call by k_tdma_setup (the
-// coefficients) and per iteration by k_tdma_d (D).  Measured on one
-// MI355X at 258x130 (u and v together): an x-pass chain step (forward and
-// back) costs ~110 ns and a y-pass step ~150 ns, against ~25 ns of
-// dependent FP64 arithmetic (6 cycles per dependent operation): the LDS
-// operand traffic and the ring's load issue take the rest.  Several
+// coefficients) and per iteration by k_tdma_d (D).  What bounds a chain is
+// the instructions its wave issues, one every 4.7 cycles whether dependent or
+// not: 9 FP64 operations, 6 LDS reads and 2 LDS writes per step forward and
+// back, about 40 ns.  The ring's loads and their addresses, another third,
+// are therefore another wave's; the line's first chunk takes the same
+// pipelined path as the others, and the tile goes out without a division
+// per point.  258x130, u and v together: k_tdma_line 27.7 -> 19.6 us (x) and
+// 19.3 -> 13.2 us (y), 5 iterations 333 -> 263 us.  Several
 // systems of one grid size (u and v of a SIMPLEC iteration) run in the
 // same launches.
 #include <math.h>
@@ -366,6 +370,38 @@ __device__ __forceinline__ void tdma_lane_offsets(long (&goff)[kTdmaNI], long LP
     }
 }
 
+// Barrier of the workgroup that orders LDS only: the wait leaves the vector
+// memory counter alone (vmcnt 63, expcnt 7, lgkmcnt 0), so loads in flight
+// stay in flight.
+__device__ __forceinline__ void tdma_handoff()
+{
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    __builtin_amdgcn_s_barrier();
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+}
+
+// The loading wave of a line chain of n chunks of NA arrays: barrier c (c =
+// -1 .. n-1) follows chunk c; before it chunk c + 1 is complete in the ring,
+// and up to two later ones are on their way.  issue(c) loads chunk c into
+// slot c % kTdmaSlots, which chunk c - kTdmaSlots no longer needs; chunks
+// past the line's end re-read its last step, so that every chunk has the same
+// number of loads.
+template <int NA, typename ISSUE>
+__device__ __forceinline__ void tdma_feed(int n, ISSUE issue)
+{
+    constexpr int kAhead = kTdmaSlots - 2;
+    for (int c = 0; c < kTdmaSlots - 1; ++c) issue(c);
+    tdma_wait_vmem<kAhead * NA * kTdmaNI>();
+    tdma_handoff();
+    for (int c = 0; c < n; ++c) {
+        issue(c + kTdmaSlots - 1);
+        tdma_wait_vmem<kAhead * NA * kTdmaNI>();
+        tdma_handoff();
+    }
+    tdma_wait_vmem<0>();
+}
+
 // Block b of a chain launch over one pass -> (system, first line)
 struct TdmaBlock {
     int q, l0, len;
@@ -459,7 +495,8 @@ __global__ __launch_bounds__(256) void k_tdma_pre(TdmaBatch B, int nbx)
 }
 
 // Q chain and back substitution of every line of one pass (each
-// iteration); the result goes to the reference layout: x-pass into the
+// iteration): wave 0 computes, wave 1 loads, the other two wait to help
+// store.  The result goes to the reference layout: x-pass into the
 // scratch's x-pass result, y-pass into the system's x.  The operands a_lo,
 // den, 1/den, D (forward) and P (backward) stream through the LDS ring; Q
 // and then x over it stay in an LDS tile, stored by every thread once the
@@ -475,146 +512,145 @@ __global__ __launch_bounds__(256) void k_tdma_line(TdmaBatch B)
     const int len = k.len;
     double *ring = lds, *tile = lds + kTdmaSlots * NA * kTdmaChunk;
     tdma_ldouble *lring = (tdma_ldouble *)lds;
-    if (threadIdx.x < 64) {
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64);
+    const int nf = (len + K - 1) / K;      // chunks forward
+    const int nb = (len - 1 + K - 1) / K;  // chunks back (steps len-2 .. 0)
+    if (wave == 1) {
+        // chunk c + 1 is in the ring before barrier c (c = -1, 0, ..)
+        const int lane = threadIdx.x - 64;
+        const double *const fa[NA] = {tdma_arr(B, S, XPASS, kTLo), tdma_arr(B, S, XPASS, kTDen),
+                                      tdma_arr(B, S, XPASS, kTRd), tdma_arr(B, S, XPASS, kTD)};
+        long goff[kTdmaNI];
+        tdma_lane_offsets<R>(goff, k.LP, k.l0, lane, 1);
+        tdma_feed<NA>(nf, [&](int c) {
+            tdma_ldouble *slot = lring + (c % kTdmaSlots) * NA * kTdmaChunk;
+            if (c * K + K <= len)
+                tdma_issue_at<NA>(slot, fa, (long)(c * K) * k.LP, goff);
+            else
+                tdma_issue<NA, R>(slot, fa, k.LP, k.l0, lane,
+                                  [&](int s) { return min(c * K + s, len - 1); });
+        });
+        const double *const ba[1] = {tdma_arr(B, S, XPASS, kTP)};
+        tdma_lane_offsets<R>(goff, k.LP, k.l0, lane, -1);
+        tdma_feed<1>(nb, [&](int c) {
+            tdma_ldouble *slot = lring + (c % kTdmaSlots) * kTdmaChunk;
+            if (len - 2 - c * K - (K - 1) >= 0)
+                tdma_issue_at<1>(slot, ba, (long)(len - 2 - c * K) * k.LP, goff);
+            else
+                tdma_issue<1, R>(slot, ba, k.LP, k.l0, lane,
+                                 [&](int s) { return max(len - 2 - c * K - s, 0); });
+        });
+    } else if (wave > 1) {
+        for (int c = 0; c < nf + nb + 2; ++c) tdma_handoff();
+    } else {
         const int lane = threadIdx.x;
         const int wl = lane < R ? lane : R + (lane - R) * RS;  // idle lanes (R >= 32)
         const int rl = lane < R ? lane : 0;
         // forward: Q(0) = D(0) / den(0) (den(0) = a_P), then
-        // Q(t) = (D(t) - a_lo Q(t-1)) / den(t), each quotient exact through 1/den
-        {
-            const double *const arr[NA] = {tdma_arr(B, S, XPASS, kTLo),
-                                           tdma_arr(B, S, XPASS, kTDen),
-                                           tdma_arr(B, S, XPASS, kTRd), tdma_arr(B, S, XPASS, kTD)};
-            const int nch = (len + K - 1) / K;
-            long goff[kTdmaNI];
-            tdma_lane_offsets<R>(goff, k.LP, k.l0, lane, 1);
-            auto issue = [&](int c) {
-                tdma_ldouble *slot = lring + (c % kTdmaSlots) * NA * kTdmaChunk;
-                if (c * K + K <= len)
-                    tdma_issue_at<NA>(slot, arr, (long)(c * K) * k.LP, goff);
-                else
-                    tdma_issue<NA, R>(slot, arr, k.LP, k.l0, lane,
-                                      [&](int s) { return min(c * K + s, len - 1); });
+        // Q(t) = (D(t) - a_lo Q(t-1)) / den(t), each quotient exact through
+        // 1/den; a_lo(0) is taken as 0 (and Q(-1) is 0)
+        double Qm = 0.0;
+        tdma_handoff();
+        for (int c = 0; c < nf; ++c) {
+            const double *sl = ring + (c % kTdmaSlots) * NA * kTdmaChunk;
+            const double *slo = sl, *sden = sl + kTdmaChunk, *srd = sl + 2 * kTdmaChunk,
+                         *sD = sl + 3 * kTdmaChunk;
+            const int t0 = c * K;
+            // G steps at a time: the operands of group g+1 are read from LDS
+            // while group g computes
+            constexpr int G = 4, NG = K / G;
+            double lo[2][G], dn[2][G], rd[2][G], dv[2][G];
+            auto fetch = [&](int b, int s0) {
+#pragma unroll
+                for (int u = 0; u < G; ++u) {
+                    const int o = (s0 + u) * R + rl;
+                    lo[b][u] = slo[o];
+                    dn[b][u] = sden[o];
+                    rd[b][u] = srd[o];
+                    dv[b][u] = sD[o];
+                }
             };
-            for (int c = 0; c < kTdmaSlots - 1; ++c) issue(c);
-            double Qm = 0.0;
-            for (int c = 0; c < nch; ++c) {
-                issue(c + kTdmaSlots - 1);
-                tdma_wait_vmem<(kTdmaSlots - 1) * NA * kTdmaNI>();
-                const double *sl = ring + (c % kTdmaSlots) * NA * kTdmaChunk;
-                const double *slo = sl, *sden = sl + kTdmaChunk, *srd = sl + 2 * kTdmaChunk,
-                             *sD = sl + 3 * kTdmaChunk;
-                const int t0 = c * K;
-                if (c > 0 && t0 + K <= len) {
-                    // full chunk past step 0, G steps at a time: the operands
-                    // of group g+1 are read from LDS while group g computes
-                    constexpr int G = 4, NG = K / G;
-                    double lo[2][G], dn[2][G], rd[2][G], dv[2][G];
-                    auto fetch = [&](int b, int s0) {
+            auto step = [&](int b, int g, int u) {
+                Qm = div_by_rcp<double>(dv[b][u] - lo[b][u] * Qm, dn[b][u], rd[b][u]);
+                if (tdma_writes<R>(lane)) tile[(t0 + g * G + u) * RS + wl] = Qm;
+            };
+            fetch(0, 0);
+            if (c == 0) lo[0][0] = 0.0;
+            if (t0 + K <= len) {
 #pragma unroll
-                        for (int u = 0; u < G; ++u) {
-                            const int o = (s0 + u) * R + rl;
-                            lo[b][u] = slo[o];
-                            dn[b][u] = sden[o];
-                            rd[b][u] = srd[o];
-                            dv[b][u] = sD[o];
-                        }
-                    };
-                    fetch(0, 0);
+                for (int g = 0; g < NG; ++g) {
+                    if (g + 1 < NG) fetch((g + 1) & 1, (g + 1) * G);
 #pragma unroll
-                    for (int g = 0; g < NG; ++g) {
-                        if (g + 1 < NG) fetch((g + 1) & 1, (g + 1) * G);
-                        const int b = g & 1;
+                    for (int u = 0; u < G; ++u) step(g & 1, g, u);
+                }
+            } else {  // the line's last steps
 #pragma unroll
-                        for (int u = 0; u < G; ++u) {
-                            Qm = div_by_rcp<double>(dv[b][u] - lo[b][u] * Qm, dn[b][u], rd[b][u]);
-                            if (tdma_writes<R>(lane)) tile[(t0 + g * G + u) * RS + wl] = Qm;
-                        }
-                    }
-                } else {
-                    const int ns = min(K, len - t0);
-                    for (int s = 0; s < ns; ++s) {
-                        const int o = s * R + rl, t = t0 + s;
-                        Qm = t == 0 ? div_by_rcp<double>(sD[o], sden[o], srd[o])
-                                    : div_by_rcp<double>(sD[o] - slo[o] * Qm, sden[o], srd[o]);
-                        if (tdma_writes<R>(lane)) tile[t * RS + wl] = Qm;
-                    }
+                for (int g = 0; g < NG; ++g) {
+                    if (t0 + g * G >= len) break;
+                    if (g + 1 < NG) fetch((g + 1) & 1, (g + 1) * G);
+#pragma unroll
+                    for (int u = 0; u < G; ++u)
+                        if (t0 + g * G + u < len) step(g & 1, g, u);
                 }
             }
-            tdma_wait_vmem<0>();  // the ring is reused below
+            tdma_handoff();
         }
         // back substitution: x(len-1) = Q(len-1) (already in the tile), then
         // x(t) = P(t) x(t+1) + Q(t) (x-pass, tdma2d9.f90:175-193) or
         // x(t) = x(t+1) P(t) + Q(t) (y-pass, :298-316), t = len-2 .. 0,
         // P streamed in descending steps
-        if (len > 1) {
-            const double *const arr[1] = {tdma_arr(B, S, XPASS, kTP)};
-            const int nst = len - 1, nch = (nst + K - 1) / K;
-            long goff[kTdmaNI];
-            tdma_lane_offsets<R>(goff, k.LP, k.l0, lane, -1);
-            auto issue = [&](int c) {
-                tdma_ldouble *slot = lring + (c % kTdmaSlots) * kTdmaChunk;
-                if (len - 2 - c * K - (K - 1) >= 0)
-                    tdma_issue_at<1>(slot, arr, (long)(len - 2 - c * K) * k.LP, goff);
-                else
-                    tdma_issue<1, R>(slot, arr, k.LP, k.l0, lane,
-                                     [&](int s) { return max(len - 2 - c * K - s, 0); });
-            };
-            for (int c = 0; c < kTdmaSlots - 1; ++c) issue(c);
-            double xv = tile[(len - 1) * RS + rl];
-            for (int c = 0; c < nch; ++c) {
-                issue(c + kTdmaSlots - 1);
-                tdma_wait_vmem<(kTdmaSlots - 1) * kTdmaNI>();
-                const double *sP = ring + (c % kTdmaSlots) * kTdmaChunk;
-                const int ns = min(K, nst - c * K);
-                int t = len - 2 - c * K;
-                if (ns == K) {  // G steps at a time, group g+1's reads beside group g
-                    constexpr int G = 4, NG = K / G;
-                    double pv[2][G], qv[2][G];
-                    auto fetch = [&](int b, int s0) {
+        double xv = tile[(len - 1) * RS + rl];
+        tdma_handoff();
+        for (int c = 0; c < nb; ++c) {
+            const double *sP = ring + (c % kTdmaSlots) * kTdmaChunk;
+            const int ns = min(K, len - 1 - c * K);
+            int t = len - 2 - c * K;
+            if (ns == K) {  // G steps at a time, group g+1's reads beside group g
+                constexpr int G = 4, NG = K / G;
+                double pv[2][G], qv[2][G];
+                auto fetch = [&](int b, int s0) {
 #pragma unroll
-                        for (int u = 0; u < G; ++u) {
-                            pv[b][u] = sP[(s0 + u) * R + rl];
-                            qv[b][u] = tile[(t - s0 - u) * RS + rl];
-                        }
-                    };
-                    fetch(0, 0);
-#pragma unroll
-                    for (int g = 0; g < NG; ++g) {
-                        if (g + 1 < NG) fetch((g + 1) & 1, (g + 1) * G);
-                        const int b = g & 1;
-#pragma unroll
-                        for (int u = 0; u < G; ++u) {
-                            xv = XPASS ? pv[b][u] * xv + qv[b][u] : xv * pv[b][u] + qv[b][u];
-                            if (tdma_writes<R>(lane)) tile[(t - g * G - u) * RS + wl] = xv;
-                        }
+                    for (int u = 0; u < G; ++u) {
+                        pv[b][u] = sP[(s0 + u) * R + rl];
+                        qv[b][u] = tile[(t - s0 - u) * RS + rl];
                     }
-                } else {
-                    for (int s = 0; s < ns; ++s) {
-                        const double pv = sP[s * R + rl], qv = tile[(t - s) * RS + rl];
-                        xv = XPASS ? pv * xv + qv : xv * pv + qv;
-                        if (tdma_writes<R>(lane)) tile[(t - s) * RS + wl] = xv;
+                };
+                fetch(0, 0);
+#pragma unroll
+                for (int g = 0; g < NG; ++g) {
+                    if (g + 1 < NG) fetch((g + 1) & 1, (g + 1) * G);
+                    const int b = g & 1;
+#pragma unroll
+                    for (int u = 0; u < G; ++u) {
+                        xv = XPASS ? pv[b][u] * xv + qv[b][u] : xv * pv[b][u] + qv[b][u];
+                        if (tdma_writes<R>(lane)) tile[(t - g * G - u) * RS + wl] = xv;
                     }
                 }
+            } else {
+                for (int s = 0; s < ns; ++s) {
+                    const double pv = sP[s * R + rl], qv = tile[(t - s) * RS + rl];
+                    xv = XPASS ? pv * xv + qv : xv * pv + qv;
+                    if (tdma_writes<R>(lane)) tile[(t - s) * RS + wl] = xv;
+                }
             }
-            tdma_wait_vmem<0>();
+            tdma_handoff();
         }
     }
     __syncthreads();
     const int LS = XPASS ? B.ny : B.nx;
     const int lanes = min(R, LS - k.l0);  // lines of the grid (the rest is padding)
     if (lanes <= 0) return;
-    if (XPASS) {  // rows l0.. into the x-pass result, row by row
+    // the tile out, a wave at a time, without a division per point
+    const int q = threadIdx.x & 63;
+    if (XPASS) {  // rows l0.. into the x-pass result: a row per wave
         double *out = tdma_tmp(B, S);
-        for (int e = threadIdx.x; e < lanes * len; e += 256) {
-            const int lane = e / len, t = e - lane * len;
-            out[(long)(k.l0 + lane) * B.nx + t] = tile[t * RS + lane];
-        }
-    } else {  // columns l0.. into x
-        for (int e = threadIdx.x; e < lanes * len; e += 256) {
-            const int t = e / lanes, lane = e - t * lanes;
-            S.x[(long)t * B.nx + k.l0 + lane] = tile[t * RS + lane];
-        }
+        for (int lane = wave; lane < lanes; lane += 4)
+            for (int t = q; t < len; t += 64)
+                out[(long)(k.l0 + lane) * B.nx + t] = tile[t * RS + lane];
+    } else {  // columns l0.. into x: 64 / R steps per wave
+        const int lane = q % R;
+        for (int t = wave * (64 / R) + q / R; t < len; t += 4 * (64 / R))
+            if (lane < lanes) S.x[(long)t * B.nx + k.l0 + lane] = tile[t * RS + lane];
     }
 }
 
