@@ -6,6 +6,7 @@
 #include <stdint.h>
 
 #include "mach2d_hip.h"
+#include "seq_layout.h"
 
 namespace m2d {
 
@@ -157,9 +158,8 @@ void cc_terms_enqueue(int nx, int ny, int K, const double *const *a, const int *
                       hipStream_t s);
 // K sums of consecutive arrays of n terms (t + k*n), each the left-to-right
 // loop's value bit for bit, over n if mean, into out[k]; scratch:
-// seq_scratch(n, K) doubles, 16-byte aligned or not
-constexpr int kSeqSegDoubles = 7;
-long seq_scratch(long n, int K);
+// seq_scratch(n, K) doubles (seq_layout.h), 16-byte aligned or not.  A double
+// follows the terms in their allocation (the scratch itself or another one).
 void seq_sums_enqueue(const double *t, long n, int K, double *out, bool mean, double *scratch,
                       hipStream_t s);
 // check_mass_conservation's terms (in = rp, re, rn, Jp, ro, roa, ron, roe,

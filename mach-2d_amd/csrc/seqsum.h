@@ -7,15 +7,16 @@
 // registers) issued kSeqSlots - 1 chunks ahead, which covers the latency of
 // memory another XCD wrote; every lane then adds the terms in order from
 // LDS, with lane-uniform 16-byte reads (a broadcast) issued a few groups of
-// terms ahead of the additions that use them.  Call from a workgroup of
-// kSeqThreads (one wave); every lane returns the sum.
+// terms ahead of the additions that use them.  One wave calls it (no barrier
+// inside); every lane returns the sum.
 #pragma once
 
 #include <hip/hip_runtime.h>
 
+#include "seq_layout.h"
+
 namespace m2d {
 
-constexpr int kSeqThreads = 64;
 constexpr int kSeqChunk = 512, kSeqSlots = 4, kSeqLoads = kSeqChunk / 128;
 
 typedef __attribute__((address_space(1))) const void seq_gvoid;
@@ -196,9 +197,9 @@ __device__ __forceinline__ double seq_add_chunk(const double *slot, double m)
 
 // m + p[0] + p[1] + ... + p[n-1], added left to right; lds: kSeqSlots *
 // kSeqChunk doubles of LDS.  The loads start at p rounded down to 16
-// bytes (the memory before a misaligned p belongs to the same array: every
-// caller's arrays are 256-byte aligned) and never read past the last
-// 16-byte pair that holds p[n-1].
+// bytes (a p that is not on such a boundary lies at least one double inside
+// its allocation, whose start is) and end with the 16-byte pair that holds
+// p[n-1]; the double after it belongs to the sum's scratch (seq_scratch).
 __device__ __forceinline__ double seq_sum(const double *__restrict__ p, long n, double *lds,
                                           double m)
 {
@@ -206,7 +207,7 @@ __device__ __forceinline__ double seq_sum(const double *__restrict__ p, long n, 
     const int sh = (int)(((unsigned long)p >> 3) & 1);  // p[0] at position sh of the stream
     const double *q = p - sh;
     const long nt = n + sh;                            // stream length
-    const long last = (nt - 1) & ~1L;                  // first term of the last pair
+    const long last = seq_last_pair(n, sh);
     const long nch = (nt + kSeqChunk - 1) / kSeqChunk;
     auto issue = [&](long c) {
         double *slot = lds + (c % kSeqSlots) * kSeqChunk;

@@ -45,13 +45,8 @@ namespace m2d {
 
 namespace {
 
-constexpr int kSeqSeg = 512;         // terms of a segment: 8 per lane
 constexpr int kSeqLaneTerms = 8;     // terms per lane of the scans over terms
 constexpr int kSeqGroup = 64 * kSeqLaneTerms;
-// One launch (k_seq_final, every segment from its terms, about 3 us each) up
-// to this many terms, three above: 10 us against 13 at 2048 terms, 17 against
-// 13 at 4096.
-constexpr long kSeqDirect = 2048;
 constexpr double kTwo53 = 9007199254740992.0;
 
 struct Seg {
@@ -451,16 +446,12 @@ __global__ __launch_bounds__(kFinalThreads) void k_seq_final(const double *__res
     if (lane == 0) out[blockIdx.x] = mean ? s / (double)n : s;
 }
 
-int segments(long n) { return n <= kSeqDirect ? 0 : (int)((n + kSeqSeg - 1) / kSeqSeg); }
-
 }  // namespace
-
-long seq_scratch(long n, int K) { return (long)segments(n) * K * kSeqSegDoubles; }
 
 void seq_sums_enqueue(const double *t, long n, int K, double *out, bool mean, double *scratch,
                       hipStream_t s)
 {
-    const int nseg = segments(n);
+    const int nseg = seq_segments(n);
     Seg *segs = (Seg *)scratch;
     if (nseg) {
         const dim3 g((unsigned)((nseg + kSegWaves - 1) / kSegWaves), (unsigned)K);

@@ -39,6 +39,7 @@ def emu():
     E.emu_lu2d9.argtypes = [dp, dp, dp, C.c_int, C.c_int, C.c_double, C.c_int, C.c_uint]
     E.emu_msi_iteration.argtypes = [dp, dp, dp, dp, dp, C.c_int, C.c_int, C.c_int, C.c_uint]
     E.emu_residual.argtypes = [dp, dp, dp, dp, C.c_int, C.c_int]
+    E.emu_seq_loads.argtypes = [C.c_long, C.c_int, C.c_long]
     E.emu_error.restype = C.c_char_p
     return E
 

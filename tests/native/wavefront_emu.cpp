@@ -1,6 +1,6 @@
 // wavefront_emu.cpp -- CPU emulation of the gfx950 wavefront kernels
 // (mach-2d_amd/csrc/sweep.hip: k_factor, k_forward, k_backward, k_to_skew,
-// k_from_skew, k_update).
+// k_from_skew, k_update), and the reach of the in-order sums' loads.
 //
 // Test infrastructure.  The solver's own arrays live in the skewed layout of
 // skew.h (same header as the kernels).  Each band (one wave of 64 lanes)
@@ -29,6 +29,7 @@
 #include <vector>
 
 #include "msi_stencil.h"
+#include "seq_layout.h"
 #include "skew.h"
 
 using namespace m2d;
@@ -573,6 +574,26 @@ void emu_residual(const double *a, const double *x, const double *rhs, double *r
             const long p = (long)j * nx + i;
             r[p] = residual_point<double, double, double>(a, N, x, rhs[p], i, j, nx, ny);
         }
+}
+
+// The one-by-one loads of the in-order sums (seqsum.h, seq_sum): K arrays of
+// n terms at doubles off .. off + K n of an allocation that ends with their
+// scratch, every array read from each segment's start to its end.  0 if every
+// 16-byte pair lies inside the allocation.
+int emu_seq_loads(long n, int K, long off)
+{
+    g_failed = false;
+    const long size = off + K * n + seq_scratch(n, K);
+    for (int k = 0; k < K; ++k)
+        for (long at = 0; at < n; at += kSeqSeg) {
+            const long p = off + k * n + at;
+            const int sh = (int)(p & 1);
+            for (long e = 0; e < n - at + sh + 4 * kSeqSeg; e += 2) {
+                const long q = p - sh + std::min(e, seq_last_pair(n - at, sh));
+                if (q < 0 || q + 1 >= size) fail("a pair outside the terms and their scratch", q, size);
+            }
+        }
+    return g_failed ? 1 : 0;
 }
 
 }  // extern "C"

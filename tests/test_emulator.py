@@ -48,3 +48,13 @@ def test_iteration_schedule_matches_oracle(orc, emu, nx, ny):
         rc = emu.emu_msi_iteration(r, dl, du, x, w, nx, ny, 1 + 7 * k, 100 + k)
         assert rc == 0, emu.emu_error()
     assert np.array_equal(x, ref)
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 511, 512, 513, 514, 1025, 2047, 2048, 2049, 2561, 31873])
+def test_in_order_sum_loads_stay_inside(emu, n):
+    """The in-order sums' one-by-one path reads 16-byte pairs: none may leave
+    the terms and the scratch that follows them, for one array and for the
+    four of a time step, on a 16-byte boundary and off it."""
+    for K in (1, 4, 5):
+        for off in (0, 1, 2, 31):
+            assert emu.emu_seq_loads(n, K, off) == 0, (K, off, emu.emu_error())
