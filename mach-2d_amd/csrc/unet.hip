@@ -784,7 +784,7 @@ __global__ __launch_bounds__(256) void k_pack_weights(PackArgs A)
 }
 
 // Loss 0.5 * sum over masked pixels of (pred - target)^2 / count (1 / count
-// from inv_count, or from the count in device memory), its
+// from inv_count, or from the count in device memory, 0 for a count of 0), its
 // gradient (bf16, `cs` channels with the value in channel 0) and per-block
 // partial sums of the loss.
 __global__ __launch_bounds__(256) void k_mse(const float *pred, int ps, const float *target,
@@ -792,7 +792,7 @@ __global__ __launch_bounds__(256) void k_mse(const float *pred, int ps, const fl
                                              const float *count, __bf16 *grad, int gs,
                                              float *partial)
 {
-    if (count) inv_count = (float)(1.0 / (double)*count);
+    if (count) inv_count = *count != 0.0f ? (float)(1.0 / (double)*count) : 0.0f;
     const long i = (long)blockIdx.x * 256 + threadIdx.x;
     float l = 0.0f;
     if (i < npix) {

@@ -145,6 +145,7 @@ class UNet:
             w[:lay.cout, :9 * lay.cin] = torch.randn(lay.cout, 9 * lay.cin, generator=g) * std
             lay.w.copy_(w)
         self.step_count = 0
+        self._count = None      # pinned copy of a mask's count, its event
         self.pack()
 
     def _one_buffer(self):
@@ -204,13 +205,23 @@ class UNet:
 
     def loss_and_backward(self, x, target, mask, stream=None):
         """One forward and backward pass: loss = 0.5 mean over the mask of
-        (out[..., 0] - target)^2; weight gradients into lay.gw / lay.gb."""
+        (out[..., 0] - target)^2; weight gradients into lay.gw / lay.gb.  A
+        mask without a set pixel has no mean: ZeroDivisionError, and nothing
+        is written."""
         t = self.torch
         n, h, w, _ = x.shape
+        npix = n * h * w
+        # the kernels read the count on the device; the host looks at its copy
+        # while the forward pass runs, so the device does not wait for it
+        cnt = mask.sum(dtype=t.float32)
+        looked = not t.cuda.is_current_stream_capturing()
+        if looked:
+            if self._count is None:
+                self._count = t.empty((), pin_memory=True), t.cuda.Event()
+            self._count[0].copy_(cnt, non_blocking=True)
+            self._count[1].record()
         out = self.forward(x, stream, keep=True)
         acts = self._acts
-        npix = n * h * w
-        cnt = mask.sum(dtype=t.float32)     # stays on the device
         head = self.layers[-1]
         g = t.empty(n, h, w, head.cout, dtype=t.bfloat16, device=self.dev)
         partial = t.empty((npix + 255) // 256, dtype=t.float32, device=self.dev)
@@ -218,6 +229,11 @@ class UNet:
                                          _ptr(cnt), _ptr(g), head.cout, _ptr(partial), stream),
                "mse")
         loss = partial.sum()
+        if looked:
+            self._count[1].synchronize()
+            if float(self._count[0]) == 0.0:
+                self._acts = None
+                raise ZeroDivisionError("loss_and_backward: the mask has no set pixel")
         if self._one_buffer():
             self._flat["g"].zero_()
         else:

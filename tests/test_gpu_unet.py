@@ -526,3 +526,34 @@ def test_grad_in_is_its_pieces(gpu, n, h, w, c, m1, m2):
                               None) == 0
     torch.cuda.synchronize()
     assert torch.equal(got, want)
+
+
+def test_empty_mask_is_refused(gpu):
+    """A mask without a set pixel has no mean: the step raises before any
+    gradient is written, weights and moments stay, and the next step on an
+    ordinary mask runs; the kernel's loss and gradient for a count of 0 are 0."""
+    import ctypes as C
+
+    import torch
+
+    from mach2d import unet as U
+    net = U.UNet(seed=4)
+    g = torch.Generator().manual_seed(9)
+    x, target = _dev(torch.randn(1, 8, 16, 8, generator=g)), torch.ones(1, 8, 16, device="cuda")
+    mask = torch.ones_like(target)
+    net.loss_and_backward(x, target, mask)
+    net.adam_step()
+    keep = [t.clone() for lay in net.layers for t in (lay.w, lay.gw, lay.gb, lay.mw, lay.vw)]
+    with pytest.raises(ZeroDivisionError):
+        net.loss_and_backward(x, target, torch.zeros_like(mask))
+    now = [t for lay in net.layers for t in (lay.w, lay.gw, lay.gb, lay.mw, lay.vw)]
+    assert all(torch.equal(u, v) for u, v in zip(keep, now)) and net.step_count == 1
+    assert bool(torch.isfinite(net.loss_and_backward(x, target, mask)))
+    p = lambda t: C.c_void_p(t.data_ptr())  # noqa: E731
+    pred, grad = torch.randn(300, 8, device="cuda"), torch.ones(300, 8, device="cuda").bfloat16()
+    tgt, msk, cnt = (torch.zeros(k, device="cuda") for k in (300, 300, 1))
+    part = torch.ones(2, device="cuda")
+    assert net.L.m2d_unet_mse_count(p(pred), 8, p(tgt), p(msk), 300, p(cnt), p(grad), 8, p(part),
+                                    None) == 0
+    torch.cuda.synchronize()
+    assert not part.any() and not grad.float().any()
