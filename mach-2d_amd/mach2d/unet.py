@@ -127,14 +127,16 @@ class UNet:
         # step zeroes and updates them all at once
         sizes = [k for lay in self.layers for k in (lay.cpad * lay.kpad, _r(lay.cout, 4))]
         self._flat = {k: torch.zeros(sum(sizes), device=device) for k in ("p", "g", "m", "v")}
+        self._places = {k: [] for k in self._flat}   # (layer, name, byte offset, shape)
         for k, (wn, bn) in (("p", ("w", "b")), ("g", ("gw", "gb")), ("m", ("mw", "mb")),
                             ("v", ("vw", "vb"))):
             parts = iter(torch.split(self._flat[k], sizes))
             for lay in self.layers:
                 setattr(lay, wn, next(parts).view(lay.cpad, lay.kpad))
                 setattr(lay, bn, next(parts)[:lay.cout])
-        self._views = [(lay, k, getattr(lay, k)) for lay in self.layers
-                       for k in ("w", "b", "gw", "gb", "mw", "mb", "vw", "vb")]
+                for name in (wn, bn):
+                    v = getattr(lay, name)
+                    self._places[k].append((lay, name, 4 * v.storage_offset(), v.shape))
         for lay in self.layers:
             lay.wb = torch.zeros(lay.cpad, lay.kpad, dtype=torch.bfloat16, device=device)
             lay.wr = torch.zeros(lay.cin_pad, lay.kpad_r, dtype=torch.bfloat16, device=device)
@@ -148,10 +150,16 @@ class UNet:
         self._count = None      # pinned copy of a mask's count, its event
         self.pack()
 
-    def _one_buffer(self):
-        """The layers' tensors are still the views of the one buffer (a caller
-        may have put others in their place)."""
-        return all(getattr(lay, k) is v for lay, k, v in self._views)
+    def _one_buffer(self, kinds="pgmv"):
+        """The layers' tensors still lie in the one buffer of their kind (a
+        caller may have put others, or other storage, in their place)."""
+        for k in kinds:
+            base = self._flat[k].data_ptr()
+            for lay, name, off, shape in self._places[k]:
+                t = getattr(lay, name)
+                if t.data_ptr() != base + off or t.shape != shape:
+                    return False
+        return True
 
     def pack(self, stream=None):
         """bf16 copies of the weights (forward and input-gradient forms)."""
@@ -234,7 +242,7 @@ class UNet:
             if float(self._count[0]) == 0.0:
                 self._acts = None
                 raise ZeroDivisionError("loss_and_backward: the mask has no set pixel")
-        if self._one_buffer():
+        if self._one_buffer("g"):
             self._flat["g"].zero_()
         else:
             for lay in self.layers:

@@ -557,3 +557,43 @@ def test_empty_mask_is_refused(gpu):
                                     None) == 0
     torch.cuda.synchronize()
     assert not part.any() and not grad.float().any()
+
+
+@pytest.mark.parametrize("what", ["tensors", "storage", "one bias gradient"])
+def test_training_follows_replaced_tensors(gpu, what):
+    """Weights, gradients and moments that a caller puts in the place of the
+    layers' own, as new tensors or as new storage of the old ones, are the
+    ones that training reads and updates: the same steps as on the layers'
+    own tensors (gradients to the order of their atomic additions)."""
+    import torch
+
+    from mach2d import unet as U
+    g = torch.Generator().manual_seed(21)
+    x, target = _dev(torch.randn(2, 16, 24, 8, generator=g)), torch.randn(2, 16, 24, generator=g).cuda()
+    mask = torch.ones_like(target)
+    own, net = U.UNet(seed=6), U.UNet(seed=6)
+    names = ("w", "b", "gw", "gb", "mw", "mb", "vw", "vb")
+    if what == "one bias gradient":
+        net.layers[2].gb.data = torch.full_like(net.layers[2].gb, 7.0)
+    else:
+        for lay in net.layers:
+            for k in names:
+                if what == "tensors":
+                    setattr(lay, k, getattr(lay, k).clone())
+                else:
+                    getattr(lay, k).data = getattr(lay, k).clone()
+    before = [lay.w.clone() for lay in net.layers]
+    for n in (own, net):
+        losses = [float(n.loss_and_backward(x, target, mask))]
+        n.adam_step()
+        losses.append(float(n.loss_and_backward(x, target, mask)))
+        n.losses = losses
+    for u, v, w in zip(own.layers, net.layers, before):
+        assert not torch.equal(v.w, w), v.name
+        for k in names:
+            a, b = getattr(u, k), getattr(v, k)
+            # a step is at most lr = 1e-3; a gradient near zero may turn its sign
+            tol = 2e-3 if k in ("w", "b") else 1e-2 * float(a.norm()) + 1e-12
+            assert float((a - b).abs().max()) <= tol, (v.name, k)
+    assert net.losses[0] == pytest.approx(own.losses[0], rel=1e-5)
+    assert net.losses[1] < net.losses[0] and net.losses[1] == pytest.approx(own.losses[1], rel=1e-2)
