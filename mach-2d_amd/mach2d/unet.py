@@ -253,12 +253,7 @@ class UNet:
             lv = LEVEL[lay.name]
             hh, ww = h >> lv, w >> lv
             if lay.name != "head":
-                g = t.empty_like(acts[lay.name])
-                srcs = into.pop(lay.name)
-                (g1, cs1, c01, m1), (g2, cs2, c02, m2) = (srcs + [(None, 0, 0, 0)])[:2]
-                _check(self.L.m2d_unet_grad_in(_ptr(g1), cs1, c01, m1, _ptr(g2), cs2, c02, m2,
-                                               _ptr(acts[lay.name]), lay.cout, n, hh, ww, _ptr(g),
-                                               stream), "grad_in")
+                g = self._grad_out(lay, into.pop(lay.name), acts[lay.name], stream)
             src, skip = acts[lay.src], acts[lay.skip] if lay.skip else None
             _check(self.L.m2d_unet_conv3x3_wgrad(_ptr(src), lay.c1, lay.mode, _ptr(skip), lay.c2,
                                                  _ptr(g), lay.cout, lay.kpad, n, hh, ww,
@@ -275,6 +270,29 @@ class UNet:
                     into.setdefault(name, []).append((gi, lay.cin, c0, mode))
         self._acts = None
         return loss
+
+    def _grad_out(self, lay, srcs, y, stream):
+        """bf16 gradient at a layer's pre-activation output y from those of
+        the convolution inputs it went into (FP32 tensor, its channels, first
+        channel, mode): one pass for up to two of them and a ReLU, as all of
+        LAYERS have; else added one by one, rounded, and cut where there is a
+        ReLU."""
+        t = self.torch
+        n, h, w, c = y.shape
+        g = t.empty_like(y)
+        if lay.relu and len(srcs) <= 2:
+            (g1, cs1, c01, m1), (g2, cs2, c02, m2) = (srcs + [(None, 0, 0, 0)])[:2]
+            _check(self.L.m2d_unet_grad_in(_ptr(g1), cs1, c01, m1, _ptr(g2), cs2, c02, m2,
+                                           _ptr(y), c, n, h, w, _ptr(g), stream), "grad_in")
+            return g
+        acc = t.zeros(y.shape, dtype=t.float32, device=self.dev)
+        for gi, cs, c0, mode in srcs:
+            _check(self.L.m2d_unet_mode_bwd(_ptr(gi), cs, c0, c, mode, n, gi.shape[1],
+                                            gi.shape[2], _ptr(acc), stream), "mode_bwd")
+        _check(self.L.m2d_unet_to_bf16(_ptr(acc), _ptr(g), g.numel(), stream), "to_bf16")
+        if lay.relu:
+            _check(self.L.m2d_unet_relu_bwd(_ptr(g), _ptr(y), g.numel(), stream), "relu_bwd")
+        return g
 
     def adam_step(self, lr=1e-3, b1=0.9, b2=0.999, eps=1e-8, stream=None):
         self.step_count += 1

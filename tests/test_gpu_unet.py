@@ -597,3 +597,56 @@ def test_training_follows_replaced_tensors(gpu, what):
             assert float((a - b).abs().max()) <= tol, (v.name, k)
     assert net.losses[0] == pytest.approx(own.losses[0], rel=1e-5)
     assert net.losses[1] < net.losses[0] and net.losses[1] == pytest.approx(own.losses[1], rel=1e-2)
+
+
+def test_backward_follows_the_layer_table(gpu, monkeypatch):
+    """A network of another table: a layer without ReLU, and one whose output
+    three convolutions read.  Weight and bias gradients against autograd of
+    the FP32 network (activations and their gradients rounded to bf16, as the
+    kernels do): 2e-2 of a layer's gradient, the bound of a bf16 network; the
+    cut of a missing ReLU or a reader left out is of the order of 1."""
+    import torch
+
+    from mach2d import unet as U
+    table = [("a", "x", U.DIRECT, None, 16, False), ("b", "a", U.DIRECT, None, 16, True),
+             ("c", "b", U.DIRECT, "a", 16, True), ("d", "c", U.DIRECT, "a", 16, True),
+             ("e", "d", U.POOL, None, 16, False), ("f", "e", U.UP, "d", 16, True),
+             ("head", "f", U.DIRECT, None, 8, False)]
+    monkeypatch.setattr(U, "LAYERS", table)
+    monkeypatch.setattr(U, "LEVEL", {n: int(n == "e") for n, *_ in table})
+    net = U.UNet(seed=8)
+    g = torch.Generator().manual_seed(3)
+    x = _bf(torch.randn(2, 8, 24, 8, generator=g))
+    target, mask = torch.randn(2, 8, 24, generator=g), torch.ones(2, 8, 24)
+    mask[:, 3:5, 7:] = 0.0
+    loss = net.loss_and_backward(_dev(x), target.cuda(), mask.cuda())
+
+    def rnd(v):   # rounded to bf16 both ways
+        v = v + (_bf(v) - v).detach()
+        if v.requires_grad:
+            v.register_hook(_bf)
+        return v
+    acts, params = {"x": x}, []
+    for lay in net.layers:
+        w = _bf(lay.w.cpu()[:lay.cout, :9 * lay.cin]).requires_grad_(True)
+        b = lay.b.cpu().clone().requires_grad_(True)
+        params.append((lay, w, b))
+        src = acts[lay.src]
+        if lay.mode == U.POOL:
+            mean = src.unflatten(1, (-1, 2)).unflatten(3, (-1, 2)).mean(dim=(2, 4))
+            src = _pool(src.detach()) + (mean - mean.detach())
+        elif lay.mode == U.UP:
+            src = _effective(src, 2, None)
+        if lay.skip:
+            src = torch.cat([src, acts[lay.skip]], dim=3)
+        y = _ref_conv(src, w, b, lay.cin, lay.cout, False)
+        if y.requires_grad and lay.name != "head":
+            y.register_hook(_bf)
+        acts[lay.name] = y if lay.name == "head" else rnd(torch.relu(y) if lay.relu else y)
+    d = (acts["head"][..., 0] - target) * mask
+    want = 0.5 * (d * d).sum() / mask.sum()
+    want.backward()
+    assert float(loss) == pytest.approx(float(want.detach()), rel=2e-2)
+    for lay, w, b in params:
+        for got, ref in ((lay.gw.cpu()[:lay.cout, :9 * lay.cin], w.grad), (lay.gb.cpu(), b.grad)):
+            assert float((got - ref).norm()) <= 2e-2 * float(ref.norm()), lay.name
