@@ -184,6 +184,15 @@ int m2d_solve(m2d_system *s, const double *d_a, const double *d_rhs,
 
 int m2d_set_inner(m2d_system *s, double inner_gamma, int inner_nitm);
 
+/* FP32_IR: how many earlier directions a step is made orthogonal to (0..4).
+ * A handle is created with 4, or with as many as the free memory holds then
+ * (two vectors of nx*ny floats each); fewer keep the stopping rule and give
+ * other iterates, mostly a few more of them.  _get: the number in use; _set:
+ * M2D_ERR_ARG beyond what the handle was created with.  Solves of one window
+ * are reproducible. */
+int m2d_set_window(m2d_system *s, int directions);
+int m2d_get_window(m2d_system *s, int *directions);
+
 /* ||A.var - rhs||_2 in FP64 (device pointers), the norm fb2d9 starts from
  * (msi2d9-v03.f90:59-133); used to judge an initial guess against the zero
  * guess before a solve. */
@@ -266,6 +275,10 @@ int m2d_batch_solve_each(m2d_batch *b, const double *const *d_a, const double *c
 
 /* FP32_IR: the inner stopping rule (as m2d_set_inner). */
 int m2d_batch_set_inner(m2d_batch *b, double inner_gamma, int inner_nitm);
+
+/* FP32_IR: the window of directions (as m2d_set_window, m2d_get_window). */
+int m2d_batch_set_window(m2d_batch *b, int directions);
+int m2d_batch_get_window(m2d_batch *b, int *directions);
 
 /* Launch placement: layout 0 = systems in order, 1 = each system's bands on
  * one XCD (longest-processing-time assignment), 2 = largest systems first;

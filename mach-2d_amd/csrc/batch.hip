@@ -447,6 +447,7 @@ struct m2d_batch {
     double inner_gamma = 1e-4;
     int inner_nitm = 50;
     int kry_r = 1;  // points per thread of the correction solves' kernels (1 or 2)
+    int kry_max = 0;  // directions the correction solves' vectors hold
     bool factored = false;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
 };
@@ -862,6 +863,7 @@ extern "C" int m2d_batch_create(int count, const int *nx, const int *ny, int pre
         ok = hipMemset(p64, 0, sizeof(double) * 21 * L) == hipSuccess;
     else
         ok = hipMemset(p32, 0, sizeof(float) * 21 * L) == hipSuccess;
+    b->kry_max = win;
     b->h64.resize(count);
     if (!fp64) b->h32.resize(count);
     long ls = 0, ln = 0, lp = 0, lw = 0, lk = 0;
@@ -948,6 +950,22 @@ extern "C" int m2d_batch_set_inner(m2d_batch *b, double inner_gamma, int inner_n
         i.gamma = inner_gamma;
         i.nitm = inner_nitm;
     }
+    return M2D_OK;
+}
+
+// (the descriptors go to the device with every correction solve)
+extern "C" int m2d_batch_set_window(m2d_batch *b, int directions)
+{
+    if (!b || b->precision != M2D_FP32_IR || directions < 0 || directions > b->kry_max)
+        return M2D_ERR_ARG;
+    for (auto &i : b->h32) i.kry.win = directions;
+    return M2D_OK;
+}
+
+extern "C" int m2d_batch_get_window(m2d_batch *b, int *directions)
+{
+    if (!b || b->precision != M2D_FP32_IR || !directions) return M2D_ERR_ARG;
+    *directions = b->h32[0].kry.win;
     return M2D_OK;
 }
 

@@ -134,6 +134,7 @@ struct m2d_system {
     double *r64 = nullptr;
     float *kry_mem = nullptr;
     KrylovVec kry{};
+    int kry_max = 0;  // directions kry_mem holds
     u64 *kry_partial = nullptr;
 
     u64 *partial = nullptr;  // residual partial sums (tagged words)
@@ -328,6 +329,7 @@ extern "C" int m2d_create_stencil(int nx, int ny, int precision, int ndiag, m2d_
             s->kry_mem = nullptr;
             ok = s->kry.win > 0;
         }
+        s->kry_max = s->kry.win;
         s->kry.q = s->kry_mem;
         s->kry.r = s->kry_mem + (s->kry.win + 1) * N;
         s->kry.p = s->kry_mem + (s->kry.win + 2) * N;
@@ -380,6 +382,21 @@ extern "C" int m2d_set_inner(m2d_system *s, double inner_gamma, int inner_nitm)
     if (!s || !(inner_gamma > 0.0) || inner_nitm < 1) return M2D_ERR_ARG;
     s->inner_gamma = inner_gamma;
     s->inner_nitm = inner_nitm;
+    return M2D_OK;
+}
+
+extern "C" int m2d_set_window(m2d_system *s, int directions)
+{
+    if (!s || s->precision != M2D_FP32_IR || directions < 0 || directions > s->kry_max)
+        return M2D_ERR_ARG;
+    s->kry.win = directions;
+    return M2D_OK;
+}
+
+extern "C" int m2d_get_window(m2d_system *s, int *directions)
+{
+    if (!s || s->precision != M2D_FP32_IR || !directions) return M2D_ERR_ARG;
+    *directions = s->kry.win;
     return M2D_OK;
 }
 

@@ -48,6 +48,7 @@ EXPORTS = [
     "m2d_lu2d5", "m2d_fb2d5", "m2d_solve_msi5d", "m2d_create_stencil", "m2d_norm_l1_9d",
     "m2d_norm_l1_9d_relative", "m2d_norm_l1_b", "m2d_last_status", "m2d_create",
     "m2d_destroy", "m2d_set_stream", "m2d_factor", "m2d_solve", "m2d_set_inner",
+    "m2d_set_window", "m2d_get_window", "m2d_batch_set_window", "m2d_batch_get_window",
     "m2d_get_factor", "m2d_set_tuning", "m2d_set_staging", "m2d_tdma2d9_device",
     "m2d_residual_norm", "m2d_guess_scale", "m2d_guess_scale_energy",
     "m2d_version", "m2d_enable_kernel_timing", "m2d_kernel_timing",
@@ -136,6 +137,10 @@ def load():
     L.m2d_solve.restype = C.c_int
     L.m2d_set_inner.argtypes = [_vp, C.c_double, C.c_int]
     L.m2d_set_inner.restype = C.c_int
+    for f in (L.m2d_set_window, L.m2d_batch_set_window):
+        f.argtypes, f.restype = [_vp, C.c_int], C.c_int
+    for f in (L.m2d_get_window, L.m2d_batch_get_window):
+        f.argtypes, f.restype = [_vp, C.POINTER(C.c_int)], C.c_int
     L.m2d_residual_norm.argtypes = [_vp, _vp, _vp, _vp, C.POINTER(C.c_double)]
     for f in (L.m2d_guess_scale, L.m2d_guess_scale_energy):
         f.argtypes = [_vp, _vp, _vp, _vp, C.POINTER(C.c_double)]

@@ -438,6 +438,22 @@ class DeviceMSI:
         if rc:
             raise SolverError(rc, "m2d_set_inner")
 
+    def set_window(self, directions=4):
+        """FP32_IR: earlier directions a step is made orthogonal to (0..4, at
+        most as many as the handle was created with)."""
+        rc = _lib.load().m2d_set_window(self.h, int(directions))
+        if rc:
+            raise SolverError(rc, "m2d_set_window")
+
+    def window(self):
+        """FP32_IR: the directions in use; below 4 after creation where the
+        memory left then did not hold more."""
+        n = C.c_int()
+        rc = _lib.load().m2d_get_window(self.h, C.byref(n))
+        if rc:
+            raise SolverError(rc, "m2d_get_window")
+        return n.value
+
     def factor(self, a):
         rc = _lib.load().m2d_factor(self.h, C.c_void_p(self._chk(a, self.nd * self.N, "a")))
         if rc and rc != _lib.M2D_ERR_NONFINITE:
@@ -577,6 +593,22 @@ class BatchMSI:
         rc = _lib.load().m2d_batch_set_inner(self.h, float(inner_gamma), int(inner_nitm))
         if rc:
             raise SolverError(rc, "m2d_batch_set_inner")
+
+    def set_window(self, directions=4):
+        """FP32_IR: earlier directions a step is made orthogonal to (0..4, at
+        most as many as the handle was created with)."""
+        rc = _lib.load().m2d_batch_set_window(self.h, int(directions))
+        if rc:
+            raise SolverError(rc, "m2d_batch_set_window")
+
+    def window(self):
+        """FP32_IR: the directions in use; below 4 after creation where the
+        memory left then did not hold more."""
+        n = C.c_int()
+        rc = _lib.load().m2d_batch_get_window(self.h, C.byref(n))
+        if rc:
+            raise SolverError(rc, "m2d_batch_get_window")
+        return n.value
 
     def set_tuning(self, layout=0, chunk_iters=8):
         rc = _lib.load().m2d_batch_set_tuning(self.h, int(layout), int(chunk_iters))

@@ -133,3 +133,54 @@ def test_batch_two_points_per_thread(gpu, orc):
         bt.close()
     for u, v in zip(*xs):
         assert float((u - v).norm()) <= 1e-8 * float(u.norm())
+
+
+def test_shorter_windows(gpu, orc):
+    """Windows below the full one, which a handle gets where memory is short:
+    the same solution, the window reported, refused beyond what there is, and
+    equal calls equal bit for bit; single system and batch."""
+    import torch
+    sys_ = [P.pcorr_system(66, 34, seed=2, rhs="gauss"), _recirculating(40, 22)]
+    want = [_oracle(orc, s, 9) for s in sys_]
+    a = [torch.tensor(s.a.reshape(-1), device="cuda") for s in sys_]
+    b = [torch.tensor(s.rhs, device="cuda") for s in sys_]
+    bt = gpu.BatchMSI([(s.nx, s.ny) for s in sys_], precision="fp32_ir")
+    devs = [gpu.DeviceMSI(s.nx, s.ny, "fp32_ir") for s in sys_]
+    bt.factor(a)
+    for d, m in zip(devs, a):
+        d.factor(m)
+    for h in devs + [bt]:
+        assert h.window() == 4
+        with pytest.raises(gpu.SolverError):
+            h.set_window(5)
+        with pytest.raises(gpu.SolverError):
+            h.set_window(-1)
+        assert h.window() == 4
+    nits = set()
+    for win in (0, 1, 2, 3, 4):
+        runs = []
+        for _ in range(2):
+            x = [torch.zeros(s.N, dtype=torch.float64, device="cuda") for s in sys_]
+            y = [torch.zeros_like(t) for t in x]
+            bt.set_window(win)
+            assert bt.window() == win
+            _, st = bt.solve(a, b, x, 1e-10, 20000)
+            for q, d in enumerate(devs):
+                d.set_window(win)
+                sd = d.solve(a[q], b[q], y[q], 1e-10, 20000)
+                for stat, sol in ((st[q], x[q]), (sd, y[q])):
+                    assert stat.status == 0 and stat.rn < 1e-10 * stat.r0, (win, q)
+                    ox, onit = want[q]
+                    err = np.linalg.norm(sol.cpu().numpy() - ox)
+                    assert err <= (1e-8 if q == 0 else 5e-8) * np.linalg.norm(ox), (win, q)
+                if q == 0:
+                    nits.add(sd.nit)
+            runs.append(x + y)
+        assert all(torch.equal(u, v) for u, v in zip(*runs)), win
+    assert len(nits) > 1    # the window is what is used
+    for h in devs + [bt]:
+        h.close()
+    fp64 = gpu.DeviceMSI(8, 8, "fp64")
+    with pytest.raises(gpu.SolverError):
+        fp64.window()
+    fp64.close()

@@ -353,6 +353,9 @@ def test_tuning_entries_check_their_arguments():
     assert L.m2d_set_pl_solve_cap(None, 4) == _lib.M2D_ERR_ARG
     assert L.m2d_pl_loop_cap_info(None, C.byref(a), C.byref(b)) == _lib.M2D_ERR_ARG
     assert L.m2d_pl_loop_info(None, C.byref(a), C.byref(b)) == _lib.M2D_ERR_ARG
+    for p in ("m2d_", "m2d_batch_"):
+        assert getattr(L, p + "set_window")(None, 2) == _lib.M2D_ERR_ARG
+        assert getattr(L, p + "get_window")(None, C.byref(a)) == _lib.M2D_ERR_ARG
 
 
 def test_m2dt_round_trip_and_checks(tmp_path):
