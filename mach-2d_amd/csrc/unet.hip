@@ -992,7 +992,7 @@ extern "C" int m2d_unet_conv3x3_wgrad(const void *in1, int c1, int mode1, const 
     const int cin = c1 + c2;
     if (!in1 || c1 <= 0 || c1 % 8 || c2 < 0 || c2 % 8 || (c2 && !in2) || !g || !dw ||
         cout <= 0 || kpad < 9 * cin || kpad % 32 || n <= 0 || h <= 0 || w_ <= 0 ||
-        mode1 < 0 || mode1 > 2)
+        mode1 < 0 || mode1 > 2 || (mode1 == kModeUp && (h % 2 || w_ % 2)))
         return M2D_ERR_ARG;
     WgradArgs W;
     W.c.in1 = In{(const __bf16 *)in1, c1, mode1};

@@ -358,6 +358,22 @@ def test_tuning_entries_check_their_arguments():
         assert getattr(L, p + "get_window")(None, C.byref(a)) == _lib.M2D_ERR_ARG
 
 
+def test_unet_convolutions_refuse_odd_upsampling():
+    """An upsampled input has half the rows and columns: odd sizes would read
+    a row or column past it, so the convolution and its weight gradient both
+    refuse them before the GPU is touched."""
+    import ctypes as C
+
+    from mach2d import _lib, unet as U
+    L = U._bind()
+    p = C.c_void_p(4096)
+    for h, w in ((5, 8), (8, 5), (1, 2)):
+        assert L.m2d_unet_conv3x3(p, 16, U.UP, None, 0, p, None, 16, 16, 160, 1, h, w, 0, p, None, 0,
+                                  None) == _lib.M2D_ERR_ARG
+        assert L.m2d_unet_conv3x3_wgrad(p, 16, U.UP, None, 0, p, 16, 160, 1, h, w, p, None,
+                                        None) == _lib.M2D_ERR_ARG
+
+
 def test_m2dt_round_trip_and_checks(tmp_path):
     """The training-set format: records and metadata come back as written
     (float32), the header carries grid, diagonals, count, gamma and source,
