@@ -56,20 +56,49 @@ def _sum_patterns(n, rng):
     }
 
 
-@pytest.mark.parametrize("n", [1, 3, 4, 5, 255, 256, 257, 511, 513, 4095, 4096, 4097, 4608, 32768,
-                               33291, 66049])
-def test_in_order_sums_are_the_left_to_right_loop(gpu, orc, n):
-    """get_average of n real volumes (nx = n + 2, ny = 3): the oracle's loop
-    bit for bit, for sizes at the edges of the groups of 256 terms, the
-    segments of 512 and the one-launch range (4096)."""
+def _average(nx, ny, t):
+    """get_average on the GPU of the terms t as the real volumes."""
     import torch
 
     from mach2d import assembly as A
-    nx, ny = n + 2, 3
+    F = np.zeros((ny, nx))
+    F[1:-1, 1:-1] = t.reshape(ny - 2, nx - 2)
+    return F.reshape(-1), A.get_average(nx, ny, torch.tensor(F.reshape(-1), device="cuda"))
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 255, 256, 257, 511, 512, 513, 1023, 1024, 1025, 1535,
+                               2047, 2048, 2049, 2560, 2561, 4095, 4096, 4097, 4608, 32768, 33291,
+                               66049])
+def test_in_order_sums_are_the_left_to_right_loop(gpu, orc, n):
+    """get_average of n real volumes (nx = n + 2, ny = 3): the oracle's loop
+    bit for bit, for sizes at the edges of the segments of 512 terms, on both
+    sides of the one-launch range (2048), and for a last segment of one."""
     for name, t in _sum_patterns(n, np.random.default_rng(n)).items():
-        F = np.zeros((ny, nx))
-        F[1, 1:-1] = t
+        F, got = _average(n + 2, 3, t)
         with np.errstate(over="ignore", invalid="ignore"):
-            want = orc.get_average(nx, ny, F.reshape(-1))
-        got = A.get_average(nx, ny, torch.tensor(F.reshape(-1), device="cuda"))
+            want = orc.get_average(n + 2, 3, F)
+        assert np.array_equal(got, want, equal_nan=True), (name, got, want)
+
+
+@pytest.mark.parametrize("nx,ny", [(1026, 514), (1027, 515), (2051, 515)])
+def test_in_order_sums_beyond_the_staged_maps(gpu, orc, nx, ny):
+    """524288 terms (1024 segments: all that the last kernel stages at once)
+    and more: sums that leave their binade, stop at a bad term or meet ties in
+    the first round of staged segments, at its end, and in a later round."""
+    n = (nx - 2) * (ny - 2)
+    rng = np.random.default_rng(n)
+    base = rng.uniform(0, 1, n)
+    edge = 1024 * 512                      # first term of the second round
+    cases = {"uniform": base, "ties": rng.integers(0, 64, n) * 2.0 ** -10 + 2.0 ** -34,
+             "zeros, then one": np.r_[np.zeros(n - 1), 1.0], "constant": np.full(n, 0.1)}
+    for at in (700, edge - 1, edge, edge + 513, n - 1):
+        if at < n:
+            for name, v in (("negative", -0.25), ("nan", np.nan), ("inf", np.inf),
+                            ("next binade", 3e6), ("far binade", 1e300)):
+                cases["%s at %d" % (name, at)] = base.copy()
+                cases["%s at %d" % (name, at)][at] = v
+    for name, t in cases.items():
+        F, got = _average(nx, ny, t)
+        with np.errstate(over="ignore", invalid="ignore"):
+            want = orc.get_average(nx, ny, F)
         assert np.array_equal(got, want, equal_nan=True), (name, got, want)
