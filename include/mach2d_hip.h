@@ -699,7 +699,8 @@ int m2d_unet_grad_in(const float *g1, int cs1, int c01, int mode1, const float *
                      void *stream);
 /* 0.5*sum(mask*(pred - target)^2)*inv_count: per-256-pixel partial sums and
  * the bf16 gradient (gs channels, value in channel 0).  _count: 1 / *count, a
- * device value, for inv_count; a count of 0 gives a loss and gradient of 0. */
+ * device value, for inv_count; a count of 0 gives a loss and gradient of 0
+ * (the training step's form; the other is for a count known on the host). */
 int m2d_unet_mse_count(const float *pred, int ps, const float *target, const float *mask,
                        long npix, const float *count, void *grad, int gs, float *partial,
                        void *stream);

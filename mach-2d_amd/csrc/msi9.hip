@@ -562,6 +562,5 @@ template void launch_update_residual_norm<double>(const double *, double *, doub
 template void launch_settle<double>(double *, const double *, long, const SolveState *,
                                     hipStream_t);
 template void launch_convert<double, float>(const double *, float *, long, hipStream_t);
-template void launch_convert<float, double>(const float *, double *, long, hipStream_t);
 
 }  // namespace m2d
