@@ -71,10 +71,10 @@ BYTES_PER_POINT = {
 # WRITE_SIZE in separate runs of this script, scaled by 2.2488 and 1.1250:
 # the factors a conversion kernel of known size reads;
 # profiles/msi_1026x514_hbm_traffic.md).  "residual" is the update and the
-# residual of one launch.
+# residual of one launch, "residual32" the two launches around a sweep pair.
 MEASURED_TRAFFIC = {
-    "sweeps": 84.95e6, "residual": 67.13e6, "factor": 111.72e6,
-    "sweeps32": 39.25e6, "factor32": 55.94e6,
+    "sweeps": 83.60e6, "residual": 67.14e6, "factor": 111.44e6,
+    "sweeps32": 37.69e6, "residual32": 76.61e6, "factor32": 55.93e6,
 }
 
 

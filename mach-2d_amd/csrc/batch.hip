@@ -258,9 +258,9 @@ __global__ __launch_bounds__(kPts) void k_a32_batch(const BatchSys<double> *__re
 // ---- the accelerated FP32 correction solves (krylov.h) ---------------------
 // kPts * R points per workgroup, R per thread (256 apart).  What bounds them:
 // 16 and 17 vectors streamed; 256 systems of 64s x 32s points, s in [1, 8] (7.9
-// million points): apply 98 us, step 70 us (5.2 and 7.2 TB/s, the last-level
-// cache helping), of 360 per iteration; 112 and 75 us with one point per
-// thread, 97 and 72 with four.
+// million points), all of them still at work: apply 123 us, step 96 us (4.1
+// and 5.6 TB/s, the last-level cache helping), of 455 per iteration; 141 and
+// 97 us with one point per thread, 121 and 99 with four.
 template <int R>
 __global__ __launch_bounds__(kPts) void k_krylov_start_batch(
     const BatchSys<double> *__restrict__ s64, const BatchSys<float> *__restrict__ s32,

@@ -111,8 +111,8 @@ struct m2d_system {
     // 8: the bands of the system on one XCD (workgroups are dealt to the
     // XCDs round robin, every eighth runs a band); 1: on consecutive XCDs.
     // 1 by default: the fed sweeps of 1026x514 (9 bands, FP64, 9 diagonals)
-    // take 324 us a pair on consecutive XCDs; 8 leaves them too few CUs, and
-    // the register sweeps take 362 us on one XCD, which also holds no more
+    // take 320 us a pair on consecutive XCDs; 8 leaves them too few CUs, and
+    // the register sweeps take 364 us on one XCD, which also holds no more
     // than 64 bands at once
     int xcd_stride = 1;
     // the two-wave LDS-staged sweeps, one launch each (m2d_set_staging); off

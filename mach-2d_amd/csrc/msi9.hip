@@ -215,9 +215,10 @@ __global__ __launch_bounds__(kResThreads) void k_residual(const TA *__restrict__
 //
 // What bounds them: the 16 and 17 vectors of N floats each that they stream, from
 // the last-level cache, and on smaller grids the launch and the last
-// workgroup's wait.  Measured (apply + step): 1026x514, 9 diagonals, 17.7 +
-// 10.7 us (the residual kernel of plain MSI: 12; a sweep pair: 158); 515x259,
-// 5 diagonals, 12.6 + 6.6 us of 105 per iteration.
+// workgroup's wait.  Measured in solves (apply + step, most iterations with
+// all four kept directions): 1026x514, 9 diagonals, 20.8 + 12.5 us (the residual
+// kernel of plain MSI: 12; a sweep pair: 166); 515x259, 5 diagonals, 12.4 + 6.8
+// us beside a sweep pair of 70.
 // --------------------------------------------------------------------------
 template <int R>
 __host__ __device__ inline int krylov_blocks(long n)
@@ -227,8 +228,8 @@ __host__ __device__ inline int krylov_blocks(long n)
 
 // Points per thread: 2 once that leaves two workgroups per CU (half the
 // partial sums for the last workgroup to add up), else 1, so that more CUs
-// have work.  apply + step with 1, 2 and 4 points: 1026x514 33.8, 28.5 and
-// 29.6 us; 515x259 19.3, 20.0 and 23.5 us.
+// have work.  apply + step with 1, 2 and 4 points: 1026x514 39.2, 33.3 and
+// 35.8 us; 515x259 19.2, 20.0 and 22.1 us.
 static bool krylov_two(long n) { return n >= 512L * 512; }
 
 long krylov_partial_words(int nx, int ny)

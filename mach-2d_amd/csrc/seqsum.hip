@@ -34,8 +34,10 @@
 // What bounds it: the sequential chain took 4.2 ns (10 cycles) per term, 2.2
 // ms for the 524288 terms of a 1026x514 grid; now the last kernel's chain of
 // scans (about 900 cycles each) and the launches.  Measured on MI355X, the
-// kernels of one sum: 524288 terms 2222 -> 27 us, 32768 terms 141 ->
-// 16 us.
+// kernels of one sum: 524288 terms 2222 -> 28 us, 32768 terms 141 ->
+// 16 us.  A sum that stays zero has no binade, so its segments are taken from
+// their terms one after the other, about 1 us each: 32768 zeros (the T
+// system's neighbours in an Euler step) 141 -> 70 us.
 #include <hip/hip_runtime.h>
 
 #include "m2d_internal.h"

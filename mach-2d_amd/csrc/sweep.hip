@@ -908,9 +908,9 @@ __device__ __forceinline__ void backward_band_staged(T *__restrict__ wz, const T
 // wave with stores wait for the stores before them (one in-order counter):
 // hence a wave each.  Instructions of the computing wave per chunk (FP64, 5
 // diagonals): forward 240 -> 164, backward 200 -> 118.  A sweep pair, register
-// sweeps and fed: FP64 258x130, 5 diagonals 88.5 -> 73 us, 9 diagonals 97.6 ->
-// 78; 1026x514, 9 diagonals 362 -> 325; FP32 1026x514, 9 diagonals 167 -> 147,
-// 515x259, 5 diagonals 84 -> 74.  Five slots: a chunk's loads have two to
+// sweeps and fed, traces of one box: FP64 258x130, 5 diagonals 92 -> 74.5 us, 9
+// diagonals 87 -> 69; 1026x514, 9 diagonals 364 -> 320; FP32 1026x514, 9
+// diagonals 190 -> 166, 515x259, 5 diagonals 86 -> 70.  Five slots: a chunk's loads have two to
 // three chunks (1 us) to arrive, what the LDS holds for 9 diagonals in FP64.
 //
 // Barriers (c = -1 .. nf-1), passed by all four: barrier c follows chunk c;

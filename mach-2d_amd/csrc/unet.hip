@@ -157,10 +157,14 @@ __global__ __launch_bounds__(256) void k_conv3x3(ConvArgs A)
 // weights are the first operand, so a lane ends up with four neighbouring
 // channels of one pixel and stores them at once.  Products are added in the
 // order of k_conv3x3 (32 k at a time), so both give the same bits.
-//   bound: the 16-channel layers of the full resolution by memory (an
-// input and an output tensor), the deep ones by the LDS reads and the few
-// workgroups they have.  A pixel's channels lie an odd number of 16-byte
-// units apart, so 16 lanes' reads meet no bank twice.
+//   bound: the 16-channel layers of the full resolution by memory (1026x514:
+// 50.8 MB in 13.6 us, 3.7 TB/s); the others by latency, of the staged tile, of
+// the weights and, in the deep layers, of few workgroups: no unit is near its
+// rate (counted over the guess: matrix cores busy for 4 to 13 % of a kernel's
+// time, LDS for 4 to 25 %).  A pixel's channels lie an odd number of 16-byte
+// units apart, so that 16 neighbouring pixels start in different banks; about
+// 46 % of the LDS's busy cycles are conflicts all the same (6 % with 8
+// channels).
 constexpr int kTileW = 16, kHaloW = kTileW + 2;
 
 // channels between two pixels of the staged tile
@@ -403,8 +407,11 @@ __global__ __launch_bounds__(256) void k_conv3x3_tile(ConvArgs A)
 // come from one read of ten pixels, shifted in registers.  The next tile's
 // loads are under way while a tile is computed.  At the end the waves'
 // sums meet in LDS and leave with one FP32 atomic each.
-//   bound: the staging's two-byte LDS writes; before, every lane fetched
-// every element of both operands from memory by itself.
+//   bound: latency; a tile's transposing two-byte LDS writes, its reads and
+// its products follow one another between barriers, and no unit is near its
+// rate (258x130, 16 images: matrix cores busy for 4 to 7 % of a kernel's time,
+// LDS for 10 to 16 %).  Before, every lane fetched every element of both
+// operands from memory by itself.
 constexpr int kGradH = 16, kGradWaves = kGradH / 2, kGradThreads = 64 * kGradWaves;
 constexpr int kGradRow = 16 + 8;                      // pixels between two staged rows
 constexpr int kGradX = (kGradH + 2) * kGradRow + 8;   // ... two channels (input)
