@@ -68,13 +68,13 @@ BYTES_PER_POINT = {
 
 
 # HBM bytes per launch at 1026x514, measured with rocprofv3 (FETCH_SIZE and
-# WRITE_SIZE in separate runs of this script, scaled by 2.2488 and 1.1250:
+# WRITE_SIZE in separate runs of this script, scaled by 1.9991 and 1.0000:
 # the factors a conversion kernel of known size reads;
 # profiles/msi_1026x514_hbm_traffic.md).  "residual" is the update and the
 # residual of one launch, "residual32" the two launches around a sweep pair.
 MEASURED_TRAFFIC = {
-    "sweeps": 83.60e6, "residual": 67.14e6, "factor": 111.44e6,
-    "sweeps32": 37.69e6, "residual32": 76.61e6, "factor32": 55.93e6,
+    "sweeps": 74.32e6, "residual": 59.68e6, "factor": 99.06e6,
+    "sweeps32": 33.50e6, "residual32": 68.10e6, "factor32": 49.71e6,
 }
 
 

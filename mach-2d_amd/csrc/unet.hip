@@ -158,7 +158,7 @@ __global__ __launch_bounds__(256) void k_conv3x3(ConvArgs A)
 // channels of one pixel and stores them at once.  Products are added in the
 // order of k_conv3x3 (32 k at a time), so both give the same bits.
 //   bound: the 16-channel layers of the full resolution by memory (1026x514:
-// 50.8 MB in 13.6 us, 3.7 TB/s); the others by latency, of the staged tile, of
+// 45.1 MB in 13.6 us, 3.3 TB/s); the others by latency, of the staged tile, of
 // the weights and, in the deep layers, of few workgroups: no unit is near its
 // rate (counted over the guess: matrix cores busy for 4 to 13 % of a kernel's
 // time, LDS for 4 to 25 %).  A pixel's channels lie an odd number of 16-byte
