@@ -147,7 +147,8 @@ class UNet:
             w[:lay.cout, :9 * lay.cin] = torch.randn(lay.cout, 9 * lay.cin, generator=g) * std
             lay.w.copy_(w)
         self.step_count = 0
-        self._count = None      # pinned copy of a mask's count, its event
+        # a mask's count in pinned memory, and the event of its copy
+        self._count = torch.empty((), pin_memory=True), torch.cuda.Event()
         self.pack()
 
     def _one_buffer(self, kinds="pgmv"):
@@ -224,10 +225,8 @@ class UNet:
         cnt = mask.sum(dtype=t.float32)
         looked = not t.cuda.is_current_stream_capturing()
         if looked:
-            if self._count is None:
-                self._count = t.empty((), pin_memory=True), t.cuda.Event()
             self._count[0].copy_(cnt, non_blocking=True)
-            self._count[1].record()
+            self._count[1].record(t.cuda.current_stream(cnt.device))
         out = self.forward(x, stream, keep=True)
         acts = self._acts
         head = self.layers[-1]
