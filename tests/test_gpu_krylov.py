@@ -53,7 +53,8 @@ def test_point_blocks(gpu, orc, nx, ny, nd):
 @pytest.mark.parametrize("inner", [(1e-4, 1), (1e-4, 4), (1e-4, 6), (1e-2, 25), (1e-4, 200)])
 def test_window(gpu, orc, inner):
     """Correction solves shorter than the window of kept directions, just
-    past it, and long ones; never more sweeps than plain MSI."""
+    past it, and long ones; at most one correction solve's sweeps more than
+    plain MSI."""
     s = P.pcorr_system(66, 34, seed=2, rhs="gauss")
     ox, onit = _oracle(orc, s, 9)
     st, x = _solve(gpu, s, 9, inner)

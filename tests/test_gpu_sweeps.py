@@ -47,9 +47,11 @@ def test_fp64_bitwise(gpu, orc, nx, ny, nd):
         assert np.array_equal(_solve(gpu, s, nd, "fp64", 5, stride), ox), stride
 
 
-def test_many_bands(gpu, orc):
-    """66 bands: beyond the fed sweeps' share of the CUs."""
-    nx, ny = 6, 4163
+@pytest.mark.parametrize("ny", [4096, 4097, 4163])
+def test_many_bands(gpu, orc, ny):
+    """64 bands, the most that take the fed sweeps, and 65 and 66 (one and
+    three rows into the last band), which take the register sweeps."""
+    nx = 6
     s = _system(nx, ny, 9)
     dl, du = orc.lu2d9(s.a, nx, ny)
     ox = orc.fb2d9(s.a, dl, du, nx, ny, np.zeros(s.N), 0.0, 3, s.rhs)[0]
